@@ -67,29 +67,6 @@ __device__ __forceinline__ double wsum(double v) {
     return v;
 }
 
-// fixed-order sum over the workgroup of VT threads, returned to all
-__device__ __forceinline__ double vsum_all(double v) {
-    __shared__ double red[VT / 64];
-    __shared__ double total;
-    v = wsum(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < VT / 64; ++i) s += red[i];
-        total = s;
-    }
-    __syncthreads();
-    return total;
-}
-
-__device__ __forceinline__ double vreduce(const double *__restrict__ part, int np) {
-    return vsum_all(strided_sum<VT>(part, 0, np));
-}
-
 // E4[c * noe + e] = sum_nodes r(e, i1, i2) wx_c(i1) wy_c(i2); corner c = 0
 // bottom-left, 1 bottom-right, 2 top-left, 3 top-right; wx = 1 - xi or xi,
 // wy = 1 - xi or xi (xi = (z+1)/2: x from the element's left, y from its
@@ -284,29 +261,50 @@ __global__ __launch_bounds__(VT) void add_coarse_kernel(T *__restrict__ v, const
     }
 }
 
+// Elements per group of the kernels that interpolate from the vertex grid:
+// about 4096 values, a multiple of four elements (so that a group's values
+// divide into 16-byte vectors).
+template <int P>
+constexpr int interp_elems() {
+    constexpr int ne = (4096 / ((P + 1) * (P + 1))) & ~3;
+    return ne < 4 ? 4 : (ne > 256 ? 256 : ne);
+}
+
 // pcg_update_p_kernel with the coarse level: r.z = sum(prz) + sum(pc)
 // (the block-Jacobi part and S.C) and p = z + P0^T C + beta p.
+//
+// Bound: memory, five vector passes (x, p, z in; x, p out).  A workgroup
+// takes groups of about 4096 values of whole elements; the interpolation
+// along each element line x = const (the value at the line's lower end and
+// its rise) is formed once per line in LDS, so that a value costs one fused
+// multiply-add instead of a bilinear interpolation with four scattered
+// vertex loads, and the streams move 16 bytes per lane.  alpha is the one
+// that the block-Jacobi kernel of this iteration recorded in the slot.
+// Measured per launch, one value per lane with the interpolation at every
+// node -> this: 16x16-node FP32 elements (128 x 128) 30.1 -> 16.6 us,
+// FP64 p = 8 (256 x 256) 44.6 -> 38.2 us.
 template <typename T, int P>
 __global__ __launch_bounds__(VT) void pcg2_update_p_kernel(T *__restrict__ x, T *__restrict__ p,
-                                                           const T *__restrict__ z, int64_t n,
-                                                           const double *__restrict__ ppAp, int np_pAp,
+                                                           const T *__restrict__ z, int64_t noe,
                                                            const double *__restrict__ prr,
                                                            const double *__restrict__ prz, int np,
                                                            const double *__restrict__ pc, int npc,
                                                            const double *__restrict__ Cpad,
                                                            const double *__restrict__ xi, int dimx, cg_state *st,
                                                            int slot, T *__restrict__ xlo) {
-    constexpr int N1 = P + 1, NQ = N1 * N1;
+    constexpr int N1 = P + 1, NQ = N1 * N1, NEG = interp_elems<P>(), VL = 16 / (int)sizeof(T);
+    static_assert(NEG * NQ % VL == 0, "a group divides into vectors");
     __shared__ double sx[N1];
+    __shared__ double lo[NEG * N1], up[NEG * N1];       // per line: value at its lower end, rise to the upper one
     const cg_slot cur = st->s[slot];
     if (cur.done | st->err) {
         if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot ^ 1] = cur;   // carry forward
         return;
     }
     if (threadIdx.x < N1) sx[threadIdx.x] = xi[threadIdx.x];
-    const double rr_new = vreduce(prr, np);
-    const double rz_new = vreduce(prz, np) + vreduce(pc, npc);
-    const double pAp = vreduce(ppAp, np_pAp);
+    double sum[3];
+    multi_sum<VT, 3>({prr, prz, pc}, {np, np, npc}, sum);      // its barrier publishes sx
+    const double rr_new = sum[0], rz_new = sum[1] + sum[2];
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
     const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rz_new / cur.rz;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -327,25 +325,79 @@ __global__ __launch_bounds__(VT) void pcg2_update_p_kernel(T *__restrict__ x, T 
         if (!isfinite(rr_new) || !isfinite(rz_new)) st->err = 3;
         else if (!(rz_new > 0.0) && rr_new > 0.0) st->err = 2;   // M not positive on r
     }
-    const T alpha = (T)(cur.rz / pAp);
+    const T alpha = (T)cur.alpha;
     const T beta = (T)beta_d;
-    for (int64_t i = (int64_t)blockIdx.x * VT + threadIdx.x; i < n; i += (int64_t)gridDim.x * VT) {
-        const int e = (int)(i / NQ), node = (int)(i - (int64_t)e * NQ);
-        const int i1 = node / N1, i2 = node - (node / N1) * N1;
-        const T pi = p[i];
-        if (!replaced) {
-            if (xlo) {
-                T xh = x[i], xl = xlo[i];
-                comp_axpy(xh, xl, alpha, pi);
-                x[i] = xh;
-                xlo[i] = xl;
-            } else {
-                x[i] = x[i] + alpha * pi;
+    const int ld = dimx + 1;
+    const int64_t ngroup = (noe + NEG - 1) / NEG;
+    for (int64_t g = blockIdx.x; g < ngroup; g += gridDim.x) {
+        const int64_t e0 = g * NEG;
+        const int ne = (int)min<int64_t>(NEG, noe - e0);
+        for (int l = threadIdx.x; l < ne * N1; l += VT) {
+            const int el = l / N1, i1 = l - el * N1;
+            const int e = (int)e0 + el, row = e / dimx, col = e - row * dimx;
+            const double *c = Cpad + (int64_t)row * ld + col;
+            const double t = sx[i1];
+            const double top = (1.0 - t) * c[0] + t * c[1], bot = (1.0 - t) * c[ld] + t * c[ld + 1];
+            lo[l] = bot;
+            up[l] = top - bot;
+        }
+        __syncthreads();
+        const int n = ne * NQ;
+        T *xg = x + e0 * NQ, *pg = p + e0 * NQ, *lg = xlo + (xlo ? e0 * NQ : 0);
+        const T *zg = z + e0 * NQ;
+#pragma unroll 2
+        for (int i = VL * threadIdx.x; i < n; i += VL * VT) {
+            if (i + VL <= n) {
+                T pv[VL], zv[VL], xv[VL];
+                load_vec<T, VL>(pg + i, pv);
+                load_vec<T, VL>(zg + i, zv);
+                if (!replaced) {
+                    load_vec<T, VL>(xg + i, xv);
+                    if (xlo) {
+                        T xl[VL];
+                        load_vec<T, VL>(lg + i, xl);
+#pragma unroll
+                        for (int q = 0; q < VL; ++q) comp_axpy(xv[q], xl[q], alpha, pv[q]);
+                        store_vec<T, VL>(lg + i, xl);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < VL; ++q) xv[q] = xv[q] + alpha * pv[q];
+                    }
+                    store_vec<T, VL>(xg + i, xv);
+                }
+#pragma unroll
+                for (int q = 0; q < VL; ++q) {
+                    const int l = (i + q) / N1, i2 = i + q - l * N1;
+                    pv[q] = (T)((double)zv[q] + (lo[l] + sx[i2] * up[l])) + beta * pv[q];
+                }
+                store_vec<T, VL>(pg + i, pv);
+            } else {                                     // the mesh's last values
+                for (int q = i; q < n; ++q) {
+                    const int l = q / N1, i2 = q - l * N1;
+                    const T pi = pg[q];
+                    if (!replaced) {
+                        if (xlo) comp_axpy(xg[q], lg[q], alpha, pi);
+                        else xg[q] = xg[q] + alpha * pi;
+                    }
+                    pg[q] = (T)((double)zg[q] + (lo[l] + sx[i2] * up[l])) + beta * pi;
+                }
             }
         }
-        p[i] = (T)((double)z[i] + prolong<P>(Cpad, sx, dimx, e, i1, i2)) + beta * pi;
+        __syncthreads();                                 // the lines are free for the next group
     }
 }
+
+struct coarse_args {
+    const void *r = nullptr;
+    void *v = nullptr, *x = nullptr, *xlo = nullptr;
+    const void *z = nullptr;
+    const double *xi = nullptr, *Cpad = nullptr, *prr = nullptr, *prz = nullptr, *pc = nullptr;
+    double *E4 = nullptr;
+    int64_t noe = 0, n = 0;
+    int dimx = 0, nblk = 0, np = 0, npc = 0, slot = 0;
+    cg_state *st = nullptr;
+    hipStream_t s = nullptr;
+};
 
 template <int P>
 struct CoarseFns {
@@ -359,24 +411,12 @@ struct CoarseFns {
         hipLaunchKernelGGL((add_coarse_kernel<T, P>), dim3(nblk), dim3(VT), 0, s, (T *)v, Cpad, xi, dimx, n);
     }
     template <typename T>
-    static void update_(void *x, void *p, const void *z, int64_t n, const double *ppAp, int np_pAp, const double *prr,
-                        const double *prz, int np, const double *pc, int npc, const double *Cpad, const double *xi,
-                        int dimx, int nblk, cg_state *st, int slot, hipStream_t s, void *xlo) {
-        hipLaunchKernelGGL((pcg2_update_p_kernel<T, P>), dim3(nblk), dim3(VT), 0, s, (T *)x, (T *)p, (const T *)z, n,
-                           ppAp, np_pAp, prr, prz, np, pc, npc, Cpad, xi, dimx, st, slot, (T *)xlo);
+    static void update_(const coarse_args &a) {
+        const int nb = (int)std::min<int64_t>((a.noe + interp_elems<P>() - 1) / interp_elems<P>(), 2048);
+        hipLaunchKernelGGL((pcg2_update_p_kernel<T, P>), dim3(nb), dim3(VT), 0, a.s, (T *)a.x, (T *)a.v,
+                           (const T *)a.z, a.noe, a.prr, a.prz, a.np, a.pc, a.npc, a.Cpad, a.xi, a.dimx, a.st, a.slot,
+                           (T *)a.xlo);
     }
-};
-
-struct coarse_args {
-    const void *r = nullptr;
-    void *v = nullptr, *x = nullptr, *xlo = nullptr;
-    const void *z = nullptr;
-    const double *xi = nullptr, *Cpad = nullptr, *ppAp = nullptr, *prr = nullptr, *prz = nullptr, *pc = nullptr;
-    double *E4 = nullptr;
-    int64_t noe = 0, n = 0;
-    int dimx = 0, nblk = 0, np_pAp = 0, np = 0, npc = 0, slot = 0;
-    cg_state *st = nullptr;
-    hipStream_t s = nullptr;
 };
 
 template <int P>
@@ -394,12 +434,8 @@ int dispatch_p(int p, int dtype, int what, const coarse_args &a) {
         if (f64) F::template add_<double>(a.v, a.Cpad, a.xi, a.dimx, a.n, a.nblk, a.s);
         else F::template add_<float>(a.v, a.Cpad, a.xi, a.dimx, a.n, a.nblk, a.s);
     } else {
-        if (f64)
-            F::template update_<double>(a.x, a.v, a.z, a.n, a.ppAp, a.np_pAp, a.prr, a.prz, a.np, a.pc, a.npc, a.Cpad,
-                                        a.xi, a.dimx, a.nblk, a.st, a.slot, a.s, a.xlo);
-        else
-            F::template update_<float>(a.x, a.v, a.z, a.n, a.ppAp, a.np_pAp, a.prr, a.prz, a.np, a.pc, a.npc, a.Cpad,
-                                       a.xi, a.dimx, a.nblk, a.st, a.slot, a.s, a.xlo);
+        if (f64) F::template update_<double>(a);
+        else F::template update_<float>(a);
     }
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
@@ -582,14 +618,13 @@ int launch_coarse_add(int dtype, int p, void *v, int dimx, int64_t n, const coar
 int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_pAp,
                          int np_pAp, const double *part_rr, const double *part_rz, int np, int npc, int dimx,
                          const coarse_tables &c, int nblk, cg_state *st, int slot, hipStream_t s, void *xlo) {
+    (void)part_pAp, (void)np_pAp, (void)nblk;           // alpha: recorded in the slot by launch_pcg_rz
     coarse_args a{};
     a.x = x;
     a.xlo = xlo;
     a.v = pv;
     a.z = z;
-    a.n = n;
-    a.ppAp = part_pAp;
-    a.np_pAp = np_pAp;
+    a.noe = n / ((p + 1) * (p + 1));
     a.prr = part_rr;
     a.prz = part_rz;
     a.np = np;
@@ -598,7 +633,6 @@ int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int
     a.Cpad = c.Cpad;
     a.xi = c.xi;
     a.dimx = dimx;
-    a.nblk = nblk;
     a.st = st;
     a.slot = slot;
     a.s = s;

@@ -105,6 +105,7 @@ void pcg_rz_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ 
             return;
         }
         alpha = (T)a;
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot].alpha = a;    // for the p update
     }
     constexpr cx::PrecTables<P> PT = cx::make_prec<P>();
     struct CS {
@@ -308,6 +309,7 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
             return;
         }
         alpha = (T)a;
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot].alpha = a;    // for the p update
     }
     // 1 / (lambda_a + lambda_c), read per lane (row j) from LDS
     for (int q = threadIdx.x; q < NQ; q += NT) {
@@ -620,7 +622,6 @@ __device__ __forceinline__ double vreduce(const double *__restrict__ part, int n
 template <typename T>
 __global__ __launch_bounds__(VT) void pcg_update_p_kernel(T *__restrict__ x, T *__restrict__ p,
                                                           const T *__restrict__ z, int64_t n,
-                                                          const double *__restrict__ ppAp, int np_pAp,
                                                           const double *__restrict__ prr,
                                                           const double *__restrict__ prz, int np,
                                                           cg_state *st, int slot, T *__restrict__ xlo) {
@@ -629,9 +630,9 @@ __global__ __launch_bounds__(VT) void pcg_update_p_kernel(T *__restrict__ x, T *
         if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot ^ 1] = cur;   // carry forward
         return;
     }
-    const double rr_new = vreduce(prr, np);
-    const double rz_new = vreduce(prz, np);
-    const double pAp = vreduce(ppAp, np_pAp);
+    double sum[2];
+    multi_sum<VT, 2>({prr, prz}, {np, np}, sum);
+    const double rr_new = sum[0], rz_new = sum[1];
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
     const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rz_new / cur.rz;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -652,19 +653,39 @@ __global__ __launch_bounds__(VT) void pcg_update_p_kernel(T *__restrict__ x, T *
         if (!isfinite(rr_new) || !isfinite(rz_new)) st->err = 3;
         else if (!(rz_new > 0.0) && rr_new > 0.0) st->err = 2;   // M not positive on r
     }
-    const T alpha = (T)(cur.rz / pAp);
+    const T alpha = (T)cur.alpha;                        // recorded by the block-Jacobi kernel
     const T beta = (T)beta_d;
-    for (int64_t i = (int64_t)blockIdx.x * VT + threadIdx.x; i < n; i += (int64_t)gridDim.x * VT) {
+    constexpr int VL = 16 / (int)sizeof(T);
+    const int64_t nv = n / VL;
+    for (int64_t k = (int64_t)blockIdx.x * VT + threadIdx.x; k < nv; k += (int64_t)gridDim.x * VT) {
+        const int64_t i = k * VL;
+        T pv[VL], zv[VL], xv[VL];
+        load_vec<T, VL>(p + i, pv);
+        load_vec<T, VL>(z + i, zv);
+        if (!replaced) {
+            load_vec<T, VL>(x + i, xv);
+            if (xlo) {
+                T xl[VL];
+                load_vec<T, VL>(xlo + i, xl);
+#pragma unroll
+                for (int q = 0; q < VL; ++q) comp_axpy(xv[q], xl[q], alpha, pv[q]);
+                store_vec<T, VL>(xlo + i, xl);
+            } else {
+#pragma unroll
+                for (int q = 0; q < VL; ++q) xv[q] = xv[q] + alpha * pv[q];
+            }
+            store_vec<T, VL>(x + i, xv);
+        }
+#pragma unroll
+        for (int q = 0; q < VL; ++q) pv[q] = zv[q] + beta * pv[q];
+        store_vec<T, VL>(p + i, pv);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n - nv * VL) {
+        const int64_t i = nv * VL + threadIdx.x;
         const T pi = p[i];
         if (!replaced) {
-            if (xlo) {
-                T xh = x[i], xl = xlo[i];
-                comp_axpy(xh, xl, alpha, pi);
-                x[i] = xh;
-                xlo[i] = xl;
-            } else {
-                x[i] = x[i] + alpha * pi;
-            }
+            if (xlo) comp_axpy(x[i], xlo[i], alpha, pi);
+            else x[i] = x[i] + alpha * pi;
         }
         p[i] = z[i] + beta * pi;
     }
@@ -753,12 +774,13 @@ int launch_pcg_rz(int dtype, int p, double pen, int mode, void *r, const void *A
 int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_pAp,
                         int np_pAp, const double *part_rr, const double *part_rz, int np, int nblk,
                         cg_state *st, int slot, hipStream_t s, void *xlo) {
+    (void)part_pAp, (void)np_pAp;                       // alpha: recorded in the slot by launch_pcg_rz
     if (dtype == SIPG_F64)
         hipLaunchKernelGGL(pcg_update_p_kernel<double>, dim3(nblk), dim3(VT), 0, s, (double *)x, (double *)p,
-                           (const double *)z, n, part_pAp, np_pAp, part_rr, part_rz, np, st, slot, (double *)xlo);
+                           (const double *)z, n, part_rr, part_rz, np, st, slot, (double *)xlo);
     else
         hipLaunchKernelGGL(pcg_update_p_kernel<float>, dim3(nblk), dim3(VT), 0, s, (float *)x, (float *)p,
-                           (const float *)z, n, part_pAp, np_pAp, part_rr, part_rz, np, st, slot, (float *)xlo);
+                           (const float *)z, n, part_rr, part_rz, np, st, slot, (float *)xlo);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }

@@ -25,6 +25,67 @@ __device__ __forceinline__ double strided_sum(const double *__restrict__ part, i
     return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
 }
 
+// The sums of K arrays of block sums (np[k] values each), returned to every
+// thread of a workgroup of NT, in one exchange: the K wave sums are formed
+// together and cross the workgroup behind one barrier, where K separate
+// reductions would wait for two each.  Loads past the end of an array are
+// clamped to its last value and discarded, so that all of them are in
+// flight at once.  Fixed order, as strided_sum.
+template <int NT, int K>
+__device__ __forceinline__ void multi_sum(const double *const (&part)[K], const int (&np)[K], double (&out)[K]) {
+    __shared__ double red[K][NT / 64];
+    double v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        double a[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int i = (int)threadIdx.x; i < np[k]; i += 4 * NT) {
+            double t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = part[k][min(i + u * NT, np[k] - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] += i + u * NT < np[k] ? t[u] : 0.0;
+        }
+        v[k] = (a[0] + a[1]) + (a[2] + a[3]);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) red[k][threadIdx.x >> 6] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) s += red[k][i];
+        out[k] = s;
+    }
+}
+
+// VL consecutive values at an address that is aligned to one value only
+// (one 16-byte access where the hardware allows it, which on gfx950 is any
+// multiple of four bytes).
+template <typename T, int VL>
+struct __attribute__((packed, aligned(sizeof(T)))) VecU {
+    T v[VL];
+};
+template <typename T, int VL>
+__device__ __forceinline__ void load_vec(const T *p, T (&r)[VL]) {
+    const VecU<T, VL> v = *reinterpret_cast<const VecU<T, VL> *>(p);
+#pragma unroll
+    for (int i = 0; i < VL; ++i) r[i] = v.v[i];
+}
+template <typename T, int VL>
+__device__ __forceinline__ void store_vec(T *p, const T (&r)[VL]) {
+    VecU<T, VL> v;
+#pragma unroll
+    for (int i = 0; i < VL; ++i) v.v[i] = r[i];
+    *reinterpret_cast<VecU<T, VL> *>(p) = v;
+}
+
 // xh += a p with the rounding errors kept in xl, so that xh + xl carries
 // the running sum to about twice the working precision: the product's
 // error from an fma, the sum's by Knuth's TwoSum (both exact).  Contraction
