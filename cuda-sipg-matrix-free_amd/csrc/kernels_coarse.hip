@@ -31,14 +31,13 @@
 // and the p update interpolates Cpad into every node (p = z + P0^T C + beta p)
 // with r.z = r.z_BJ + S.C.
 //
-// Large vertex grids (kBlasVertices and up: from about 271 x 271 elements)
+// Large vertex grids (kBlasVertices and up: from about 541 x 541 elements)
 // take the four products as rocBLAS FP64 GEMMs instead, with the
 // gather, the 1/Lambda scaling and the S.C partials as small kernels of
 // their own: the dense products grow as the cube of the mesh side, and the
-// library's matrix-core GEMM runs them several times faster than the
-// folded VALU kernel, which is latency-bound and wins below that size.
-// rocBLAS is opened on first use (dlopen); without it the folded kernel
-// runs at every size.
+// folded kernel, which reads its operands from L2 once per 16 x 16 tile, then
+// is bound by those reads.  rocBLAS is opened on first use (dlopen); without
+// it the folded kernel runs at every size.
 #include "sipg_internal.hpp"
 #include "partials.hpp"
 
@@ -57,9 +56,15 @@ constexpr int VT = kVecThreads;
 template <int P>
 constexpr int rne() { return 4096 / ((P + 1) * (P + 1)) < 32 ? 4096 / ((P + 1) * (P + 1)) : 32; }
 constexpr int GT = 16;           // gemm output tile (GT x GT)
-constexpr int KC2 = 128;         // folded k chunk staged in LDS
-constexpr int KS = 4;            // gemm k slices per output
-constexpr int GEMM_T = GT * GT * KS;
+// waves per tile, which split the k range: more where an operand value is
+// eight scattered loads (MODE 3)
+__host__ __device__ constexpr int dst_waves(int mode) { return mode == 3 ? 16 : 8; }
+
+typedef double dd4 __attribute__((ext_vector_type(4)));
+
+// Tiles of GT indices of one parity in 0..n-1: the even indices, and all.
+__host__ __device__ constexpr int dst_tiles_even(int n) { return ((n + 1) / 2 + GT - 1) / GT; }
+__host__ __device__ constexpr int dst_tiles(int n) { return dst_tiles_even(n) + (n / 2 + GT - 1) / GT; }
 
 __device__ __forceinline__ double wsum(double v) {
 #pragma unroll
@@ -102,131 +107,116 @@ __global__ __launch_bounds__(VT) void restrict_kernel(const T *__restrict__ r, c
 // so each product folds its k range in half: with h = n / 2,
 //   (Q X)[j][m] = sum_{k<h} Q[j][k] (X[k][m] +- X[n-1-k][m]) (+ Q[j][h] X[h][m], n odd)
 //   (X Q)[m][j] = sum_{k<h} (X[m][k] +- X[m][n-1-k]) Q[k][j]  (+ X[m][h] Q[h][j], n odd)
-// with + for even j and - for odd j.  One workgroup per GT x GT output tile
-// (GT = 16, so a 255 x 255 product has 256 of them, one per CU); the folded
-// strips (KC2 values of the half range at a time, one chunk up to n = 256)
-// are staged in LDS, and the 1024 threads split that range four ways (four
-// waves per SIMD), the partial sums added in LDS in a fixed order.
+// with + for even j and - for odd j.  The products run on the FP64 matrix
+// cores (v_mfma_f64_16x16x4f64: lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and, in register r, D[4 r + l / 16][l % 16]).  An output
+// tile takes 16 indices j of one parity (j = 2 t + parity), so that one fold
+// of X serves the whole tile; the other dimension is cut plainly.  One
+// workgroup per tile; its waves (KS of them) take the k blocks of four in
+// turn, straight from memory (the operands are a few hundred KB and
+// sit in L2), and the partial tiles are added in LDS in a fixed order.
+//
+// Bound: latency (33 MFLOP at 255 x 255).  All loads of a wave's k blocks
+// are issued before the first product, so that a product is one round trip
+// to L2, the matrix instructions and one LDS exchange; the previous kernel
+// staged both operands in LDS and read two LDS values per multiply-add on
+// the vector ALUs.  255 x 255: 8.8 + 6.9 + 7.2 + 6.9 -> 5.9 + 4.9 + 5.0 + 4.9 us for the four
+// products; 127 x 127: 25.7 -> 18.7 us in all.
 //   SIDE 0: out (n x N) = Q X (X: n x N);  SIDE 1: out (M x n) = X Q (X: M x n)
-//   MODE 0: out = the product                (SIDE 1)
-//   MODE 1: out = product .* W               (SIDE 0; W the 1/Lambda table)
-//   MODE 2: Cpad[(i+1)*(N+2) + j+1] = product, and per-workgroup partials of
-//           sum product .* W into part[blockIdx.y * gridDim.x + blockIdx.x]   (SIDE 0)
+//   MODE 0: out = the product
+//   MODE 1: out = product .* W               (W the 1/Lambda table)
+//   MODE 2: Cpad[(i+1)*(cols+2) + j+1] = product, and per-workgroup partials of
+//           sum product .* W into part[blockIdx.y * gridDim.x + blockIdx.x]
 //   MODE 3: as MODE 0 with X = S gathered from the corner sums E4 (X is E4,
-//           M + 1 by n + 1 elements; the first tile column also stores S
-//           into W)
+//           n + 1 by N + 1 elements; the first tile row also stores S into
+//           W).  On SIDE 0, where a load covers 16 neighbouring vertices: the
+//           rows of E4 are a power of two apart on the usual meshes, and four
+//           vertices from each of 16 rows (SIDE 1) took 10.9 against 5.9 us.
 template <int SIDE, int MODE>
-__global__ __launch_bounds__(GEMM_T) void dst_gemm_kernel(const double *__restrict__ X,
+__global__ __launch_bounds__(64 * dst_waves(MODE)) void dst_gemm_kernel(const double *__restrict__ X,
                                                           const double *__restrict__ Q, int M, int n, int N,
                                                           double *__restrict__ W, double *__restrict__ out,
                                                           double *__restrict__ part, const cg_state *st, int slot) {
     // inside a solve: nothing to do once it has finished (the launches
     // queued past the finish run as no-ops)
     if (st && (st->s[slot].done | st->err)) return;
-    // SIDE 0: A = Q rows (plain), B0/B1 = folded X (+/-); SIDE 1: A0/A1 =
-    // folded X rows (+/-), B = Q columns
-    __shared__ double Aq[SIDE == 1 ? 2 : 1][GT][KC2 + 1];
-    __shared__ double Bq[SIDE == 0 ? 2 : 1][KC2][GT];
+    constexpr int KS = dst_waves(MODE);
+    constexpr int KB = MODE == 3 ? 2 : 4;               // k blocks in flight per wave (n = 255: all of them)
     __shared__ double ps[KS][GT][GT + 1];
-    const int o = threadIdx.x % (GT * GT), ks = threadIdx.x / (GT * GT);
-    const int tx = o % GT, ty = o / GT;
-    const int row0 = blockIdx.y * GT, col0 = blockIdx.x * GT;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lk = lane >> 4;
     const int rows = SIDE == 0 ? n : M, cols = SIDE == 0 ? N : n;
-    const int h = n / 2, kh = h + (n & 1);          // folded length (with the middle)
-    // X element (r, k) of the (rows x n) or (n x N) operand
-    auto xval = [&](int r, int k) -> double {
+    const int h = n / 2, kh = h + (n & 1);              // folded length (with the middle)
+    // the folded dimension's tiles: the even indices first, then the odd ones
+    const int te = dst_tiles_even(n);
+    const int tf = SIDE == 0 ? blockIdx.y : blockIdx.x;
+    const int par = tf >= te ? 1 : 0, f0 = 2 * GT * (par ? tf - te : tf) + par, fs = 2;
+    const int r0 = SIDE == 0 ? f0 : (int)blockIdx.y * GT, rs = SIDE == 0 ? fs : 1;
+    const int c0 = SIDE == 0 ? (int)blockIdx.x * GT : f0, cs = SIDE == 0 ? 1 : fs;
+    const double sgn = par ? -1.0 : 1.0;
+    // X element (m, k): k in the folded direction
+    const int dimx = N + 1;
+    const int64_t noe = (int64_t)dimx * (n + 1);
+    auto xval = [&](int m, int k) -> double {
         if (MODE == 3) {
-            const int a = r + 1, b = k + 1, dimx = n + 1;
-            const int64_t noe = (int64_t)dimx * (M + 1);
-            return (X[1 * noe + (int64_t)(a - 1) * dimx + (b - 1)] + X[0 * noe + (int64_t)(a - 1) * dimx + b]) +
-                   (X[3 * noe + (int64_t)a * dimx + (b - 1)] + X[2 * noe + (int64_t)a * dimx + b]);
+            const int64_t a = (int64_t)k * dimx + m, b = a + dimx;
+            return (X[1 * noe + a] + X[0 * noe + a + 1]) + (X[3 * noe + b] + X[2 * noe + b + 1]);
         }
-        return SIDE == 0 ? X[(int64_t)k * N + r] : X[(int64_t)r * n + k];
+        return SIDE == 0 ? X[(int64_t)k * N + m] : X[(int64_t)m * n + k];
     };
-    // output (gr, gc): its parity picks the folded operand
-    const int gr = row0 + ty, gc = col0 + tx;
-    const bool odd = SIDE == 0 ? (gr & 1) : (gc & 1);
-    double acc[2] = {0.0, 0.0};
-    for (int k0 = 0; k0 < kh; k0 += KC2) {
-        const int kc = min(KC2, kh - k0);
-        for (int i = threadIdx.x; i < GT * KC2; i += GEMM_T) {
-            const int r = i / KC2, kk = i - (i / KC2) * KC2, k = k0 + kk;
-            if (SIDE == 0) {
-                const int gq = row0 + r;
-                Aq[0][r][kk] = (gq < rows && kk < kc) ? Q[(int64_t)gq * n + k] : 0.0;
-            } else {
-                const int gx = row0 + r;
-                double p = 0.0, q = 0.0;
-                if (gx < rows && kk < kc) {
-                    const double a = xval(gx, k);
-                    if (k < h) {
-                        const double b = xval(gx, n - 1 - k);
-                        p = a + b;
-                        q = a - b;
-                        if (MODE == 3 && blockIdx.x == 0) {
-                            W[(int64_t)gx * n + k] = a;
-                            W[(int64_t)gx * n + n - 1 - k] = b;
-                        }
-                    } else {                                  // the middle (n odd)
-                        p = q = a;
-                        if (MODE == 3 && blockIdx.x == 0) W[(int64_t)gx * n + k] = a;
-                    }
-                }
-                Aq[0][r][kk] = p;
-                Aq[SIDE == 1 ? 1 : 0][r][kk] = q;
+    // this lane's row of Q (its folded index) and its line of X
+    const int jq = f0 + fs * li, mx = (SIDE == 0 ? c0 : r0) + li;
+    const bool qok = jq < n, xok = mx < (SIDE == 0 ? N : M);
+    const double *Qj = Q + (int64_t)(qok ? jq : 0) * n;
+    const int m = xok ? mx : 0;
+    const int nkb = (kh + 3) / 4;
+    dd4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int b0 = w; b0 < nkb; b0 += KS * KB) {
+        double q[KB], xa[KB], xb[KB];
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+            // (clamped: blocks past the end are loaded from the last k and weighted zero)
+            const int k = min(4 * (b0 + KS * i) + lk, kh - 1);
+            q[i] = Qj[k];
+            xa[i] = xval(m, k);
+            xb[i] = xval(m, n - 1 - k);
+        }
+#pragma unroll
+        for (int i = 0; i < KB; ++i) {
+            const int k = 4 * (b0 + KS * i) + lk;
+            if (MODE == 3 && blockIdx.y == 0 && xok && k < kh) {
+                W[(int64_t)k * N + m] = xa[i];
+                W[(int64_t)(n - 1 - k) * N + m] = xb[i];
             }
+            // the middle (n odd) enters once
+            const double xf = k < h ? xa[i] + sgn * xb[i] : xa[i];
+            const double qv = qok && k < kh ? q[i] : 0.0, xv = xok && k < kh ? xf : 0.0;
+            acc = SIDE == 0 ? __builtin_amdgcn_mfma_f64_16x16x4f64(qv, xv, acc, 0, 0, 0)
+                            : __builtin_amdgcn_mfma_f64_16x16x4f64(xv, qv, acc, 0, 0, 0);
         }
-        for (int i = threadIdx.x; i < KC2 * GT; i += GEMM_T) {
-            const int kk = i / GT, c = i % GT, k = k0 + kk;
-            if (SIDE == 0) {
-                const int gx = col0 + c;
-                double p = 0.0, q = 0.0;
-                if (kk < kc && gx < cols) {
-                    const double a = xval(gx, k);
-                    if (k < h) {
-                        const double b = xval(gx, n - 1 - k);
-                        p = a + b;
-                        q = a - b;
-                    } else {
-                        p = q = a;
-                    }
-                }
-                Bq[0][kk][c] = p;
-                Bq[SIDE == 0 ? 1 : 0][kk][c] = q;
-            } else {
-                const int gq = col0 + c;
-                Bq[0][kk][c] = (kk < kc && gq < cols) ? Q[(int64_t)k * n + gq] : 0.0;
-            }
-        }
-        __syncthreads();
-        const int kb = ks * (KC2 / KS);
-        const int ia = SIDE == 1 ? (int)odd : 0, ib = SIDE == 0 ? (int)odd : 0;
-#pragma unroll 8
-        for (int kk = 0; kk < KC2 / KS; kk += 2) {
-            acc[0] += Aq[ia][ty][kb + kk] * Bq[ib][kb + kk][tx];
-            acc[1] += Aq[ia][ty][kb + kk + 1] * Bq[ib][kb + kk + 1][tx];
-        }
-        __syncthreads();
     }
-    ps[ks][ty][tx] = acc[0] + acc[1];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ps[w][4 * r + lk][li] = acc[r];
     __syncthreads();
+    const int ty = threadIdx.x / GT, tx = threadIdx.x % GT;
+    const int gr = r0 + rs * ty, gc = c0 + cs * tx;
     double dot = 0.0;
-    if (ks == 0) {
-        const double v = (ps[0][ty][tx] + ps[1][ty][tx]) + (ps[2][ty][tx] + ps[3][ty][tx]);
-        if (gr < rows && gc < cols) {
-            const int64_t oo = (int64_t)gr * cols + gc;
-            if (MODE == 0 || MODE == 3) out[oo] = v;
-            if (MODE == 1) out[oo] = v * W[oo];
-            if (MODE == 2) {
-                out[(int64_t)(gr + 1) * (cols + 2) + gc + 1] = v;
-                dot = v * W[oo];
-            }
+    if (ty < GT && gr < rows && gc < cols) {            // four waves finish the tile
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) v += ps[i][ty][tx];
+        const int64_t oo = (int64_t)gr * cols + gc;
+        if (MODE == 0 || MODE == 3) out[oo] = v;
+        if (MODE == 1) out[oo] = v * W[oo];
+        if (MODE == 2) {
+            out[(int64_t)(gr + 1) * (cols + 2) + gc + 1] = v;
+            dot = v * W[oo];
         }
     }
     if (MODE == 2) {
-        __shared__ double red[GT * GT / 64];
+        __shared__ double red[KS];
         dot = wsum(dot);
-        if (ks == 0 && (threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dot;
+        if (lane == 0) red[w] = dot;                    // (waves 4 and up: zero)
         __syncthreads();
         if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
     }
@@ -441,12 +431,14 @@ int dispatch_p(int p, int dtype, int what, const coarse_args &a) {
     return SIPG_OK;
 }
 
-dim3 gemm_grid(int M, int N) { return dim3((N + GT - 1) / GT, (M + GT - 1) / GT); }
+dim3 tile_grid(int M, int N) { return dim3((N + GT - 1) / GT, (M + GT - 1) / GT); }
 
 // ---- the rocBLAS route for large vertex grids -------------------------------
-// Two-level PCG at p = 8, us per iteration, folded kernel / rocBLAS:
-// 256^2 elements 135.5 / 198.8, 288^2 217.3 / 191.9, 384^2 377.4 / 324.9.
-constexpr int64_t kBlasVertices = 270 * 270;
+// A whole two-level preconditioner application at p = 4, us, folded kernel /
+// rocBLAS: 288 x 288 elements 53.4 / 67.2, 384 x 384 87.2 / 84.0, 448 x 448
+// 108.9 / 121.2, 512 x 512 121.2 / 137.1, 640 x 640 234 / 175, 1024 x 1024
+// 685 / 405.
+constexpr int64_t kBlasVertices = 540 * 540;
 
 // S(a, b): the sum of the four elements' corner sums meeting at interior
 // vertex (a, b) (the gather of dst_gemm_kernel MODE 3), into S (nvy x nvx)
@@ -467,8 +459,7 @@ __global__ __launch_bounds__(VT) void scale_kernel(double *__restrict__ T, const
     for (int64_t i = (int64_t)blockIdx.x * VT + threadIdx.x; i < nv; i += (int64_t)gridDim.x * VT) T[i] *= W[i];
 }
 
-// per-tile sums of S .* C (C the interior of the zero-bordered grid Cpad),
-// on the tiles and in the partial order of dst_gemm_kernel MODE 2
+// per-tile sums of S .* C (C the interior of the zero-bordered grid Cpad)
 __global__ __launch_bounds__(GT * GT) void sc_partials_kernel(const double *__restrict__ S,
                                                               const double *__restrict__ Cpad, int nvy, int nvx,
                                                               double *__restrict__ part) {
@@ -560,17 +551,20 @@ int coarse_solve_blas(int nvy, int nvx, const coarse_tables &c, hipStream_t s) {
         set_last_hip_error(hipErrorLaunchFailure);
         return SIPG_ERR_HIP;
     }
-    hipLaunchKernelGGL(sc_partials_kernel, gemm_grid(nvy, nvx), dim3(GT * GT), 0, s, c.S, c.Cpad, nvy, nvx, c.part);
+    hipLaunchKernelGGL(sc_partials_kernel, tile_grid(nvy, nvx), dim3(GT * GT), 0, s, c.S, c.Cpad, nvy, nvx, c.part);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
+
+// Whether the four products of this vertex grid run as rocBLAS calls.
+bool coarse_by_blas(int nvy, int nvx) { return (int64_t)nvx * nvy >= kBlasVertices && blas().ok(); }
 
 }  // namespace
 
 int coarse_num_partials(int dimx, int dimy) {
     const int nvx = dimx - 1, nvy = dimy - 1;
     if (nvx < 1 || nvy < 1) return 0;
-    const dim3 g = gemm_grid(nvy, nvx);
+    const dim3 g = coarse_by_blas(nvy, nvx) ? tile_grid(nvy, nvx) : dim3(dst_tiles(nvx), (nvy + GT - 1) / GT);
     return (int)(g.x * g.y);
 }
 
@@ -587,17 +581,18 @@ int launch_coarse_solve(int dtype, int p, const void *r, int dimx, int dimy, con
     a.s = s;
     int rc = have_e4 ? SIPG_OK : dispatch_p<1>(p, dtype, 0, a);
     if (rc) return rc;
-    if ((int64_t)nvx * nvy >= kBlasVertices && blas().ok()) return coarse_solve_blas(nvy, nvx, c, s);
-    // T1 = S Qx (S gathered from E4 on the fly, and stored); T2 = (Qy T1) ./
-    // Lambda; T1 = T2 Qx; C = Qy T1 (into Cpad), partials of S.C
-    const dim3 g = gemm_grid(nvy, nvx), b(GEMM_T);
-    hipLaunchKernelGGL((dst_gemm_kernel<1, 3>), g, b, 0, s, c.E4, c.Qx, nvy, nvx, nvx, c.S, c.T1, nullptr, st, slot);
-    hipLaunchKernelGGL((dst_gemm_kernel<0, 1>), g, b, 0, s, c.T1, c.Qy, nvy, nvy, nvx, c.Linv, c.T2, nullptr, st,
-                       slot);
-    hipLaunchKernelGGL((dst_gemm_kernel<1, 0>), g, b, 0, s, c.T2, c.Qx, nvy, nvx, nvx, nullptr, c.T1, nullptr, st,
-                       slot);
-    hipLaunchKernelGGL((dst_gemm_kernel<0, 2>), g, b, 0, s, c.T1, c.Qy, nvy, nvy, nvx, c.S, c.Cpad, c.part, st,
-                       slot);
+    if (coarse_by_blas(nvy, nvx)) return coarse_solve_blas(nvy, nvx, c, s);
+    // T1 = Qy S (S gathered from E4 on the fly, and stored); T2 = (T1 Qx) ./
+    // Lambda; T1 = Qy T2; C = T1 Qx (into Cpad), partials of S.C
+    const dim3 gx(dst_tiles(nvx), (nvy + GT - 1) / GT), gy((nvx + GT - 1) / GT, dst_tiles(nvy));
+    hipLaunchKernelGGL((dst_gemm_kernel<0, 3>), gy, dim3(64 * dst_waves(3)), 0, s, c.E4, c.Qy, nvy, nvy, nvx, c.S, c.T1,
+                       nullptr, st, slot);
+    hipLaunchKernelGGL((dst_gemm_kernel<1, 1>), gx, dim3(64 * dst_waves(1)), 0, s, c.T1, c.Qx, nvy, nvx, nvx, c.Linv,
+                       c.T2, nullptr, st, slot);
+    hipLaunchKernelGGL((dst_gemm_kernel<0, 0>), gy, dim3(64 * dst_waves(0)), 0, s, c.T2, c.Qy, nvy, nvy, nvx, nullptr,
+                       c.T1, nullptr, st, slot);
+    hipLaunchKernelGGL((dst_gemm_kernel<1, 2>), gx, dim3(64 * dst_waves(2)), 0, s, c.T1, c.Qx, nvy, nvx, nvx, c.S,
+                       c.Cpad, c.part, st, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
