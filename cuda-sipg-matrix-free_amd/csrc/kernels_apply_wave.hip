@@ -88,10 +88,17 @@ void apply_kernel_wave(const T *__restrict__ x, T *__restrict__ y, int dimx, int
         const int n = ncol * NQ;
         const T *src = lds + (ey + 1) * BX * NQ;
         T *dst = y + ((size_t)gy * dimx + x0) * NQ;
+        // (all LDS reads first: a read inside the bounds check of its store
+        // would wait for its own round trip nine times over)
+        constexpr int KO = (BX * NQ + 63) / 64;
+        static_assert((BY + 1) * BX * NQ + 64 * KO <= G::LDS, "the last read stays inside the image");
+        T o[KO];
 #pragma unroll
-        for (int k = 0; k < (BX * NQ + 63) / 64; ++k) {
+        for (int k = 0; k < KO; ++k) o[k] = src[lane + 64 * k];
+#pragma unroll
+        for (int k = 0; k < KO; ++k) {
             const int idx = lane + 64 * k;
-            if (idx < n) dst[idx] = src[idx];
+            if (idx < n) dst[idx] = o[k];
         }
     }
     if (DOT) {

@@ -128,21 +128,27 @@ void pcg_rz_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ 
         const int64_t base = g * (int64_t)(NE * NQ);
         T rv[KR];
         double cv[4] = {0.0, 0.0, 0.0, 0.0};
+        // loads first, clamped to the last value instead of guarded: a load
+        // that is used inside its own bounds check waits there, one round
+        // trip after the other
+        T av[KR];
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const int64_t gi = min<int64_t>(base + tid + k * NT, nval - 1);
+            rv[k] = r[gi];
+            if (UPDATE) av[k] = Ap[gi];
+        }
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
             const int idx = tid + k * NT;
-            const int64_t gi = base + idx;
-            T v = T(0);
-            if (idx < G::NV && gi < nval) {
-                v = r[gi];
-                if (UPDATE) {
-                    v = v - alpha * Ap[gi];
-                    r[gi] = v;
-                }
-                srr += (double)v * (double)v;
-            }
+            const bool in = base + idx < nval;
+            T v = rv[k];
+            if (UPDATE) v = v - alpha * av[k];
+            v = in ? v : T(0);
+            if (UPDATE && in) r[base + idx] = v;
+            srr += (double)v * (double)v;
             rv[k] = v;
-            if (idx < G::NV) lds[lds_index<NQ, TS>(idx)] = v;
+            lds[lds_index<NQ, TS>(idx)] = v;
         }
         __syncthreads();
         T *tile = lds + s_el * TS;
@@ -217,16 +223,17 @@ void pcg_rz_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ 
             for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
         }
         __syncthreads();
+        T zv[KR];
+#pragma unroll
+        for (int k = 0; k < KR; ++k) zv[k] = lds[lds_index<NQ, TS>(tid + k * NT)];
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int idx = tid + k * NT;
-            const int64_t gi = base + idx;
-            if (idx < G::NV && gi < nval) {
-                const T zv = lds[lds_index<NQ, TS>(idx)];
-                z[gi] = zv;
-                if (COPYP) pcopy[gi] = zv;
-                srz += (double)rv[k] * (double)zv;
+            const int64_t gi = base + tid + k * NT;
+            if (gi < nval) {
+                z[gi] = zv[k];
+                if (COPYP) pcopy[gi] = zv[k];
             }
+            srz += (double)rv[k] * (double)zv[k];        // rv is zero past the end
         }
         __syncthreads();                               // LDS free for the next group
         if (FUSE && E4) {
@@ -269,7 +276,6 @@ struct RzWave {
     static constexpr int EPW = 64 / N1;
     static constexpr int TS = tile_stride(NQ);
     static constexpr int NV = EPW * NQ;                 // values per run
-    static constexpr int KR = (NV + 63) / 64;
     static constexpr int W = 4;                         // waves per workgroup
     static constexpr int NT = 64 * W;
 };
@@ -291,7 +297,9 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
                         double *__restrict__ prz, cg_state *st, int slot, double *__restrict__ E4)
 {
     using G = RzWave<P>;
-    constexpr int N1 = G::N1, NQ = G::NQ, TS = G::TS, EPW = G::EPW, NV = G::NV, KR = G::KR, NT = G::NT;
+    constexpr int N1 = G::N1, NQ = G::NQ, TS = G::TS, EPW = G::EPW, NV = G::NV, NT = G::NT;
+    constexpr int VL = 16 / (int)sizeof(T), KR = (NV + 64 * VL - 1) / (64 * VL);
+    static_assert(NQ >= VL && (TS == NQ || NQ % VL == 0), "vectors stay inside a tile's LDS image");
     __shared__ __attribute__((aligned(16))) T lds[G::W * EPW * TS];
     __shared__ T linv[NQ];
     __shared__ double csum[RESTR ? G::W * 4 * N1 * EPW : 1];
@@ -331,23 +339,32 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
 
     for (int64_t run = (int64_t)blockIdx.x * G::W + w; run < nrun; run += (int64_t)gridDim.x * G::W) {
         const int64_t base = run * NV;
-        T rv[KR];
+        T rv[KR][VL];
         double cv[4] = {0.0, 0.0, 0.0, 0.0};
+        // The run's nv values in vectors of VL, lane l of chunk k on values
+        // o = VL (l + 64 k) and up; a vector past the end moves back to the
+        // last VL values (the same values written twice, counted once).
+        // All loads are issued before the first is used: guarded one by one
+        // they waited one memory round trip after the other.
+        const int nv = (int)min<int64_t>(NV, nval - base);
+        const T *rb = r + base, *Ab = Ap + (UPDATE ? base : 0);
+        T av[KR][VL];
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int idx = lane + 64 * k;
-            const int64_t gi = base + idx;
-            T v = T(0);
-            if (idx < NV && gi < nval) {
-                v = r[gi];
-                if (UPDATE) {
-                    v = v - alpha * Ap[gi];
-                    r[gi] = v;
-                }
-                srr += (double)v * (double)v;
+            const int idx = min(VL * (lane + 64 * k), nv - VL);
+            load_vec<T, VL>(rb + idx, rv[k]);
+            if (UPDATE) load_vec<T, VL>(Ab + idx, av[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const int o = VL * (lane + 64 * k), idx = min(o, nv - VL);
+#pragma unroll
+            for (int q = 0; q < VL; ++q) {
+                if (UPDATE) rv[k][q] = rv[k][q] - alpha * av[k][q];
+                srr += idx + q >= o ? (double)rv[k][q] * (double)rv[k][q] : 0.0;
             }
-            rv[k] = v;
-            if (idx < NV) wl[lds_index<NQ, TS>(idx)] = v;
+            if (UPDATE) store_vec<T, VL>(r + base + idx, rv[k]);
+            store_vec<T, VL>(wl + lds_index<NQ, TS>(idx), rv[k]);
         }
         wave_sync();
         // 1: column j of S^T R
@@ -405,16 +422,17 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
             }
         }
         wave_sync();
+        T zv[KR][VL];
+#pragma unroll
+        for (int k = 0; k < KR; ++k)
+            load_vec<T, VL>(wl + lds_index<NQ, TS>(min(VL * (lane + 64 * k), nv - VL)), zv[k]);
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int idx = lane + 64 * k;
-            const int64_t gi = base + idx;
-            if (idx < NV && gi < nval) {
-                const T zv = wl[lds_index<NQ, TS>(idx)];
-                z[gi] = zv;
-                if (COPYP) pcopy[gi] = zv;
-                srz += (double)rv[k] * (double)zv;
-            }
+            const int o = VL * (lane + 64 * k), idx = min(o, nv - VL);
+            store_vec<T, VL>(z + base + idx, zv[k]);
+            if (COPYP) store_vec<T, VL>(pcopy + base + idx, zv[k]);
+#pragma unroll
+            for (int q = 0; q < VL; ++q) srz += idx + q >= o ? (double)rv[k][q] * (double)zv[k][q] : 0.0;
         }
         if (RESTR && E4) {
             // E4[c * noe + e]: the lines' shares summed in a fixed order
