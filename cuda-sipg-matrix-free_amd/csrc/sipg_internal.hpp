@@ -210,6 +210,13 @@ int launch_cg_update_xr(int dtype, void *x, const void *p, void *r, const void *
                         cg_state *st, int slot, hipStream_t s, void *xlo = nullptr);
 int launch_cg_update_p(int dtype, const void *r, void *p, int64_t n, const double *part_rr,
                        int np_rr, int nblk, cg_state *st, int slot, hipStream_t s);
+// n_it whole CG iterations of a small problem in one launch
+// (kernels_small.hip), from the slot `slot`; the result is that of n_it
+// times apply, x/r update and p update.  Weak: a build without the kernel
+// iterates by the three launches.
+__attribute__((weak)) bool cg_small_fits(int p, int dimx, int dimy);
+__attribute__((weak)) int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy,
+                                          double pen, int n_it, cg_state *st, int slot, hipStream_t s);
 int launch_residual(int dtype, const void *b, const void *Ax, void *r, int64_t n, hipStream_t s);
 // out = (out dtype)(b - Ax) with b, Ax in in_dtype; optionally p = out;
 // block sums of (b-Ax).(b-Ax) and, when pbb != nullptr, of b.b.

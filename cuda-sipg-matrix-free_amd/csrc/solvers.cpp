@@ -70,6 +70,7 @@ struct Engine {
     parts P{};
     int nb = 0;
     bool fold = false;
+    bool one_group = false;          // chunks of iterations run inside one workgroup
     int64_t launched = 0;
 
     int64_t noe() const { return (int64_t)opI->dimx * opI->dimy; }
@@ -216,7 +217,31 @@ struct Engine {
         return SIPG_OK;
     }
 
+    // Plain CG on a problem that fits one workgroup: iterations without a
+    // replacement run as one launch per chunk.
+    bool small() const {
+        return !pcg && !xL && opI->kernel == SIPG_KERNEL_AUTO && launch_cg_small != nullptr &&
+               cg_small_fits(opI->p, opI->dimx, opI->dimy);
+    }
+
+    // n_it iterations, the first of them replacing when asked
+    int iterations(int n_it, bool replace, bool restart_p) {
+        int rc;
+        for (int c = 0; c < n_it; ++c) {
+            if (one_group && !(replace && c == 0)) {
+                if ((rc = launch_cg_small(opI->dtype, opI->p, xI, r, p, opI->dimx, opI->dimy, opI->pen, n_it - c, st,
+                                          (int)(launched & 1), s)))
+                    return rc;
+                launched += n_it - c;
+                return SIPG_OK;
+            }
+            if ((rc = iteration(replace && c == 0, restart_p))) return rc;
+        }
+        return SIPG_OK;
+    }
+
     int run(sipg_cg_info *info) {
+        one_group = small();
         hipEvent_t ev[2];
         SIPG_HIP_TRY(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
         SIPG_HIP_TRY(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
@@ -227,7 +252,11 @@ struct Engine {
         cg_state cur = hst[0];
         int64_t cur_launched = 0;          // launches reflected in `cur`
         int nrep_enq = 0;
-        int chunk = 4;
+        // (FP32 cycles keep the short ones: their recursion leaves the true
+        // residual within a few iterations of a decade)
+        const bool longer = one_group && opI == opO;
+        int chunk = longer ? 16 : 4;
+        const int near_chunk = longer ? 16 : 8;
         int inflight = 0, buf = 0;
         int64_t pending_launched[2] = {0, 0};
         // adaptive restart: the direction is kept while each true residual
@@ -276,7 +305,8 @@ struct Engine {
         constexpr double kAheadFrac = 0.85;
         const double rr_start = cur.s[0].rr;
         // Each pass: decide on the newest polled state `cur`, enqueue one
-        // chunk of iterations (4 growing to 32; 8 near the tolerance) and a
+        // chunk of iterations (4 growing to 32, 8 near the tolerance; inside one
+        // workgroup, where an iteration is several times shorter, 16 and 16) and a
         // state copy, and block on the older of two outstanding copies.  Iterations past the finish are no-ops on
         // the device, so running one or two chunks ahead costs little.
         for (;;) {
@@ -350,7 +380,7 @@ struct Engine {
             }
             // near the tolerance, short chunks keep the host's lag small
             const bool near = true_stop && cs.rr <= 1e4 * cur.stop * cur.stop;
-            int n_it = near ? std::min(chunk, 8) : chunk;
+            int n_it = near ? std::min(chunk, near_chunk) : chunk;
             const double goal = cur.stop * cur.stop;
             // drain: this pass waits for the newest state copy (the device
             // idles for one host round trip), not the older one
@@ -378,9 +408,7 @@ struct Engine {
                 drain = true;
                 n_it = 1;
             }
-            for (int c = 0; c < n_it; ++c)
-                if ((rc = iteration(want_rep && c == 0, restart_p))) break;
-            if (rc) break;
+            if ((rc = iterations(n_it, want_rep, restart_p))) break;
             if (want_rep) {
                 ++nrep_enq;
                 check_pending = true;
