@@ -66,12 +66,6 @@ typedef double dd4 __attribute__((ext_vector_type(4)));
 __host__ __device__ constexpr int dst_tiles_even(int n) { return ((n + 1) / 2 + GT - 1) / GT; }
 __host__ __device__ constexpr int dst_tiles(int n) { return dst_tiles_even(n) + (n / 2 + GT - 1) / GT; }
 
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // E4[c * noe + e] = sum_nodes r(e, i1, i2) wx_c(i1) wy_c(i2); corner c = 0
 // bottom-left, 1 bottom-right, 2 top-left, 3 top-right; wx = 1 - xi or xi,
 // wy = 1 - xi or xi (xi = (z+1)/2: x from the element's left, y from its
@@ -215,7 +209,7 @@ __global__ __launch_bounds__(64 * dst_waves(MODE)) void dst_gemm_kernel(const do
     }
     if (MODE == 2) {
         __shared__ double red[KS];
-        dot = wsum(dot);
+        dot = wave_total(dot);
         if (lane == 0) red[w] = dot;                    // (waves 4 and up: zero)
         __syncthreads();
         if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
@@ -468,7 +462,7 @@ __global__ __launch_bounds__(GT * GT) void sc_partials_kernel(const double *__re
     const int gr = blockIdx.y * GT + ty, gc = blockIdx.x * GT + tx;
     double dot = 0.0;
     if (gr < nvy && gc < nvx) dot = S[(int64_t)gr * nvx + gc] * Cpad[(int64_t)(gr + 1) * (nvx + 2) + gc + 1];
-    dot = wsum(dot);
+    dot = wave_total(dot);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dot;
     __syncthreads();
     if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);

@@ -14,7 +14,7 @@
 //
 // Bound: latency of four barriers and the dependent LDS reads between them.
 // Measured 8 x 8, p = 3 (1,024 unknowns): 15 -> 3.1 us per iteration, a solve
-// to 1e-10 3.17 -> 0.64 ms.  kSmallMax: three arrays of 4,096 padded values fill the
+// to 1e-10 2.8 -> 0.56 ms.  kSmallMax: three arrays of 4,096 padded values fill the
 // LDS; there (16 x 16, p = 3 and 4 x 4, p = 15) the
 // workgroup takes 4.9 and 4.1 us per iteration against 14.0 and 19.5 for the launches.
 #include "line_math.hpp"
@@ -28,37 +28,14 @@ constexpr int kSmallMax = 4096;      // unknowns
 constexpr int NT = 512;              // threads: eight waves
 constexpr int KR = kSmallMax / NT;   // values per thread
 
-// Sum over the wave in lane order of the row shifts: rows of 16 lanes, then
-// across rows; the total is read from lane 63.  (Register moves inside the
-// SIMD: a cross-lane exchange through LDS costs several times as much, six
-// times over.)
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
-    return v + __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double wave_total(double v) {
-    v = dpp_add<0x111, 0xf>(v);      // row_shr:1
-    v = dpp_add<0x112, 0xf>(v);      // row_shr:2
-    v = dpp_add<0x114, 0xf>(v);      // row_shr:4
-    v = dpp_add<0x118, 0xf>(v);      // row_shr:8: lane 15 of each row holds its sum
-    v = dpp_add<0x142, 0xa>(v);      // row_bcast:15 into rows 1 and 3
-    v = dpp_add<0x143, 0xc>(v);      // row_bcast:31 into rows 2 and 3
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
-                            __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
-
 // One barrier: the waves' sums cross through red, which alternates between
 // two buffers, and every thread adds them in the same order.
 __device__ __forceinline__ double group_total(double v, double *red) {
     v = wave_total(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) s += red[i];
-    return s;
+    static_assert(NT == 512, "a tree over eight waves: three dependent adds");
+    return ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
 }
 
 template <typename T, int P>

