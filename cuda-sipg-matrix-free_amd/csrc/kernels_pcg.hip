@@ -32,26 +32,6 @@ namespace sipg_internal {
 
 namespace {
 
-// elements per workgroup group; thread (s, j) owns line j of element s
-template <int P>
-struct PcgShape {
-    static constexpr int N1 = P + 1;
-    static constexpr int NE = N1 > 16 ? 32 : 64;
-    static constexpr int NT = NE * N1;
-    static constexpr int NQ = N1 * N1;
-    static constexpr int TS = tile_stride(NQ);
-    static constexpr int NV = NE * NQ;                  // values per group
-    static constexpr int KR = (NV + NT - 1) / NT;       // = N1
-};
-
-// The restriction's line shares (4 (p+1) doubles per element) are summed in
-// the element tiles' LDS once z has left it, where they fit: FP64 from
-// p = 3, FP32 from p = 7; elsewhere the separate restriction kernel runs.
-// es: bytes per value.
-__host__ __device__ constexpr bool rz_fuses_restrict(int p, int es) {
-    return 4 * (p + 1) * 8 <= tile_stride((p + 1) * (p + 1)) * es;
-}
-
 // Sum over the workgroup, returned to every thread (fixed order).
 template <int NT>
 __device__ __forceinline__ double group_sum_all(double v, double *red, double *total) {
@@ -63,7 +43,8 @@ __device__ __forceinline__ double group_sum_all(double v, double *red, double *t
     return out;
 }
 
-// z = M^-1 r over every element, with the block sums of r.r and r.z.
+// ---- z = M^-1 r -----------------------------------------------------------
+// Over every element, with the block sums of r.r and r.z.
 //   UPDATE: first r -= alpha Ap with alpha = slot.rz / p.Ap (the p.Ap block
 //   sums of this iteration's apply), r written back -- the r half of the
 //   reference's alpha step; returns at once when the slot is finished.
@@ -74,238 +55,36 @@ __device__ __forceinline__ double group_sum_all(double v, double *red, double *t
 //   pen = 5 (p+1)^2 (prec is then unused); otherwise they are read from prec.
 //   RESTR: with E4, also the two-level restriction's corner sums (its own
 //   instantiation, so that the plain kernel keeps its registers).
-template <typename T, int P, bool UPDATE, bool COPYP, bool CX, bool RESTR = false>
-__global__ __launch_bounds__(PcgShape<P>::NT)
-void pcg_rz_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ z,
-                   T *__restrict__ pcopy, int64_t noe, const T *__restrict__ prec,
-                   const double *__restrict__ ppAp, int np, double *__restrict__ prr,
-                   double *__restrict__ prz, cg_state *st, int slot, double *__restrict__ E4)
-{
-    using G = PcgShape<P>;
-    constexpr int N1 = G::N1, NQ = G::NQ, TS = G::TS, NE = G::NE, NT = G::NT, KR = G::KR;
-    __shared__ __attribute__((aligned(16))) T lds[NE * TS];
-    __shared__ double red[(NT + 63) / 64];
-    __shared__ double total;
-    // with E4 (the two-level preconditioner's restriction): each line's
-    // share of its element's four corner-weighted sums, per corner c
-    // (0 bottom-left, 1 bottom-right, 2 top-left, 3 top-right), held in
-    // registers and summed over the lines in the tile LDS at the end
-    constexpr bool FUSE = RESTR && rz_fuses_restrict(P, (int)sizeof(T));
-    constexpr cx::Tables<P> TB = cx::make_tables<P>();
-
-    T alpha = T(0);
-    if (UPDATE) {
-        if (st->s[slot].done | st->err) return;
-        const double pAp = group_sum_all<NT>(strided_sum<NT>(ppAp, 0, np), red, &total);
-        const double a = st->s[slot].rz / pAp;
-        if (!(pAp > 0.0) || !isfinite(a)) {
-            // every workgroup takes this branch (same p.Ap); the first
-            // records it in a word that the p update reads afterwards
-            if (blockIdx.x == 0 && threadIdx.x == 0) st->err = isfinite(pAp) ? 2 : 3;
-            return;
-        }
-        alpha = (T)a;
-        if (blockIdx.x == 0 && threadIdx.x == 0) st->s[slot].alpha = a;    // for the p update
-    }
-    constexpr cx::PrecTables<P> PT = cx::make_prec<P>();
-    struct CS {
-        const T *p;
-        __device__ T operator()(int i, int a) const { return CX ? (T)PT.S[i][a] : p[i * N1 + a]; }
-    } S{prec};
-    struct CL {
-        const T *p;
-        __device__ T operator()(int a, int c) const { return CX ? (T)PT.Linv[a][c] : p[a * N1 + c]; }
-    } Linv{prec + NQ};
-    const int tid = threadIdx.x;
-    const int s_el = tid % NE;
-    int j = tid / NE;
-    if (NE % 64 == 0) j = __builtin_amdgcn_readfirstlane(j);
-    const int64_t nval = noe * NQ;
-    const int64_t ngroups = (noe + NE - 1) / NE;
-    double srr = 0.0, srz = 0.0;
-
-    for (int64_t g = blockIdx.x; g < ngroups; g += gridDim.x) {
-        const int64_t base = g * (int64_t)(NE * NQ);
-        T rv[KR];
-        double cv[4] = {0.0, 0.0, 0.0, 0.0};
-        // loads first, clamped to the last value instead of guarded: a load
-        // that is used inside its own bounds check waits there, one round
-        // trip after the other
-        T av[KR];
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int64_t gi = min<int64_t>(base + tid + k * NT, nval - 1);
-            rv[k] = r[gi];
-            if (UPDATE) av[k] = Ap[gi];
-        }
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int idx = tid + k * NT;
-            const bool in = base + idx < nval;
-            T v = rv[k];
-            if (UPDATE) v = v - alpha * av[k];
-            v = in ? v : T(0);
-            if (UPDATE && in) r[base + idx] = v;
-            srr += (double)v * (double)v;
-            rv[k] = v;
-            lds[lds_index<NQ, TS>(idx)] = v;
-        }
-        __syncthreads();
-        T *tile = lds + s_el * TS;
-        // 1: column j of S^T R
-        {
-            T c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-            if (FUSE && E4) {
-                // column j is the x line r(., j) at y node j: x weights here,
-                // the y weight of line j, summed over the lines below
-                double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-                for (int i = 0; i < N1; ++i) {
-                    const double xi = 0.5 * (TB.z[i] + 1.0);
-                    a0 += (1.0 - xi) * (double)c[i];
-                    a1 += xi * (double)c[i];
-                }
-                const double eta = 0.5 * (TB.z[j] + 1.0);
-                cv[0] = (1.0 - eta) * a0;
-                cv[1] = (1.0 - eta) * a1;
-                cv[2] = eta * a0;
-                cv[3] = eta * a1;
-            }
-#pragma unroll
-            for (int a = 0; a < N1; ++a) {
-                T acc = T(0);
-#pragma unroll
-                for (int i = 0; i < N1; ++i) acc += S(i, a) * c[i];
-                t[a] = acc;
-            }
-#pragma unroll
-            for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
-        }
-        __syncthreads();
-        // 2: row j of ((S^T R S) ./ L) S^T
-        {
-            T w[N1], v[N1];
-#pragma unroll
-            for (int b = 0; b < N1; ++b) w[b] = tile[j * N1 + b];
-#pragma unroll
-            for (int c = 0; c < N1; ++c) {
-                T acc = T(0);
-#pragma unroll
-                for (int b = 0; b < N1; ++b) acc += w[b] * S(b, c);
-                v[c] = acc * Linv(j, c);
-            }
-#pragma unroll
-            for (int d = 0; d < N1; ++d) {
-                T acc = T(0);
-#pragma unroll
-                for (int c = 0; c < N1; ++c) acc += v[c] * S(d, c);
-                w[d] = acc;
-            }
-#pragma unroll
-            for (int d = 0; d < N1; ++d) tile[j * N1 + d] = w[d];
-        }
-        __syncthreads();
-        // 3: column j of S (...)
-        {
-            T c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-#pragma unroll
-            for (int a = 0; a < N1; ++a) {
-                T acc = T(0);
-#pragma unroll
-                for (int i = 0; i < N1; ++i) acc += S(a, i) * c[i];
-                t[a] = acc;
-            }
-#pragma unroll
-            for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
-        }
-        __syncthreads();
-        T zv[KR];
-#pragma unroll
-        for (int k = 0; k < KR; ++k) zv[k] = lds[lds_index<NQ, TS>(tid + k * NT)];
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int64_t gi = base + tid + k * NT;
-            if (gi < nval) {
-                z[gi] = zv[k];
-                if (COPYP) pcopy[gi] = zv[k];
-            }
-            srz += (double)rv[k] * (double)zv[k];        // rv is zero past the end
-        }
-        __syncthreads();                               // LDS free for the next group
-        if (FUSE && E4) {
-            // E4[c * noe + e]: the lines' shares summed in a fixed order
-            double *cs = reinterpret_cast<double *>(lds);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) cs[(c * N1 + j) * NE + s_el] = cv[c];
-            __syncthreads();
-            for (int q = tid; q < 4 * NE; q += NT) {
-                const int c = q / NE, el = q - (q / NE) * NE;
-                const int64_t e = g * NE + el;
-                double sum = 0.0;
-#pragma unroll
-                for (int jj = 0; jj < N1; ++jj) sum += cs[(c * N1 + jj) * NE + el];
-                if (e < noe) E4[(int64_t)c * noe + e] = sum;
-            }
-            __syncthreads();
-        }
-    }
-    const double a = block_sum<NT>(srr, red);
-    __syncthreads();
-    const double b = block_sum<NT>(srz, red);
-    if (threadIdx.x == 0) {
-        prr[blockIdx.x] = a;
-        prz[blockIdx.x] = b;
-    }
-}
-
-// ---- z = M^-1 r with wave-owned elements ----------------------------------
-// The same preconditioner and pass structure with another work split: a
-// wave holds EPW = 64 / (p+1) whole elements (7 at p = 8), lane (s, j) =
-// s (p+1) + j on line j of element s, and streams runs of EPW consecutive
-// elements on its own.  The transposes between the three contraction
-// passes stay inside the wave, so the element loop has no workgroup barrier;
-// with the standard penalty the contractions take the even-odd form of S
+// A wave streams runs of EPW consecutive elements on its own
+// (prec_block.hpp): the transposes between the three contraction passes stay
+// inside the wave, so the element loop has no workgroup barrier; with the
+// standard penalty the contractions take the even-odd form of S
 // (cx::PrecEvenOdd), half the multiplies of the plain one.
-template <int P>
-struct RzWave {
-    static constexpr int N1 = P + 1, NQ = N1 * N1;
-    static constexpr int EPW = 64 / N1;
-    static constexpr int TS = tile_stride(NQ);
-    static constexpr int NV = EPW * NQ;                 // values per run
-    static constexpr int W = 4;                         // waves per workgroup
-    static constexpr int NT = 64 * W;
-};
+//
+// Bound: memory at p = 8 (four passes: 28 us cached, 36 us inside a solve
+// whose vectors do not all stay in the last-level cache); at high degree the
+// LDS transposes, whose rows are padded to an odd stride: FP32 p = 15
+// (128 x 128) 21.0 -> 17.9 us.  A workgroup-wide split that had the small
+// degrees before was up to 15 % faster there than the wave's 8-byte accesses,
+// and is slower than these: block-Jacobi PCG at p = 1 (1118 x 1118) 100.7 ->
+// 83.5 us an iteration, p = 3 97.2 -> 82.7, FP32 p = 7 (279 x 279) 66 -> 52.
+constexpr int kRzWaves = 4, kRzThreads = 64 * kRzWaves;       // per workgroup
 
-// LDS writes of one pass are visible to every lane of the wave in the next
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// Arguments and flags as pcg_rz_kernel; RESTR: with E4, the restriction's
-// corner sums (for every degree: they are summed in an LDS array of their
-// own).
 template <typename T, int P, bool UPDATE, bool COPYP, bool CX, bool RESTR = false>
-__global__ __launch_bounds__(RzWave<P>::NT)
-void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ z,
+__global__ __launch_bounds__(kRzThreads)
+void pcg_rz_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restrict__ z,
                         T *__restrict__ pcopy, int64_t noe, const T *__restrict__ prec,
                         const double *__restrict__ ppAp, int np, double *__restrict__ prr,
                         double *__restrict__ prz, cg_state *st, int slot, double *__restrict__ E4)
 {
-    using G = RzWave<P>;
-    constexpr int N1 = G::N1, NQ = G::NQ, TS = G::TS, EPW = G::EPW, NV = G::NV, NT = G::NT;
-    constexpr int VL = 16 / (int)sizeof(T), KR = (NV + 64 * VL - 1) / (64 * VL);
-    static_assert(NQ >= VL && (TS == NQ || NQ % VL == 0), "vectors stay inside a tile's LDS image");
-    __shared__ __attribute__((aligned(16))) T lds[G::W * EPW * TS];
+    using G = RunGeo<T, P>;
+    constexpr int N1 = G::N1, NQ = G::NQ, EPW = G::EPW, NV = G::NV, W = kRzWaves, NT = kRzThreads;
+    __shared__ __attribute__((aligned(16))) T lds[W * G::BUF];
     __shared__ T linv[NQ];
-    __shared__ double csum[RESTR ? G::W * 4 * N1 * EPW : 1];
-    __shared__ double red[G::W];
+    __shared__ double csum[RESTR ? W * 2 * 64 : 1];
+    __shared__ double eta[N1];
+    __shared__ double red[W];
     __shared__ double total;
-    using TB = cx::Basis<P>;                           // TB::T.z: the nodes (a lane's own j: a load)
 
     T alpha = T(0);
     if (UPDATE) {
@@ -324,134 +103,46 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
         if constexpr (CX) linv[q] = (T)PrecEO<P>::V.Linv[q / N1][q % N1];
         else linv[q] = prec[NQ + q];
     }
+    if (RESTR && threadIdx.x < N1) eta[threadIdx.x] = 0.5 * (cx::Basis<P>::T.z[threadIdx.x] + 1.0);
     __syncthreads();
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int s = lane / N1, j = lane - s * N1;
-    const bool act = s < EPW;                          // lanes past the last element: copies, no writes
-    T *wl = lds + w * (EPW * TS);
-    T *tile = wl + (act ? s : EPW - 1) * TS;
-    const T *lrow = linv + j * N1;
     const int64_t nval = noe * NQ;
     const int64_t nrun = (noe + EPW - 1) / EPW;
     double srr = 0.0, srz = 0.0;
-
-    for (int64_t run = (int64_t)blockIdx.x * G::W + w; run < nrun; run += (int64_t)gridDim.x * G::W) {
+    for (int64_t run = (int64_t)blockIdx.x * W + w; run < nrun; run += (int64_t)gridDim.x * W) {
         const int64_t base = run * NV;
-        T rv[KR][VL];
-        double cv[4] = {0.0, 0.0, 0.0, 0.0};
-        // The run's nv values in vectors of VL, lane l of chunk k on values
-        // o = VL (l + 64 k) and up; a vector past the end moves back to the
-        // last VL values (the same values written twice, counted once).
-        // All loads are issued before the first is used: guarded one by one
-        // they waited one memory round trip after the other.
         const int nv = (int)min<int64_t>(NV, nval - base);
-        const T *rb = r + base, *Ab = Ap + (UPDATE ? base : 0);
-        T av[KR][VL];
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int idx = min(VL * (lane + 64 * k), nv - VL);
-            load_vec<T, VL>(rb + idx, rv[k]);
-            if (UPDATE) load_vec<T, VL>(Ab + idx, av[k]);
-        }
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int o = VL * (lane + 64 * k), idx = min(o, nv - VL);
-#pragma unroll
-            for (int q = 0; q < VL; ++q) {
-                if (UPDATE) rv[k][q] = rv[k][q] - alpha * av[k][q];
-                srr += idx + q >= o ? (double)rv[k][q] * (double)rv[k][q] : 0.0;
-            }
-            if (UPDATE) store_vec<T, VL>(r + base + idx, rv[k]);
-            store_vec<T, VL>(wl + lds_index<NQ, TS>(idx), rv[k]);
-        }
-        wave_sync();
-        // 1: column j of S^T R
-        {
-            T c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-            if (RESTR && E4) {
-                // column j is the x line r(., j) at y node j: x weights here,
-                // the y weight of line j, summed over the lines below
-                double a0 = 0.0, a1 = 0.0;
-#pragma unroll
-                for (int i = 0; i < N1; ++i) {
-                    const double xi = 0.5 * (TB::T.z[i] + 1.0);
-                    a0 += (1.0 - xi) * (double)c[i];
-                    a1 += xi * (double)c[i];
-                }
-                const double eta = 0.5 * (TB::T.z[j] + 1.0);
-                cv[0] = (1.0 - eta) * a0;
-                cv[1] = (1.0 - eta) * a1;
-                cv[2] = eta * a0;
-                cv[3] = eta * a1;
-            }
-            contract_st<T, P, CX>(prec, c, t);
-            if (act) {
-#pragma unroll
-                for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
-            }
-        }
-        wave_sync();
-        // 2: row j of ((S^T R S) ./ L) S^T
-        {
-            T wv[N1], v[N1];
-#pragma unroll
-            for (int b = 0; b < N1; ++b) wv[b] = tile[j * N1 + b];
-            contract_st<T, P, CX>(prec, wv, v);
-#pragma unroll
-            for (int c = 0; c < N1; ++c) v[c] *= lrow[c];
-            contract_s<T, P, CX>(prec, v, wv);
-            if (act) {
-#pragma unroll
-                for (int d = 0; d < N1; ++d) tile[j * N1 + d] = wv[d];
-            }
-        }
-        wave_sync();
-        // 3: column j of S (...)
-        {
-            T c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-            contract_s<T, P, CX>(prec, c, t);
-            if (act) {
-#pragma unroll
-                for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
-            }
-        }
-        wave_sync();
-        T zv[KR][VL];
-#pragma unroll
-        for (int k = 0; k < KR; ++k)
-            load_vec<T, VL>(wl + lds_index<NQ, TS>(min(VL * (lane + 64 * k), nv - VL)), zv[k]);
-#pragma unroll
-        for (int k = 0; k < KR; ++k) {
-            const int o = VL * (lane + 64 * k), idx = min(o, nv - VL);
-            store_vec<T, VL>(z + base + idx, zv[k]);
-            if (COPYP) store_vec<T, VL>(pcopy + base + idx, zv[k]);
-#pragma unroll
-            for (int q = 0; q < VL; ++q) srz += idx + q >= o ? (double)rv[k][q] * (double)zv[k][q] : 0.0;
-        }
+        double x0 = 0.0, x1 = 0.0;
+        prec_run<T, P, UPDATE, COPYP, CX, RESTR>(r + base, r + base, UPDATE ? Ap + base : nullptr, z + base,
+                                                 COPYP ? pcopy + base : nullptr, nv, [&] { return alpha; }, prec,
+                                                 linv, lds + w * G::BUF, lane, srr, srz, x0, x1);
         if (RESTR && E4) {
-            // E4[c * noe + e]: the lines' shares summed in a fixed order
-            double *cs = csum + w * (4 * N1 * EPW);
-            if (act) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) cs[(c * N1 + j) * EPW + s] = cv[c];
-            }
-            wave_sync();
-            for (int q = lane; q < 4 * EPW; q += 64) {
-                const int c = q / EPW, el = q - c * EPW;
+            // E4[c * noe + e]: the lines' x sums, weighted in y, in a fixed
+            // order; corner c = 0 bottom-left, 1 bottom-right, 2 top-left, 3
+            // top-right (lane q: element q / 2, x half q % 2)
+            double *cs = csum + w * 128;
+            cs[lane] = x0;
+            cs[64 + lane] = x1;
+            run_sync();
+            if (lane < 2 * EPW) {
+                const int el = lane >> 1, h = lane & 1;
                 const int64_t e = run * EPW + el;
-                double sum = 0.0;
+                double lo = 0.0, hi = 0.0;
 #pragma unroll
-                for (int jj = 0; jj < N1; ++jj) sum += cs[(c * N1 + jj) * EPW + el];
-                if (e < noe) E4[(int64_t)c * noe + e] = sum;
+                for (int jj = 0; jj < N1; ++jj) {
+                    const double v = cs[64 * h + el * N1 + jj];
+                    lo += (1.0 - eta[jj]) * v;
+                    hi += eta[jj] * v;
+                }
+                if (e < noe) {
+                    E4[(int64_t)h * noe + e] = lo;
+                    E4[(int64_t)(2 + h) * noe + e] = hi;
+                }
             }
+            run_sync();
         }
-        wave_sync();                                   // the wave's LDS is free for its next run
     }
     const double a = block_sum<NT>(srr, red);
     __syncthreads();
@@ -460,15 +151,6 @@ void pcg_rz_wave_kernel(T *__restrict__ r, const T *__restrict__ Ap, T *__restri
         prr[blockIdx.x] = a;
         prz[blockIdx.x] = b;
     }
-}
-
-// Which split z = M^-1 r takes at degree p with es bytes per value: the
-// wave-owned one where it measured faster (z = M^-1 r over ~5.3M values on
-// MI355X, FP64: 23.9 against 28.5 us at p = 8, 31.3 against 68.5 at
-// p = 16; FP32 likewise at p = 4, 6 and from 8), the workgroup-wide one
-// below (up to 15 % faster there: p <= 3, and FP32 at p = 5, 7).
-__host__ __device__ constexpr bool rz_by_wave(int p, int es) {
-    return es == 8 ? p >= 4 : (p == 4 || p == 6 || p >= 8);
 }
 
 // Workgroups of one pcg_rz kernel that the device holds at once, cached per
@@ -483,63 +165,40 @@ int pcg_resident() {
     if (g > 0) return g;
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
-    hipError_t e;
-    if constexpr (rz_by_wave(P, (int)sizeof(T)))
-        // the instantiation that also restricts (more registers) where it exists
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&pcg_rz_wave_kernel<T, P, UPDATE, COPYP, CX, CX>), RzWave<P>::NT, 0);
-    else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&pcg_rz_kernel<T, P, UPDATE, COPYP, CX>), PcgShape<P>::NT, 0);
+    // the instantiation that also restricts (more registers) where it exists
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per, reinterpret_cast<const void *>(&pcg_rz_kernel<T, P, UPDATE, COPYP, CX, CX>), kRzThreads, 0);
     if (e != hipSuccess) per = 0;
     g = (cus > 0 ? cus : 1) * (per > 0 ? per : 1);
     cache[dev].store(g, std::memory_order_relaxed);
     return g;
 }
 
-// The wave-owned split: W runs of EPW elements per workgroup and pass, in
-// as many passes as it takes for the grid to fit on the device at once
-// (at most kMaxPartials workgroups), with the runs spread evenly over the
-// passes.  Fewer workgroups also means fewer block sums for the kernels
-// that reduce them afterwards (each of their workgroups reads all of them).
+// One run of EPW elements per wave and pass, in as many passes as it takes
+// for the grid to fit on the device at once (at most kMaxPartials
+// workgroups), with the runs spread evenly over the passes.  Fewer
+// workgroups also means fewer block sums for the kernels that reduce them
+// afterwards (each of their workgroups reads all of them).
 template <typename T, int P, bool UPDATE, bool COPYP, bool CX>
 int pcg_grid(int64_t noe) {
-    if constexpr (rz_by_wave(P, (int)sizeof(T))) {
-        using G = RzWave<P>;
-        const int64_t runs = (noe + G::EPW - 1) / G::EPW;
-        const int64_t wgs = std::max<int64_t>(1, (runs + G::W - 1) / G::W);
-        const int64_t cap = std::min<int64_t>(pcg_resident<T, P, UPDATE, COPYP, CX>(), kMaxPartials);
-        const int64_t rounds = (wgs + cap - 1) / cap;
-        return (int)((wgs + rounds - 1) / rounds);
-    } else {
-        const int64_t groups = (noe + PcgShape<P>::NE - 1) / PcgShape<P>::NE;
-        return (int)std::min<int64_t>(std::min<int64_t>(groups, pcg_resident<T, P, UPDATE, COPYP, CX>()),
-                                      kMaxPartials);
-    }
+    const int64_t epw = RunGeo<T, P>::EPW, runs = (noe + epw - 1) / epw;
+    const int64_t wgs = std::max<int64_t>(1, (runs + kRzWaves - 1) / kRzWaves);
+    const int64_t cap = std::min<int64_t>(pcg_resident<T, P, UPDATE, COPYP, CX>(), kMaxPartials);
+    const int64_t rounds = (wgs + cap - 1) / cap;
+    return (int)((wgs + rounds - 1) / rounds);
 }
 
 // grid: that of the plain kernel (the block-sum count the solver expects);
-// with E4 on a degree where it fits, the restricting instantiation
+// with E4, the restricting instantiation
 template <typename T, int P, bool UPDATE, bool COPYP, bool CX>
 void rz_launch(dim3 grid, void *r, const void *Ap, void *z, void *pcopy, int64_t noe, const void *prec,
                const double *ppAp, int np, double *prr, double *prz, cg_state *st, int slot, double *E4,
                hipStream_t s) {
-    if constexpr (rz_by_wave(P, (int)sizeof(T))) {
-        if (CX && E4)
-            hipLaunchKernelGGL((pcg_rz_wave_kernel<T, P, UPDATE, COPYP, CX, CX>), grid, dim3(RzWave<P>::NT), 0, s,
-                               (T *)r, (const T *)Ap, (T *)z, (T *)pcopy, noe, (const T *)prec, ppAp, np, prr, prz,
-                               st, slot, E4);
-        else
-            hipLaunchKernelGGL((pcg_rz_wave_kernel<T, P, UPDATE, COPYP, CX>), grid, dim3(RzWave<P>::NT), 0, s,
-                               (T *)r, (const T *)Ap, (T *)z, (T *)pcopy, noe, (const T *)prec, ppAp, np, prr, prz,
-                               st, slot, nullptr);
-        return;
-    }
-    if (CX && E4 && rz_fuses_restrict(P, (int)sizeof(T)))
-        hipLaunchKernelGGL((pcg_rz_kernel<T, P, UPDATE, COPYP, CX, CX>), grid, dim3(PcgShape<P>::NT), 0, s, (T *)r,
+    if (CX && E4)
+        hipLaunchKernelGGL((pcg_rz_kernel<T, P, UPDATE, COPYP, CX, CX>), grid, dim3(kRzThreads), 0, s, (T *)r,
                            (const T *)Ap, (T *)z, (T *)pcopy, noe, (const T *)prec, ppAp, np, prr, prz, st, slot, E4);
     else
-        hipLaunchKernelGGL((pcg_rz_kernel<T, P, UPDATE, COPYP, CX>), grid, dim3(PcgShape<P>::NT), 0, s, (T *)r,
+        hipLaunchKernelGGL((pcg_rz_kernel<T, P, UPDATE, COPYP, CX>), grid, dim3(kRzThreads), 0, s, (T *)r,
                            (const T *)Ap, (T *)z, (T *)pcopy, noe, (const T *)prec, ppAp, np, prr, prz, st, slot,
                            nullptr);
 }
@@ -774,8 +433,8 @@ int pcg_num_blocks(int dtype, int p, double pen, int mode, int64_t noe) {
 }
 
 bool pcg_rz_fuses_restrict(int dtype, int p, double pen) {
-    const int es = dtype == SIPG_F64 ? 8 : 4;
-    return p >= 1 && p <= kMaxDegree && standard_pen(p, pen) && (rz_by_wave(p, es) || rz_fuses_restrict(p, es));
+    (void)dtype;
+    return p >= 1 && p <= kMaxDegree && standard_pen(p, pen);
 }
 
 int launch_pcg_rz(int dtype, int p, double pen, int mode, void *r, const void *Ap, void *z, void *pcopy,

@@ -245,8 +245,7 @@ int launch_mark_replaced(cg_state *st, int slot, int restart, hipStream_t s);
 int pcg_num_blocks(int dtype, int p, double pen, int mode, int64_t noe);
 // E4 non-null: also the two-level restriction's corner sums of r (as
 // launch_coarse_solve's first step), from the same read of r, where
-// pcg_rz_fuses_restrict (the standard penalty's kernels, where the LDS has
-// room); ignored elsewhere
+// pcg_rz_fuses_restrict (the standard penalty's kernels); ignored elsewhere
 bool pcg_rz_fuses_restrict(int dtype, int p, double pen);
 int launch_pcg_rz(int dtype, int p, double pen, int mode, void *r, const void *Ap, void *z, void *pcopy,
                   int64_t noe, const void *prec, const double *part_pAp, int np_pAp, double *part_rr,
