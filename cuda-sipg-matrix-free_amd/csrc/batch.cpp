@@ -6,10 +6,11 @@
 // are concatenated (element-major within an instance).  The solver runs
 // every instance's CG in the same launches:
 //
-//   per iteration  one fused apply + p.Ap launch per degree present (over a
-//                  device list of (instance, block) items), then alpha per
+//   per iteration  one fused apply + p.Ap launch (over device lists, one to a
+//                  degree, of (instance, block) items), then alpha per
 //                  instance, x/r update (+ r.r per chunk), beta per instance
-//                  and the p update, over device lists of chunks;
+//                  and the p update, over device lists of chunks; PCG has
+//                  two launches after the operator's (kernels_batch_pcg.hip);
 //   hipGraph       kGraphIters iterations are captured once per solve and
 //                  replayed; the lists and their lengths live in device
 //                  memory, so shrinking them as instances finish keeps the
@@ -107,10 +108,11 @@ struct sipg_batch {
 namespace {
 
 int items_for(const sipg_batch &b, int i, int shape, std::vector<batch_item> &out) {
-    const int BX = kBatchShapeBX[shape], BY = kBatchShapeBY[shape];
+    int BX, BY;
+    batch_extent(b.p[i], shape, &BX, &BY);
     const int nbx = (b.dimx[i] + BX - 1) / BX, nby = (b.dimy[i] + BY - 1) / BY;
     for (int by = 0; by < nby; ++by)
-        for (int bx = 0; bx < nbx; ++bx) out.push_back({i, bx * BX, by * BY, 0});
+        for (int bx = 0; bx < nbx; ++bx) out.push_back({i, bx * BX, by * BY, BY});
     return nbx * nby;
 }
 
@@ -173,12 +175,25 @@ int upload_lists(sipg_batch &b, int set, const Lists &L) {
     return SIPG_OK;
 }
 
-// y = A x over the instances of a list set (no p.Ap)
-int apply_set(sipg_batch &b, int set, const double *x, double *y) {
+batch_groups groups_of(sipg_batch &b, int set) {
+    batch_groups G;
+    G.n = (int)b.groups.size();
+    for (int g = 0; g < G.n; ++g)
+        G.g[g] = {b.groups[g].d_items[set], b.count(set, 2 + g), b.groups[g].base, b.groups[g].p};
+    return G;
+}
+
+// y = A x over the instances of a list set; with p.Ap, of those that have
+// not finished at `slot`
+int apply_set(sipg_batch &b, int set, const double *x, double *y, double *item_part = nullptr, int slot = 0) {
+    const cg_state *st = item_part ? b.d_state : nullptr;
+    if (launch_batch_apply_groups)
+        return launch_batch_apply_groups(groups_of(b, set), b.item_total, x, y, b.d_inst, item_part, st, slot,
+                                         b.stream);
     for (size_t g = 0; g < b.groups.size(); ++g) {
         auto &G = b.groups[g];
         int rc = launch_batch_apply(G.p, G.shape, x, y, b.d_inst, G.d_items[set], b.count(set, 2 + (int)g),
-                                    G.cap, nullptr, nullptr, 0, b.stream);
+                                    G.cap, item_part ? item_part + G.base : nullptr, st, slot, b.stream);
         if (rc) return rc;
     }
     return SIPG_OK;
@@ -186,6 +201,9 @@ int apply_set(sipg_batch &b, int set, const double *x, double *y) {
 
 // z = M^-1 r over the items of a list set (PCG; pv non-null: also p = z)
 int prec_set(sipg_batch &b, int set, double *pv, const cg_state *states, int slot) {
+    if (launch_batch_prec_groups)
+        return launch_batch_prec_groups(groups_of(b, set), b.item_total, b.R(), b.d_zq, pv, b.d_inst, b.d_item_rr,
+                                        b.d_item_rz, states, slot, b.stream);
     for (size_t g = 0; g < b.groups.size(); ++g) {
         auto &G = b.groups[g];
         int rc = launch_batch_prec(G.p, G.shape, b.R(), b.d_zq, pv, b.d_inst, G.d_items[set],
@@ -204,12 +222,22 @@ int prec_set(sipg_batch &b, int set, double *pv, const cg_state *states, int slo
 int enqueue_iteration(sipg_batch &b, double *X, const double *Bv, int slot, bool repl, bool pcg) {
     const int A = SET_ACTIVE, Q = SET_REPL;
     int rc;
-    for (size_t g = 0; g < b.groups.size(); ++g) {
-        auto &G = b.groups[g];
-        if ((rc = launch_batch_apply(G.p, G.shape, b.Pv(), b.AP(), b.d_inst, G.d_items[A],
-                                     b.count(A, 2 + (int)g), G.cap, b.d_item_part + G.base, b.d_state, slot,
-                                     b.stream)))
+    if ((rc = apply_set(b, A, b.Pv(), b.AP(), b.d_item_part, slot))) return rc;
+    if (pcg && launch_batch_pcg_step) {
+        // alpha and beta in the launches that use them; the replacement set
+        // (marked by the fold) has A x in Ap and takes b - A x for its r
+        if (repl && ((rc = launch_batch_pcg_fold(X, b.Z(), b.Pv(), b.d_chunks[Q], b.count(Q, 1), b.chunk_cap,
+                                                 b.d_chunk_range[Q], b.d_item_range[A], b.d_item_part, b.d_state,
+                                                 slot, b.stream)) ||
+                     (rc = apply_set(b, Q, X, b.AP()))))
             return rc;
+        if ((rc = launch_batch_pcg_step(groups_of(b, A), b.item_total, b.R(), b.AP(), Bv, b.d_zq, b.d_inst,
+                                        b.d_item_range[A], b.d_item_part, b.d_item_rr, b.d_item_rz, b.d_state, slot,
+                                        b.stream)))
+            return rc;
+        return launch_batch_pcg_update(b.Z(), b.Pv(), b.d_zq, b.d_chunks[A], b.count(A, 1), b.chunk_cap,
+                                       b.d_chunk_range[A], b.d_item_range[A], b.d_item_rr, b.d_item_rz, b.d_state,
+                                       slot, b.stream);
     }
     if ((rc = launch_batch_alpha(b.d_list[A], b.count(A, 0), b.ninst, b.d_item_range[A], b.d_item_part,
                                  b.d_state, slot, b.stream)))

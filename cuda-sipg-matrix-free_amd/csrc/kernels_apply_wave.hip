@@ -1,23 +1,25 @@
 // kernels_apply_wave.hip -- the fused SIPG operator apply y = A x with
-// wave-owned elements (volume + flux_term6a + flux_term6b of the reference,
-// volume_gpu_kernels.hpp:9-86, sipg_sem_2d_gpu_kernels.hpp:189-316).
+// wave-owned elements on a block staged in LDS (volume + flux_term6a +
+// flux_term6b of the reference, volume_gpu_kernels.hpp:9-86,
+// sipg_sem_2d_gpu_kernels.hpp:189-316), for even degrees up to 8.
 //
-// Same operator and same per-line arithmetic as apply_kernel / _lds
-// (line_operator in apply_block.hpp), another work split: a wave holds
-// EPW = 64 / (p+1) whole elements (7 at p = 8), one block row, with lane
-// (s, j) = s (p+1) + j on line j of element s.  A workgroup of BY waves
-// owns an EPW x BY block, staged in LDS with its halo ring by direct
-// global -> LDS loads.  Because each element's lines sit in one wave, the
-// column-to-row assembly of the output tile and the copy-out of the block
-// row are wave-local: a block costs two workgroup barriers (the staged
-// block is complete; every wave is done reading it), against four when an
-// element's lines are spread over the workgroup's waves.
+// The same line arithmetic as the strip kernel (line_math.hpp), to the bit,
+// another work split: a wave holds EPW = 64 / (p+1) whole elements (7 at
+// p = 8), one block row, with lane (s, j) = s (p+1) + j on line j of element
+// s.  A workgroup of BY waves owns an EPW x BY block, staged in LDS with
+// its halo ring by direct global -> LDS loads.  Neighbours in x are lanes of
+// the same wave (the block's sides: their staged tiles), neighbours in y
+// staged tiles.  Because each element's lines sit in one wave, the assembly
+// of the output tile and the copy-out of the block row are wave-local: a
+// block costs two workgroup barriers (the staged block is complete; every
+// wave is done reading it).  Whole rows are stored as contiguous runs, which
+// is what a store stream to memory needs.
 //
 // Launch: one block per workgroup, one LDS image per workgroup, so several
 // workgroups share a CU and one computes while another streams its block
 // in.  Block -> workgroup mapping is XCD-aware as in the other operator
 // kernels.  Even degrees (unpadded tiles, which the direct loads need).
-#include "apply_block.hpp"
+#include "line_math.hpp"
 
 #include <algorithm>
 
@@ -49,35 +51,83 @@ void apply_kernel_wave(const T *__restrict__ x, T *__restrict__ y, int dimx, int
     const int gx = x0 + ex, gy = y0 + ey;
     const bool valid = s < BX && gx < dimx && gy < dimy;
     const bool Lb = gx == 0, Rb = gx == dimx - 1;
-    const bool Ub = gy == 0, Db = gy == dimy - 1;       // y grows downwards
     const int sl = (ey + 1) * BX + ex;
     T *tile = lds + sl * NQ;
-    const T *tlL = lds + (ex > 0 ? sl - 1 : G::SL_COL + ey) * NQ;
-    const T *tlR = lds + (ex < BX - 1 ? sl + 1 : G::SL_COL + BY + ey) * NQ;
-    const T *tlD = lds + (sl + BX) * NQ;
-    const T *tlU = lds + (sl - BX) * NQ;
+    const bool isR = s >= BX - 1;                       // the side tile that this lane reads
+    const T *side = lds + (G::SL_COL + (isR ? BY : 0) + ey) * NQ;
+    const T pL = Lb ? T(0.5) * pen : pen, pR = Rb ? T(0.5) * pen : pen;
+    const T wj = coef.w(j);
 
     block_issue_wait();
     __syncthreads();                                    // the staged block is complete
-    T v[N1], Yx[N1], Yy[N1];
-    line_operator<T, P, C>(tile, tlL, tlR, tlD, tlU, j, Lb, Rb, Db, Ub, pen, Yx, Yy, v, coef);
+    T u[N1], q[N1], ox[N1], oy[N1];
+    {
+        Line<T, P> V, Q;
+#pragma unroll
+        for (int i = 0; i < N1; ++i) q[i] = tile[j * N1 + i];
+        V.from(q, coef);
+        // below (y grows downwards) and above: staged rows, or the ghost
+        T tB = -V.t0, nB = V.d0, tA = -V.tP, nA = V.dP, pB = T(0.5) * pen, pA = pB;
+        if (gy < dimy - 1) {
+#pragma unroll
+            for (int i = 0; i < N1; ++i) q[i] = tile[BX * NQ + j * N1 + i];
+            Q.from(q, coef);
+            tB = Q.tP;
+            nB = Q.dP;
+            pB = pen;
+        }
+        if (gy > 0) {
+#pragma unroll
+            for (int i = 0; i < N1; ++i) q[i] = (tile - BX * NQ)[j * N1 + i];
+            Q.from(q, coef);
+            tA = Q.t0;
+            nA = Q.d0;
+            pA = pen;
+        }
+        line_apply<T, P>(V, tB, nB, tA, nA, pB, pA, oy, coef);
+    }
+    {
+        Line<T, P> U, Q;
+#pragma unroll
+        for (int i = 0; i < N1; ++i) {
+            u[i] = tile[i * N1 + j];
+            q[i] = side[i * N1 + j];
+        }
+        U.from(u, coef);
+        Q.from(q, coef);
+        T tL = __shfl(U.tP, lane - N1, 64), nL = __shfl(U.dP, lane - N1, 64);
+        T tR = __shfl(U.t0, lane + N1, 64), nR = __shfl(U.d0, lane + N1, 64);
+        if (s == 0) {
+            tL = Lb ? -U.t0 : Q.tP;
+            nL = Lb ? U.d0 : Q.dP;
+        }
+        if (isR) {
+            tR = Q.t0;
+            nR = Q.d0;
+        }
+        if (Rb) {
+            tR = -U.tP;
+            nR = U.dP;
+        }
+        line_apply<T, P>(U, tL, nL, tR, nR, pL, pR, ox, coef);
+    }
     __syncthreads();                                    // every wave is done reading the block
 
-    // wave-local from here: the element's tile takes the column results,
-    // then each lane adds its row results to its row
+    // wave-local from here: the element's tile takes the row results, then
+    // each lane adds its column's
     if (valid) {
 #pragma unroll
-        for (int a = 0; a < N1; ++a) tile[a * N1 + j] = Yx[a];
+        for (int a = 0; a < N1; ++a) tile[j * N1 + a] = wj * oy[a];
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     double dot = 0.0;
     if (valid) {
 #pragma unroll
-        for (int c = 0; c < N1; ++c) {
-            const T yv = tile[j * N1 + c] + Yy[c];
-            tile[j * N1 + c] = yv;
-            if (DOT) dot += (double)v[c] * (double)yv;
+        for (int a = 0; a < N1; ++a) {
+            const T yv = line_fma(wj, ox[a], tile[a * N1 + j]);
+            tile[a * N1 + j] = yv;
+            if (DOT) dot += (double)u[a] * (double)yv;
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -1,16 +1,18 @@
 // kernels_batch.hip -- many independent SIPG solves in the same launches.
 //
-// Instances of one degree share a launch of the operator kernel: the
-// workgroups walk a device-resident list of (instance, block) items, so the
-// list can shrink as instances finish without relaunching anything (the CG
-// iterations are replayed from a captured hipGraph).  Vector updates walk a
+// All instances share a launch of the operator kernel: the workgroups walk
+// device-resident lists, one to a degree, of (instance, strip, rows) items,
+// so the lists can shrink as instances finish without relaunching anything
+// (the CG iterations are replayed from a captured hipGraph).  Vector updates walk a
 // list of (instance, range) chunks.  Each instance has its own cg_state;
 // its scalars are reduced per instance in a fixed order (deterministic, and
 // independent of how the work is split).  All vectors of all instances are
 // concatenated, element-major within each instance.
-#include "apply_block.hpp"
+#include "batch_items.hpp"
+#include "strip_apply.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 
 namespace sipg_internal {
@@ -19,80 +21,65 @@ namespace {
 
 constexpr int NT = kVecThreads;
 
-// y = A x for every listed block; with DOT also this block's share of x.y
-// into item_part[k], and blocks of instances already finished (per
-// states[inst].s[slot].done) are skipped.  Persistent: workgroup ranges of
-// the item list are contiguous, so consecutive items are neighbouring blocks
-// of one instance; the next live block is loaded while the current one is
-// computed.
-template <typename T, int P, int BX, int BY, bool DOT>
-__global__ __launch_bounds__(BX * BY * (P + 1))
-void batch_apply_kernel(const T *__restrict__ X, T *__restrict__ Y, const batch_inst *__restrict__ inst,
-                        const batch_item *__restrict__ items, const int *__restrict__ count,
-                        double *__restrict__ item_part, const cg_state *__restrict__ states, int slot)
-{
-    using G = BlockGeo<T, P, BX, BY>;
-    __shared__ T lds[G::LDS];
-    __shared__ double red[(G::NT + 63) / 64];
-    const int n = *count;
-    const int NG = gridDim.x;
-    const int lw = xcd_remap(blockIdx.x, NG);
-    const int kbeg = (int)((int64_t)lw * n / NG);
-    const int kend = (int)((int64_t)(lw + 1) * n / NG);
-    // first item >= k of an unfinished instance: SCAN items per step, one
-    // per lane, then the lowest set bit of the ballot.  SCAN is the lane
-    // count of the smallest wave (the last one is partial when NT is not a
-    // multiple of 64), so every wave reaches the same answer.
-    constexpr int SCAN = (G::NT % 64) ? (G::NT % 64) : 64;
-    auto next_live = [&](int k) -> int {
-        if (!DOT) return k;
-        const int lane = threadIdx.x & 63;
-        while (k < kend) {
-            const int kk = k + lane;
-            bool lv = false;
-            if (lane < SCAN && kk < kend) {
-                const cg_state *st = states + items[kk].inst;
-                lv = !(st->s[slot].done | st->err);
-            }
-            const unsigned long long m = __ballot(lv);
-            if (m) return __builtin_amdgcn_readfirstlane(k + __ffsll((long long)m) - 1);
-            k += SCAN;
-        }
-        return kend;
-    };
+// LDS of a strip, and the most that degrees 1..p need, in doubles
+template <int P>
+constexpr int strip_lds = StripGeo<double, P>::LDS + StripGeo<double, P>::EXCH;
+template <int... Ps>
+constexpr std::array<int, sizeof...(Ps)> strip_lds_table(std::integer_sequence<int, Ps...>) {
+    return {strip_lds<Ps + 1>...};
+}
+int strip_lds_upto(int p) {
+    static constexpr auto need = strip_lds_table(std::make_integer_sequence<int, kMaxDegree>{});
+    return *std::max_element(need.begin(), need.begin() + p);
+}
 
-    BlockRegs<T, P, BX, BY> R;
-    int k = next_live(kbeg);
-    if (k < kend) {
-        const batch_item it = items[k];
-        const batch_inst in = inst[it.inst];
-        block_prefetch<T, P, BX, BY>(R, X + in.off, in.dimx, in.dimy, it.x0, it.y0);
-    }
-    while (k < kend) {
-        const batch_item it = items[k];
-        const batch_inst in = inst[it.inst];
-        block_stage<T, P, BX, BY>(lds, R);
-        __syncthreads();
-        const int kn = next_live(k + 1);
-        if (kn < kend) {
-            const batch_item nx = items[kn];
-            const batch_inst ni = inst[nx.inst];
-            block_prefetch<T, P, BX, BY>(R, X + ni.off, ni.dimx, ni.dimy, nx.x0, nx.y0);
-        }
-        const double d = block_compute<T, P, BX, BY, DOT>(lds, Y + in.off, in.dimx, in.dimy, it.x0,
-                                                          it.y0, (T)in.pen);
+// y = A x for the items of all groups (degrees), each a strip of whole
+// elements by a band of rows (strip_apply.hpp); with DOT also the item's
+// share of x.y into item_part, and items of instances already finished (per
+// states[inst].s[slot].done) are skipped.  Persistent workgroups take every
+// gridDim-th item, so that each gets a mix of degrees.
+//
+// One launch for all degrees: with a launch to each, a batch of 128
+// instances of nine degrees took 87 us an iteration on average, one launch
+// 34: the late iterations, with few instances left, were mostly launches.  The
+// registers are those of the highest degree of the class PMAX, the LDS that
+// of the highest degree present.
+template <int PMAX, bool DOT>
+__global__ __launch_bounds__(256, PMAX <= 8 ? 3 : PMAX <= 12 ? 2 : 1)
+void batch_apply_kernel(batch_groups G, const double *__restrict__ X, double *__restrict__ Y,
+                        const batch_inst *__restrict__ inst, double *__restrict__ item_part,
+                        const cg_state *__restrict__ states, int slot)
+{
+    extern __shared__ __attribute__((aligned(16))) double lds[];
+    __shared__ double red[4];
+    __shared__ int first[kMaxDegree + 1];
+    const int n = batch_offsets(G, first);
+    for (int k = xcd_remap(blockIdx.x, gridDim.x); k < n; k += gridDim.x) {
+        const int g = batch_group_at(G, first, k);
+        const int i = k - __builtin_amdgcn_readfirstlane(first[g]);
+        const batch_item it = G.g[g].items[i];
         if (DOT) {
-            const double bs = block_sum<G::NT>(d, red);
-            if (threadIdx.x == 0) item_part[k] = bs;
+            const cg_state *st = states + it.inst;
+            if (st->s[slot].done | st->err) continue;             // uniform over the workgroup
         }
-        k = kn;
+        const batch_inst in = inst[it.inst];
+        const int tid = opaque(threadIdx.x);
+        const double d = by_degree<PMAX>(G.g[g].p, [&](auto deg) {
+            constexpr int P = decltype(deg)::value, EPW = StripGeo<double, P>::EPW;
+            return strip_apply<double, P, DOT>(X + in.off, Y + in.off, in.dimx, in.dimy, in.pen, it.x0,
+                                               min(EPW, in.dimx - it.x0), it.y0, min(it.y0 + it.rows, in.dimy), lds,
+                                               lds + StripGeo<double, P>::LDS, tid);
+        });
+        if (DOT) {
+            const double bs = block_sum<256>(d, red);
+            if (threadIdx.x == 0) item_part[G.g[g].base + i] = bs;
+        }
     }
 }
 
 __device__ __forceinline__ double block_reduce(double v, double *red) {
     // fixed-order block sum, valid in every thread
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = wave_total(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __syncthreads();
     if (lane == 0) red[wid] = v;
@@ -336,64 +323,41 @@ __global__ __launch_bounds__(NT) void batch_init_kernel(const int *__restrict__ 
     }
 }
 
-// ---- per-degree operator launch table --------------------------------------
-
-template <int P, int BX, int BY, bool DOT>
-int resident_batch_groups() {
-    static std::atomic<int> cache[64];
+// Workgroups of the apply kernel that the device holds at once with the LDS
+// of degree pmax, cached per device.
+template <int PMAX, bool DOT>
+int resident_batch_groups(int pmax, size_t lds) {
+    static std::atomic<int> cache[64][kMaxDegree + 1];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    int g = cache[dev].load(std::memory_order_relaxed);
+    int g = cache[dev][pmax].load(std::memory_order_relaxed);
     if (g > 0) return g;
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&batch_apply_kernel<double, P, BX, BY, DOT>),
-            BX * BY * (P + 1), 0) != hipSuccess)
+            &per, reinterpret_cast<const void *>(&batch_apply_kernel<PMAX, DOT>), 256, lds) != hipSuccess)
         per = 0;
     g = (cus > 0 ? cus : 1) * (per > 0 ? per : 1);
-    cache[dev].store(g, std::memory_order_relaxed);
+    cache[dev][pmax].store(g, std::memory_order_relaxed);
     return g;
 }
 
-template <int P, int BX, int BY>
-int launch_batch_apply_one(const double *X, double *Y, const batch_inst *inst, const batch_item *items,
-                           const int *count, int max_items, double *item_part, const cg_state *states,
-                           int slot, hipStream_t s) {
-    if (max_items <= 0) return SIPG_OK;
-    dim3 block(BX * BY * (P + 1));
+template <int PMAX>
+int launch_apply_class(const batch_groups &G, int pmax, int max_items, const double *X, double *Y,
+                       const batch_inst *inst, double *item_part, const cg_state *states, int slot, hipStream_t s) {
+    const size_t lds = (size_t)strip_lds_upto(pmax) * sizeof(double);
     if (item_part) {
-        dim3 grid(std::min(max_items, resident_batch_groups<P, BX, BY, true>()));
-        hipLaunchKernelGGL((batch_apply_kernel<double, P, BX, BY, true>), grid, block, 0, s, X, Y, inst, items,
-                           count, item_part, states, slot);
+        const dim3 grid(std::min(max_items, resident_batch_groups<PMAX, true>(pmax, lds)));
+        hipLaunchKernelGGL((batch_apply_kernel<PMAX, true>), grid, dim3(256), lds, s, G, X, Y, inst, item_part, states,
+                           slot);
     } else {
-        dim3 grid(std::min(max_items, resident_batch_groups<P, BX, BY, false>()));
-        hipLaunchKernelGGL((batch_apply_kernel<double, P, BX, BY, false>), grid, block, 0, s, X, Y, inst, items,
-                           count, item_part, states, slot);
+        const dim3 grid(std::min(max_items, resident_batch_groups<PMAX, false>(pmax, lds)));
+        hipLaunchKernelGGL((batch_apply_kernel<PMAX, false>), grid, dim3(256), lds, s, G, X, Y, inst, item_part,
+                           states, slot);
     }
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
-
-using BatchApplyFn = int (*)(const double *, double *, const batch_inst *, const batch_item *, const int *, int,
-                             double *, const cg_state *, int, hipStream_t);
-
-template <int P>
-constexpr BatchApplyFn wide_shape() {
-    // 16 x 4 blocks need (p+1)*64 <= 1024 threads and fit LDS in FP64 up to p = 12
-    if constexpr (P <= 12) return &launch_batch_apply_one<P, 16, 4>;
-    else return nullptr;
-}
-
-template <int... Ps>
-struct BatchTable {
-    static constexpr BatchApplyFn fn[kBatchShapes][sizeof...(Ps)] = {
-        {wide_shape<Ps>()...},
-        {&launch_batch_apply_one<Ps, 8, 4>...},
-        {&launch_batch_apply_one<Ps, 8, 2>...},
-    };
-};
-using Table = BatchTable<1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>;
 
 int vec_blocks(int nchunks) { return std::max(1, std::min(nchunks, 2048)); }
 int inst_blocks(int ninst) { return std::max(1, std::min(ninst, 2048)); }
@@ -404,15 +368,44 @@ const int kBatchShapeBX[kBatchShapes] = {16, 8, 8};
 const int kBatchShapeBY[kBatchShapes] = {4, 4, 2};
 
 bool batch_shape_supported(int p, int shape) {
-    return p >= 1 && p <= kMaxDegree && shape >= 0 && shape < kBatchShapes && Table::fn[shape][p - 1] != nullptr;
+    // 16 x 4 stays a choice up to degree 12
+    return p >= 1 && p <= kMaxDegree && shape >= 0 && shape < kBatchShapes && (shape > 0 || p <= 12);
+}
+
+// An item is a strip of 64 / (p+1) elements by 16, 8 or 4 rows: one to four
+// rows to a wave.  Fewer rows make more items, which a small batch and the
+// last instances of a large one need; more rows load the rows between two
+// bands less often.
+void batch_item_extent(int p, int shape, int *bx, int *rows) {
+    *bx = 64 / (p + 1);
+    *rows = shape == 0 ? 16 : shape == 1 ? 8 : 4;
+}
+
+int launch_batch_apply_groups(const batch_groups &G, int max_items, const double *X, double *Y,
+                              const batch_inst *inst, double *item_part, const cg_state *states, int slot,
+                              hipStream_t s) {
+    int pmax = 0;
+    for (int g = 0; g < G.n; ++g) {
+        if (G.g[g].p < 1 || G.g[g].p > kMaxDegree) return SIPG_ERR_UNSUPPORTED;
+        pmax = std::max(pmax, G.g[g].p);
+    }
+    if (item_part && !states) return SIPG_ERR_INVALID;
+    if (max_items <= 0 || pmax == 0) return SIPG_OK;
+    // Classes by the registers their highest degree needs: 168 up to degree
+    // 8 (three workgroups to a CU, as their LDS allows), 252 up to 12 (two)
+    if (pmax <= 8) return launch_apply_class<8>(G, pmax, max_items, X, Y, inst, item_part, states, slot, s);
+    if (pmax <= 12) return launch_apply_class<12>(G, pmax, max_items, X, Y, inst, item_part, states, slot, s);
+    return launch_apply_class<16>(G, pmax, max_items, X, Y, inst, item_part, states, slot, s);
 }
 
 int launch_batch_apply(int p, int shape, const double *X, double *Y, const batch_inst *inst,
                        const batch_item *items, const int *count, int max_items, double *item_part,
                        const cg_state *states, int slot, hipStream_t s) {
     if (!batch_shape_supported(p, shape)) return SIPG_ERR_UNSUPPORTED;
-    if (item_part && !states) return SIPG_ERR_INVALID;
-    return Table::fn[shape][p - 1](X, Y, inst, items, count, max_items, item_part, states, slot, s);
+    batch_groups G;
+    G.n = 1;
+    G.g[0] = {items, count, 0, p};
+    return launch_batch_apply_groups(G, max_items, X, Y, inst, item_part, states, slot, s);
 }
 
 int launch_batch_alpha(const int *list, const int *count, int max_inst, const int2 *item_range,

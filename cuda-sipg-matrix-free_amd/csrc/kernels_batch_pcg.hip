@@ -1,13 +1,27 @@
-// kernels_batch_pcg.hip -- the block-Jacobi preconditioner of sipg_pcg for
-// batched solves: z = M^-1 r over the (instance, block) items of the
-// operator's lists, with per-item sums of r.r and r.z, and the PCG beta step
-// per instance.  M is the exact inverse of the interior element block of
-// the standard penalty 5 (p+1)^2 (kernels_pcg.hip), so every coefficient is
-// a compile-time constant of the degree; batched PCG requires that penalty.
+// kernels_batch_pcg.hip -- block-Jacobi PCG for batched solves: z = M^-1 r
+// over the (instance, block) items of the operator's lists, and the rest of
+// an iteration fused around it.  M is the exact inverse of the interior
+// element block of the standard penalty 5 (p+1)^2 (kernels_pcg.hip), so every
+// coefficient is a compile-time constant of the degree; batched PCG requires
+// that penalty.
+//
+// An iteration is three launches over all degrees: the operator with p.Ap
+// (kernels_batch.hip); alpha, r -= alpha Ap and z = M^-1 r; beta, x += alpha
+// p and p = z + beta p.  Each workgroup sums the p.Ap or r.r and r.z shares
+// of its instance by itself, in a fixed order.  Where some instances' r is
+// replaced by b - A x, a fold of their x and the operator on them come
+// between the first two, and the second takes b - A x for its r.
+//
+// Within a launch, an instance's state is written by the workgroup of its
+// first item or chunk only, in fields that the others do not read: the
+// next slot, err (read by the launches that do not write it), alpha and the
+// mark that the instance has been stepped.
 #include "apply_block.hpp"
+#include "batch_items.hpp"
 #include "prec_block.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 
 namespace sipg_internal {
@@ -16,214 +30,233 @@ namespace {
 
 constexpr int VT = kVecThreads;
 
-// z = M^-1 r on every element of each listed block (COPYP: also p = z);
-// item k's sums of r.r and r.z go to item_rr[k], item_rz[k].  With states,
-// blocks of instances already finished at `slot` are skipped.
-template <int P, int BX, int BY, bool COPYP>
-__global__ __launch_bounds__(BX * BY * (P + 1))
-void batch_prec_kernel(const double *__restrict__ R, double *__restrict__ Zq, double *__restrict__ Pv,
-                       const batch_inst *__restrict__ inst, const batch_item *__restrict__ items,
-                       const int *__restrict__ count, double *__restrict__ item_rr,
-                       double *__restrict__ item_rz, const cg_state *__restrict__ states, int slot)
+// 1 / (lambda_a + lambda_c) of degree p starts at linv_at(p) in LDS
+__host__ __device__ constexpr int linv_at(int p) { return p * (p + 1) * (2 * p + 1) / 6 - 1; }
+static_assert(linv_at(2) - linv_at(1) == 4 && linv_at(1) == 0, "(q+1)^2 values for each degree q < p");
+
+// LDS of the degrees up to p, in doubles: the four waves' tiles, the tables
+template <int... Ps>
+constexpr std::array<int, sizeof...(Ps)> prec_lds_table(std::integer_sequence<int, Ps...>) {
+    return {4 * RunGeo<double, Ps + 1>::BUF...};
+}
+int prec_tiles_upto(int p) {
+    static constexpr auto need = prec_lds_table(std::make_integer_sequence<int, kMaxDegree>{});
+    return *std::max_element(need.begin(), need.begin() + p);
+}
+
+// sum of part[b, e) in a fixed order, in every lane of the wave
+__device__ __forceinline__ double wave_range_sum(const double *__restrict__ part, int b, int e, int lane) {
+    double s = 0.0;
+    for (int i = b + lane; i < e; i += 64) s += part[i];
+    return wave_total(s);
+}
+
+// z = M^-1 r for the items of all groups (COPYP: also p = z); an item's sums
+// of r.r and r.z go to item_rr and item_rz.  With states, items of instances
+// already finished at `slot` are skipped.  STEP: first alpha = r.z / p.Ap and
+// r -= alpha Ap, or r = b - Ap for an instance marked replaced (Ap holds A x
+// then).  A breakdown (p.Ap not positive, or not finite) skips the instance;
+// the update that follows sets its err.
+//
+// A wave streams the runs of its item's rows on its own (prec_block.hpp).
+// With STEP four passes over memory, where the update of x and r and the
+// preconditioner took eight in two sets of launches: 46 + 74 us an iteration
+// on average over a solve of 128 instances of nine degrees, 44 now.
+template <int PMAX, bool STEP, bool COPYP>
+__global__ __launch_bounds__(256, PMAX <= 12 ? 3 : 2)
+void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__restrict__ AP,
+                       const double *__restrict__ B, double *__restrict__ Zq, double *__restrict__ Pv,
+                       const batch_inst *__restrict__ inst, const int2 *__restrict__ item_range,
+                       const double *__restrict__ item_part, double *__restrict__ item_rr,
+                       double *__restrict__ item_rz, cg_state *states, int slot)
 {
-    constexpr int N1 = P + 1, NQ = N1 * N1, NE = BX * BY, NT = NE * N1, TS = tile_stride(NQ);
-    constexpr int RUN = BX * NQ, KR = N1;               // NE*NQ values = KR per thread
-    __shared__ double lds[NE * TS];
-    __shared__ double red[(NT + 63) / 64];
-    const int tid = threadIdx.x;
-    const int s_el = tid % NE;
-    int j = tid / NE;
-    if (NE % 64 == 0) j = __builtin_amdgcn_readfirstlane(j);
-    const int n = *count;
-    for (int k = blockIdx.x; k < n; k += gridDim.x) {
-        const batch_item it = items[k];
-        if (states) {
-            const cg_state *st = states + it.inst;
-            if (st->s[slot].done | st->err) continue;     // uniform over the workgroup
-        }
+    extern __shared__ __attribute__((aligned(16))) double lds[];
+    __shared__ double red[2][4];
+    __shared__ int first[kMaxDegree + 1];
+    const int n = batch_offsets(G, first);
+    double *tab = lds + tiles;
+    for (int g = 0; g < G.n; ++g)
+        by_degree<PMAX>(G.g[g].p, [&](auto deg) {
+            constexpr int P = decltype(deg)::value, N1 = P + 1;
+            for (int q = threadIdx.x; q < N1 * N1; q += 256) tab[linv_at(P) + q] = PrecEO<P>::V.Linv[q / N1][q % N1];
+        });
+    __syncthreads();
+    for (int k = xcd_remap(blockIdx.x, gridDim.x); k < n; k += gridDim.x) {
+        const int g = batch_group_at(G, first, k);
+        const int i = k - __builtin_amdgcn_readfirstlane(first[g]);
+        const batch_item it = G.g[g].items[i];
+        cg_state *st = states + it.inst;
+        if (states && (st->s[slot].done | st->err)) continue;     // uniform over the workgroup
         const batch_inst in = inst[it.inst];
-        const int64_t RS = (int64_t)in.dimx * NQ;
-        const int64_t base = in.off + ((int64_t)it.y0 * in.dimx + it.x0) * NQ;
-        const int ncol = min(BX, in.dimx - it.x0), nrow = min(BY, in.dimy - it.y0);
-        double rv[KR];
-        unsigned valid = 0;
+        const int at = G.g[g].base + i;
+        const int tid = opaque(threadIdx.x);
+        const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const bool replaced = STEP && (st->s[slot].flags & kSlotReplaced);
+        double alpha = 0.0;
+        if (STEP) {
+            const int2 range = item_range[it.inst];
+            const double pAp = wave_range_sum(item_part, range.x, range.y, lane);
+            alpha = st->s[slot].rz / pAp;
+            if (at == range.x && tid == 0) {
+                st->s[slot].alpha = alpha;
+                st->s[slot].pAp = pAp;
+                st->s[slot].flags |= kSlotStepped;
+            }
+            if (!(pAp > 0.0) || !isfinite(alpha)) continue;       // the same in every workgroup
+            if (replaced) alpha = 1.0;
+        }
         double srr = 0.0, srz = 0.0;
-#pragma unroll
-        for (int kk = 0; kk < KR; ++kk) {
-            const int idx = tid + kk * NT;                 // < NE * NQ
-            const int rr = idx / RUN, w = idx - rr * RUN;
-            const bool ok = rr < nrow && w / NQ < ncol;
-            double v = 0.0;
-            if (ok) {
-                v = R[base + rr * RS + w];
-                valid |= 1u << kk;
-                srr += v * v;
+        by_degree<PMAX>(G.g[g].p, [&](auto deg) {
+            constexpr int P = decltype(deg)::value;
+            using Run = RunGeo<double, P>;
+            const int nv = min(Run::EPW, in.dimx - it.x0) * Run::NQ;
+            const int yb = min(it.y0 + it.rows, in.dimy);
+            double x0, x1;
+            for (int gy = it.y0 + w; gy < yb; gy += 4) {
+                const int64_t o = in.off + ((int64_t)gy * in.dimx + it.x0) * Run::NQ;
+                prec_run<double, P, STEP, COPYP, true, false>((replaced ? B : R) + o, R + o, AP + o, Zq + o, Pv + o, nv,
+                                                              [&] { return alpha; }, nullptr, tab + linv_at(P),
+                                                              lds + w * Run::BUF, lane, srr, srz, x0, x1);
             }
-            rv[kk] = v;
-            lds[lds_index<NQ, TS>(idx)] = v;
+        });
+        srr = wave_total(srr);
+        srz = wave_total(srz);
+        __syncthreads();                                          // the last item's sums have been read
+        if (lane == 0) {
+            red[0][w] = srr;
+            red[1][w] = srz;
         }
         __syncthreads();
-        double *tile = lds + s_el * TS;
-        {   // column j of S^T R
-            double c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-            contract_st<double, P, true>(nullptr, c, t);
-#pragma unroll
-            for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
+        if (tid < 2) {
+            const double *v = red[tid];
+            (tid ? item_rz : item_rr)[at] = (v[0] + v[1]) + (v[2] + v[3]);
         }
-        __syncthreads();
-        {   // row j of ((S^T R S) ./ L) S^T
-            double w[N1], v[N1];
-#pragma unroll
-            for (int b = 0; b < N1; ++b) w[b] = tile[j * N1 + b];
-            contract_st<double, P, true>(nullptr, w, v);
-#pragma unroll
-            for (int c = 0; c < N1; ++c) v[c] *= PrecEO<P>::V.Linv[j][c];
-            contract_s<double, P, true>(nullptr, v, w);
-#pragma unroll
-            for (int d = 0; d < N1; ++d) tile[j * N1 + d] = w[d];
-        }
-        __syncthreads();
-        {   // column j of S (...)
-            double c[N1], t[N1];
-#pragma unroll
-            for (int i = 0; i < N1; ++i) c[i] = tile[i * N1 + j];
-            contract_s<double, P, true>(nullptr, c, t);
-#pragma unroll
-            for (int a = 0; a < N1; ++a) tile[a * N1 + j] = t[a];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < KR; ++kk) {
-            if (valid & (1u << kk)) {
-                const int idx = tid + kk * NT;
-                const int rr = idx / RUN, w = idx - rr * RUN;
-                const int64_t gi = base + rr * RS + w;
-                const double zv = lds[lds_index<NQ, TS>(idx)];
-                Zq[gi] = zv;
-                if (COPYP) Pv[gi] = zv;
-                srz += rv[kk] * zv;
-            }
-        }
-        const double a = block_sum<NT>(srr, red);
-        __syncthreads();
-        const double b = block_sum<NT>(srz, red);
-        if (tid == 0) {
-            item_rr[k] = a;
-            item_rz[k] = b;
-        }
-        __syncthreads();                                   // LDS and red free for the next item
     }
 }
 
-template <int P, int BX, int BY, bool COPYP>
-int resident_prec_groups() {
-    static std::atomic<int> cache[64];
+template <int PMAX, bool STEP, bool COPYP>
+int resident_prec_groups(int pmax, size_t lds) {
+    static std::atomic<int> cache[64][kMaxDegree + 1];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    int g = cache[dev].load(std::memory_order_relaxed);
+    int g = cache[dev][pmax].load(std::memory_order_relaxed);
     if (g > 0) return g;
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&batch_prec_kernel<P, BX, BY, COPYP>), BX * BY * (P + 1), 0) !=
-        hipSuccess)
+            &per, reinterpret_cast<const void *>(&batch_prec_kernel<PMAX, STEP, COPYP>), 256, lds) != hipSuccess)
         per = 0;
     g = (cus > 0 ? cus : 1) * (per > 0 ? per : 1);
-    cache[dev].store(g, std::memory_order_relaxed);
+    cache[dev][pmax].store(g, std::memory_order_relaxed);
     return g;
 }
 
-template <int P, int BX, int BY>
-int launch_prec_one(const double *R, double *Zq, double *Pv, const batch_inst *inst, const batch_item *items,
-                    const int *count, int max_items, double *item_rr, double *item_rz, const cg_state *states,
-                    int slot, hipStream_t s) {
-    if (max_items <= 0) return SIPG_OK;
-    dim3 block(BX * BY * (P + 1));
-    if (Pv) {
-        dim3 grid(std::min(max_items, resident_prec_groups<P, BX, BY, true>()));
-        hipLaunchKernelGGL((batch_prec_kernel<P, BX, BY, true>), grid, block, 0, s, R, Zq, Pv, inst, items, count,
-                           item_rr, item_rz, states, slot);
-    } else {
-        dim3 grid(std::min(max_items, resident_prec_groups<P, BX, BY, false>()));
-        hipLaunchKernelGGL((batch_prec_kernel<P, BX, BY, false>), grid, block, 0, s, R, Zq, Pv, inst, items, count,
-                           item_rr, item_rz, states, slot);
-    }
+template <int PMAX, bool STEP, bool COPYP>
+int launch_prec_kernel(const batch_groups &G, int pmax, int max_items, double *R, const double *AP, const double *B,
+                       double *Zq, double *Pv, const batch_inst *inst, const int2 *item_range,
+                       const double *item_part, double *item_rr, double *item_rz, cg_state *states, int slot,
+                       hipStream_t s) {
+    const int tiles = prec_tiles_upto(pmax);
+    const size_t lds = (size_t)(tiles + linv_at(pmax + 1)) * sizeof(double);
+    const dim3 grid(std::min(max_items, resident_prec_groups<PMAX, STEP, COPYP>(pmax, lds)));
+    hipLaunchKernelGGL((batch_prec_kernel<PMAX, STEP, COPYP>), grid, dim3(256), lds, s, G, tiles, R, AP, B, Zq, Pv,
+                       inst, item_range, item_part, item_rr, item_rz, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
 
-using PrecFn = int (*)(const double *, double *, double *, const batch_inst *, const batch_item *, const int *, int,
-                       double *, double *, const cg_state *, int, hipStream_t);
-
-template <int P>
-constexpr PrecFn wide_prec() {
-    if constexpr (P <= 12) return &launch_prec_one<P, 16, 4>;
-    else return nullptr;
+template <bool STEP, bool COPYP, class... A>
+int launch_prec_any(const batch_groups &G, int max_items, A... args) {
+    int pmax = 0;
+    for (int g = 0; g < G.n; ++g) {
+        if (G.g[g].p < 1 || G.g[g].p > kMaxDegree) return SIPG_ERR_UNSUPPORTED;
+        pmax = std::max(pmax, G.g[g].p);
+    }
+    if (max_items <= 0 || pmax == 0) return SIPG_OK;
+    if (pmax <= 8) return launch_prec_kernel<8, STEP, COPYP>(G, pmax, max_items, args...);
+    if (pmax <= 12) return launch_prec_kernel<12, STEP, COPYP>(G, pmax, max_items, args...);
+    return launch_prec_kernel<16, STEP, COPYP>(G, pmax, max_items, args...);
 }
 
-template <int... Ps>
-struct PrecTable {
-    static constexpr PrecFn fn[kBatchShapes][sizeof...(Ps)] = {
-        {wide_prec<Ps>()...},
-        {&launch_prec_one<Ps, 8, 4>...},
-        {&launch_prec_one<Ps, 8, 2>...},
-    };
-};
-using PTable = PrecTable<1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>;
-
-__device__ __forceinline__ double vreduce(double v, double *red) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < VT / 64; ++i) s += red[i];
-    return s;
-}
-
-__device__ __forceinline__ double vrange(const double *__restrict__ part, int b, int e, double *red) {
-    double s = 0.0;
-    for (int i = b + (int)threadIdx.x; i < e; i += VT) s += part[i];
-    return vreduce(s, red);
-}
-
-// beta = r.z(new) / r.z(old) per active instance from the preconditioner's
-// item sums; writes the next slot with r.r (stopping test, host decisions)
-// and r.z.  Flag rules as in batch_beta_kernel; the sums are those of the
-// replaced residual when the instance's r was replaced this iteration (the
-// preconditioner runs after the replacement).
-__global__ __launch_bounds__(VT) void batch_beta_pcg_kernel(const int *__restrict__ list,
+// For the listed chunks of instances whose r is to be replaced: x += z +
+// alpha p, z = 0 (the increments since the last true residual, this
+// iteration's included, folded as one); marks the instance.
+__global__ __launch_bounds__(VT) void batch_pcg_fold_kernel(double *__restrict__ X, double *__restrict__ Z,
+                                                            const double *__restrict__ Pv,
+                                                            const batch_chunk *__restrict__ chunks,
                                                             const int *__restrict__ count,
+                                                            const int2 *__restrict__ chunk_range,
                                                             const int2 *__restrict__ item_range,
-                                                            const double *__restrict__ item_rr,
-                                                            const double *__restrict__ item_rz, cg_state *states,
+                                                            const double *__restrict__ item_part, cg_state *states,
                                                             int slot) {
-    __shared__ double red[VT / 64];
     const int n = *count;
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
-        const int i = list[k];
-        cg_state *st = states + i;
+        const batch_chunk c = chunks[k];
+        cg_state *st = states + c.inst;
+        if (st->s[slot].done | st->err) continue;
+        const int2 r = item_range[c.inst];
+        const double pAp = wave_range_sum(item_part, r.x, r.y, threadIdx.x & 63);
+        const double alpha = st->s[slot].rz / pAp;
+        if (!(pAp > 0.0) || !isfinite(alpha)) continue;
+        if (k == chunk_range[c.inst].x && threadIdx.x == 0) {
+            st->s[slot].flags |= kSlotReplaced;
+            st->nrep += 1;
+        }
+        for (int64_t i = c.begin + threadIdx.x; i < c.end; i += VT) {
+            const double z = Z[i] + alpha * Pv[i];
+            X[i] += z;
+            Z[i] = 0.0;
+        }
+    }
+}
+
+// beta = r.z(new) / r.z(old) per instance from the preconditioner's item
+// sums; z += alpha p (unless r was replaced: it is folded then) and p = zq +
+// beta p over the listed chunks; the first chunk's workgroup writes the next
+// slot with r.r (stopping test, host decisions) and r.z.  Flag rules as in
+// batch_beta_kernel.  An instance that was not stepped (finished, or err)
+// carries its slot forward.
+//
+// Five passes over memory; 16 bytes to a lane, four of them in flight for
+// each stream (37 us an iteration on average in the same solve).
+__global__ __launch_bounds__(VT) void batch_pcg_update_kernel(double *__restrict__ Z, double *__restrict__ Pv,
+                                                              const double *__restrict__ Zq,
+                                                              const batch_chunk *__restrict__ chunks,
+                                                              const int *__restrict__ count,
+                                                              const int2 *__restrict__ chunk_range,
+                                                              const int2 *__restrict__ item_range,
+                                                              const double *__restrict__ item_rr,
+                                                              const double *__restrict__ item_rz, cg_state *states,
+                                                              int slot) {
+    const int n = *count;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const batch_chunk c = chunks[k];
+        cg_state *st = states + c.inst;
         const cg_slot cur = st->s[slot];
-        if (cur.done | st->err) {
-            if (threadIdx.x == 0) st->s[slot ^ 1] = cur;          // carry forward
+        const bool lead = k == chunk_range[c.inst].x && threadIdx.x == 0;
+        const bool bad = !(cur.pAp > 0.0) || !isfinite(cur.alpha);
+        if (cur.done || !(cur.flags & kSlotStepped) || bad) {
+            if (lead) {
+                if (!cur.done && (cur.flags & kSlotStepped)) st->err = isfinite(cur.pAp) ? 2 : 3;
+                cg_slot nx = cur;
+                nx.flags &= ~kSlotStepped;
+                st->s[slot ^ 1] = nx;
+            }
             continue;
         }
-        const int2 r = item_range[i];
-        const double rr_new = vrange(item_rr, r.x, r.y, red);
-        const double rz_new = vrange(item_rz, r.x, r.y, red);
-        if (threadIdx.x == 0) {
-            const bool replaced = (cur.flags & kSlotReplaced) != 0;
+        const int2 r = item_range[c.inst];
+        const int lane = threadIdx.x & 63;
+        const double rr_new = wave_range_sum(item_rr, r.x, r.y, lane);
+        const double rz_new = wave_range_sum(item_rz, r.x, r.y, lane);
+        const double alpha = cur.alpha, beta = rz_new / cur.rz;
+        const bool replaced = (cur.flags & kSlotReplaced) != 0;
+        if (lead) {
             const bool met = !(sqrt(rr_new) > st->stop);
             const bool need_true = st->true_stop && !replaced;
             cg_slot nx{};
             nx.rr = rr_new;
             nx.rz = rz_new;
-            nx.beta = rz_new / cur.rz;
+            nx.beta = beta;
             nx.it = cur.it + 1;
             nx.done = ((met && !need_true) || nx.it >= st->maxit) ? 1 : 0;
             nx.checked = replaced ? 1 : 0;
@@ -233,28 +266,92 @@ __global__ __launch_bounds__(VT) void batch_beta_pcg_kernel(const int *__restric
             if (!isfinite(rr_new) || !isfinite(rz_new)) st->err = 3;
             else if (!(rz_new > 0.0) && rr_new > 0.0) st->err = 2;
         }
+        constexpr int U = 4;
+        const int64_t len = c.end - c.begin, nvec = len / 2;
+        double *z = Z + c.begin, *p = Pv + c.begin;
+        const double *q = Zq + c.begin;
+        auto one = [&](int64_t i) {
+            const double pv = p[i];
+            if (!replaced) z[i] = z[i] + alpha * pv;
+            p[i] = q[i] + beta * pv;
+        };
+        int64_t v0 = 0;
+        for (; v0 + U * VT <= nvec; v0 += U * VT) {
+            double pv[U][2], qv[U][2], zv[U][2];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t o = 2 * (v0 + u * VT + threadIdx.x);
+                load_vec<double, 2>(p + o, pv[u]);
+                load_vec<double, 2>(q + o, qv[u]);
+                if (!replaced) load_vec<double, 2>(z + o, zv[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t o = 2 * (v0 + u * VT + threadIdx.x);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (!replaced) zv[u][h] = zv[u][h] + alpha * pv[u][h];
+                    pv[u][h] = qv[u][h] + beta * pv[u][h];
+                }
+                if (!replaced) store_vec<double, 2>(z + o, zv[u]);
+                store_vec<double, 2>(p + o, pv[u]);
+            }
+        }
+        for (int64_t i = 2 * v0 + threadIdx.x; i < len; i += VT) one(i);
     }
 }
 
 }  // namespace
 
 bool batch_prec_supported(int p, double pen, int shape) {
-    return p >= 1 && p <= kMaxDegree && shape >= 0 && shape < kBatchShapes && PTable::fn[shape][p - 1] != nullptr &&
-           pen == 5.0 * (p + 1) * (p + 1);
+    return batch_shape_supported(p, shape) && pen == 5.0 * (p + 1) * (p + 1);
+}
+
+int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq, double *Pv,
+                             const batch_inst *inst, double *item_rr, double *item_rz, const cg_state *states,
+                             int slot, hipStream_t s) {
+    auto *r = const_cast<double *>(R);                            // read only without STEP
+    auto *st = const_cast<cg_state *>(states);
+    const double *none = nullptr;
+    const int2 *nor = nullptr;
+    return Pv ? launch_prec_any<false, true>(G, max_items, r, none, none, Zq, Pv, inst, nor, none, item_rr, item_rz, st,
+                                             slot, s)
+              : launch_prec_any<false, false>(G, max_items, r, none, none, Zq, Pv, inst, nor, none, item_rr, item_rz, st,
+                                              slot, s);
 }
 
 int launch_batch_prec(int p, int shape, const double *R, double *Zq, double *Pv, const batch_inst *inst,
                       const batch_item *items, const int *count, int max_items, double *item_rr, double *item_rz,
                       const cg_state *states, int slot, hipStream_t s) {
-    if (p < 1 || p > kMaxDegree || shape < 0 || shape >= kBatchShapes || !PTable::fn[shape][p - 1])
-        return SIPG_ERR_UNSUPPORTED;
-    return PTable::fn[shape][p - 1](R, Zq, Pv, inst, items, count, max_items, item_rr, item_rz, states, slot, s);
+    if (!batch_shape_supported(p, shape)) return SIPG_ERR_UNSUPPORTED;
+    batch_groups G;
+    G.n = 1;
+    G.g[0] = {items, count, 0, p};
+    return launch_batch_prec_groups(G, max_items, R, Zq, Pv, inst, item_rr, item_rz, states, slot, s);
 }
 
-int launch_batch_beta_pcg(const int *list, const int *count, int max_inst, const int2 *item_range,
-                          const double *item_rr, const double *item_rz, cg_state *states, int slot, hipStream_t s) {
-    hipLaunchKernelGGL(batch_beta_pcg_kernel, dim3(std::max(1, std::min(max_inst, 2048))), dim3(VT), 0, s, list,
-                       count, item_range, item_rr, item_rz, states, slot);
+int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
+                          double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
+                          double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s) {
+    double *nop = nullptr;
+    return launch_prec_any<true, false>(G, max_items, R, AP, B, Zq, nop, inst, item_range, item_part, item_rr, item_rz,
+                                        states, slot, s);
+}
+
+int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,
+                          int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_part,
+                          cg_state *states, int slot, hipStream_t s) {
+    hipLaunchKernelGGL(batch_pcg_fold_kernel, dim3(std::max(1, std::min(max_chunks, 2048))), dim3(VT), 0, s, X, Z, Pv,
+                       chunks, count, chunk_range, item_range, item_part, states, slot);
+    SIPG_HIP_TRY(hipGetLastError());
+    return SIPG_OK;
+}
+
+int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks, const int *count,
+                            int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_rr,
+                            const double *item_rz, cg_state *states, int slot, hipStream_t s) {
+    hipLaunchKernelGGL(batch_pcg_update_kernel, dim3(std::max(1, std::min(max_chunks, 2048))), dim3(VT), 0, s, Z, Pv,
+                       Zq, chunks, count, chunk_range, item_range, item_rr, item_rz, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }

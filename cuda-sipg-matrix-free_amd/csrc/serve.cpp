@@ -240,9 +240,10 @@ int upload_set(sipg_server &S, int set, const std::vector<int64_t> &ids,
         const Request &R = S.reqs.at(id);
         auto &v = items[R.p];
         const int s0 = (int)v.size();
-        const int BX = kBatchShapeBX[S.shape[R.p]], BY = kBatchShapeBY[S.shape[R.p]];
+        int BX, BY;
+        batch_extent(R.p, S.shape[R.p], &BX, &BY);
         for (int by = 0; by < (R.dim + BY - 1) / BY; ++by)
-            for (int bx = 0; bx < (R.dim + BX - 1) / BX; ++bx) v.push_back({R.slot, bx * BX, by * BY, 0});
+            for (int bx = 0; bx < (R.dim + BX - 1) / BX; ++bx) v.push_back({R.slot, bx * BX, by * BY, BY});
         item_range[R.slot] = int2{s0, (int)v.size()};   // based below
         list.push_back(R.slot);
         const int c0 = (int)chunks.size();
@@ -311,10 +312,31 @@ int upload_set(sipg_server &S, int set, const std::vector<int64_t> &ids,
     return SIPG_OK;
 }
 
-int apply_set(sipg_server &S, int set, const std::vector<int> &degrees, const double *x, double *y) {
+batch_groups groups_of(sipg_server &S, int set, const std::vector<int> &degrees, int *max_items) {
+    batch_groups G;
+    G.n = 0;
+    *max_items = 0;
+    for (int p : degrees) {
+        G.g[G.n++] = {S.d_items[set][p], S.count(set, 2 + p), S.item_base[set][p], p};
+        *max_items += S.item_cap[set][p];
+    }
+    return G;
+}
+
+// y = A x over the requests of a set; with p.Ap, of those that have not
+// finished at `slot`
+int apply_set(sipg_server &S, int set, const std::vector<int> &degrees, const double *x, double *y,
+              double *item_part = nullptr, int slot = 0) {
+    const cg_state *st = item_part ? S.d_state : nullptr;
+    if (launch_batch_apply_groups) {
+        int most = 0;
+        const batch_groups G = groups_of(S, set, degrees, &most);
+        return launch_batch_apply_groups(G, most, x, y, S.d_inst, item_part, st, slot, S.stream);
+    }
     for (int p : degrees) {
         int rc = launch_batch_apply(p, S.shape[p], x, y, S.d_inst, S.d_items[set][p], S.count(set, 2 + p),
-                                    S.item_cap[set][p], nullptr, nullptr, 0, S.stream);
+                                    S.item_cap[set][p], item_part ? item_part + S.item_base[set][p] : nullptr, st,
+                                    slot, S.stream);
         if (rc) return rc;
     }
     return SIPG_OK;
@@ -324,6 +346,12 @@ int apply_set(sipg_server &S, int set, const std::vector<int> &degrees, const do
 // per-item r.r and r.z; states non-null: finished requests are skipped
 int prec_set(sipg_server &S, int set, const std::vector<int> &degrees, double *pv, const cg_state *states,
              int slot) {
+    if (launch_batch_prec_groups) {
+        int most = 0;
+        const batch_groups G = groups_of(S, set, degrees, &most);
+        return launch_batch_prec_groups(G, most, S.pool[2], S.pool[6], pv, S.d_inst, S.d_item_rr[set],
+                                        S.d_item_rz[set], states, slot, S.stream);
+    }
     for (int p : degrees) {
         int rc = launch_batch_prec(p, S.shape[p], S.pool[2], S.pool[6], pv, S.d_inst, S.d_items[set][p],
                                    S.count(set, 2 + p), S.item_cap[set][p], S.d_item_rr[set] + S.item_base[set][p],
@@ -353,13 +381,28 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
     SIPG_HIP_TRY(hipStreamBeginCapture(S.stream, hipStreamCaptureModeRelaxed));
     for (int it = 0; it < kServeIters && !rc; ++it) {
         const int slot = it & 1;
-        for (int p : degrees) {
-            if ((rc = launch_batch_apply(p, S.shape[p], Pv, AP, S.d_inst, S.d_items[A][p], S.count(A, 2 + p),
-                                         S.item_cap[A][p], S.d_item_part + S.item_base[A][p], S.d_state, slot,
-                                         S.stream)))
+        if ((rc = apply_set(S, A, degrees, Pv, AP, S.d_item_part, slot))) break;
+        if (S.method == SIPG_METHOD_PCG && launch_batch_pcg_step) {
+            // as in the batched solver: the replacement set is folded and
+            // marked, has A x in Ap and takes b - A x for its r
+            const int Q = SET_REPL;
+            int most = 0;
+            const batch_groups G = groups_of(S, A, degrees, &most);
+            if (it == 0 &&
+                ((rc = launch_batch_pcg_fold(X, S.pool[5], Pv, S.d_chunks[Q], S.count(Q, 1), S.chunk_cap,
+                                             S.d_chunk_range[Q], S.d_item_range[A], S.d_item_part, S.d_state, slot,
+                                             S.stream)) ||
+                 (rc = apply_set(S, Q, degrees, X, AP))))
                 break;
+            if ((rc = launch_batch_pcg_step(G, most, Rv, AP, S.pool[1], S.pool[6], S.d_inst, S.d_item_range[A],
+                                            S.d_item_part, S.d_item_rr[A], S.d_item_rz[A], S.d_state, slot,
+                                            S.stream)) ||
+                (rc = launch_batch_pcg_update(S.pool[5], Pv, S.pool[6], S.d_chunks[A], S.count(A, 1), S.chunk_cap,
+                                              S.d_chunk_range[A], S.d_item_range[A], S.d_item_rr[A], S.d_item_rz[A],
+                                              S.d_state, slot, S.stream)))
+                break;
+            continue;
         }
-        if (rc) break;
         if ((rc = launch_batch_alpha(S.d_list[A], S.count(A, 0), kMaxSlots, S.d_item_range[A], S.d_item_part,
                                      S.d_state, slot, S.stream)) ||
             (rc = launch_batch_update_xr(S.pool[5], Pv, Rv, AP, S.d_chunks[A], S.count(A, 1), S.chunk_cap,

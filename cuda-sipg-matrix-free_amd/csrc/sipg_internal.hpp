@@ -70,6 +70,7 @@ struct cg_slot {
 constexpr int kSlotReplaced = 1;
 constexpr int kSlotRestart = 2;
 constexpr int kSlotWantCheck = 4;
+constexpr int kSlotStepped = 8;    // batched PCG: the iteration has its alpha (set for the update that ends it)
 // Batched and served solves: failed final true-residual checks that gain
 // less than 10% on the best failed one (counted over the whole solve) before
 // the solve is declared stuck at the floor of FP64 CG and ends, not
@@ -137,9 +138,21 @@ struct batch_ctl {
     double tol;
     int tol_mode, maxit;
 };
-// A BX x BY block of an instance for the operator kernel.
+// A block of an instance for the operator kernel: `rows` mesh rows from
+// (x0, y0), as wide as the kernel takes them.
 struct batch_item {
-    int inst, x0, y0, pad;
+    int inst, x0, y0, rows;
+};
+// The item lists of one launch, one to a degree; partial sums of list g
+// start at `base`.
+struct batch_group {
+    const batch_item *items;
+    const int *count;
+    int base, p;
+};
+struct batch_groups {
+    int n;
+    batch_group g[kMaxDegree];
 };
 // A range [begin, end) of the concatenated vectors, inside one instance.
 struct batch_chunk {
@@ -147,11 +160,21 @@ struct batch_chunk {
     int64_t begin, end;
 };
 // Candidate block shapes of the batched operator (the autotuner picks one
-// per degree): 16x4, 8x4, 8x2 elements.
+// per degree), named 16x4, 8x4 and 8x2.
 constexpr int kBatchShapes = 3;
 extern const int kBatchShapeBX[kBatchShapes];
 extern const int kBatchShapeBY[kBatchShapes];
 bool batch_shape_supported(int p, int shape);
+// The elements x rows of an item.  Weak: without it, the shape's name.
+__attribute__((weak)) void batch_item_extent(int p, int shape, int *bx, int *rows);
+inline void batch_extent(int p, int shape, int *bx, int *rows) {
+    if (batch_item_extent) {
+        batch_item_extent(p, shape, bx, rows);
+    } else {
+        *bx = kBatchShapeBX[shape];
+        *rows = kBatchShapeBY[shape];
+    }
+}
 
 // Reduction partial buffers hold at most this many block sums; consumers
 // add up at most this many themselves (more are first folded into one by a
@@ -304,6 +327,11 @@ int launch_convert(int from_dtype, int to_dtype, const void *src, void *dst, int
 int launch_batch_apply(int p, int shape, const double *X, double *Y, const batch_inst *inst,
                        const batch_item *items, const int *count, int max_items, double *item_part,
                        const cg_state *states, int slot, hipStream_t s);
+// the same over the lists of all degrees in one launch; max_items: the most
+// items they hold together.  Weak: without it, one launch to a degree.
+__attribute__((weak)) int launch_batch_apply_groups(const batch_groups &G, int max_items, const double *X, double *Y,
+                                                    const batch_inst *inst, double *item_part, const cg_state *states,
+                                                    int slot, hipStream_t s);
 int launch_batch_alpha(const int *list, const int *count, int max_inst, const int2 *item_range,
                        const double *item_part, cg_state *states, int slot, hipStream_t s);
 int launch_batch_update_xr(double *X, const double *Pv, double *Rv, const double *APv,
@@ -330,9 +358,34 @@ bool batch_prec_supported(int p, double pen, int shape);
 int launch_batch_prec(int p, int shape, const double *R, double *Zq, double *Pv, const batch_inst *inst,
                       const batch_item *items, const int *count, int max_items, double *item_rr, double *item_rz,
                       const cg_state *states, int slot, hipStream_t s);
+// An iteration around the operator's launch, over the lists of all degrees
+// (weak: a build has these, or iterates by launch_batch_alpha, update_xr,
+// fold, residual, mark, prec, beta_pcg and update_p).
+// z = M^-1 r (Pv non-null: also p = z), as launch_batch_prec
+__attribute__((weak)) int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq,
+                                                   double *Pv, const batch_inst *inst, double *item_rr,
+                                                   double *item_rz, const cg_state *states, int slot, hipStream_t s);
+// x += z + alpha p, z = 0 over the chunks of instances whose r is to be
+// replaced, and marks them; AP is to be A x of these before the step
+__attribute__((weak)) int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks,
+                                                const int *count, int max_chunks, const int2 *chunk_range,
+                                                const int2 *item_range, const double *item_part, cg_state *states,
+                                                int slot, hipStream_t s);
+// alpha = r.z / p.Ap, r -= alpha Ap (marked: r = b - Ap), z = M^-1 r
+__attribute__((weak)) int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP,
+                                                const double *B, double *Zq, const batch_inst *inst,
+                                                const int2 *item_range, const double *item_part, double *item_rr,
+                                                double *item_rz, cg_state *states, int slot, hipStream_t s);
+// beta = r.z(new) / r.z(old), z += alpha p (not where marked), p = zq + beta p;
+// next slot
+__attribute__((weak)) int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks,
+                                                  const int *count, int max_chunks, const int2 *chunk_range,
+                                                  const int2 *item_range, const double *item_rr,
+                                                  const double *item_rz, cg_state *states, int slot, hipStream_t s);
 // beta = r.z(new) / r.z(old) per instance from the item sums; next slot
-int launch_batch_beta_pcg(const int *list, const int *count, int max_inst, const int2 *item_range,
-                          const double *item_rr, const double *item_rz, cg_state *states, int slot, hipStream_t s);
+__attribute__((weak)) int launch_batch_beta_pcg(const int *list, const int *count, int max_inst,
+                                                const int2 *item_range, const double *item_rr, const double *item_rz,
+                                                cg_state *states, int slot, hipStream_t s);
 // x += z; z = 0 over the listed chunks (group update)
 int launch_batch_fold(double *X, double *Z, const batch_chunk *chunks, const int *count, int max_chunks,
                       hipStream_t s);
