@@ -73,6 +73,10 @@ void batch_apply_kernel(batch_groups G, const double *__restrict__ X, double *__
         if (DOT) {
             const double bs = block_sum<256>(d, red);
             if (threadIdx.x == 0) item_part[G.g[g].base + i] = bs;
+        } else {
+            // the next item's degree may place its waves' tiles where a wave
+            // still works on this one (with DOT the sum's barrier is between)
+            __syncthreads();
         }
     }
 }

@@ -60,6 +60,24 @@ def test_batch_of_every_degree_equals_single_applies(sipg, shape, top):
 
 
 @pytest.mark.parametrize("top", [8, 12, 16])
+def test_batch_of_more_items_than_workgroups(sipg, top):
+    """Workgroups take one item after another, of changing degrees whose tiles
+    lie elsewhere in LDS: 200 instances of each degree, to the bit the single
+    apply's results."""
+    kinds = [((64 // (p + 1) + 1, 5 + p % 5), p) for p in range(1, top + 1)]
+    xs = [np.random.default_rng(p).uniform(-1, 1, d[0] * d[1] * (p + 1) ** 2) for d, p in kinds]
+    ref = [sipg.Operator(d[0], d[1], p, sipg.pen_sigma(p), sipg.F64).apply_host(x) for (d, p), x in zip(kinds, xs)]
+    of = list(range(top)) * 200
+    B = _batch(sipg, [kinds[k][0] for k in of], [kinds[k][1] for k in of], (8, 2))
+    x, y = B.vector(), B.vector()
+    for i, k in enumerate(of):
+        B.upload(i, xs[k], x)
+    assert B.apply(x, y) == sipg.OK
+    bad = [(i, kinds[k]) for i, k in enumerate(of) if not np.array_equal(B.download(i, y), ref[k])]
+    assert not bad, (len(bad), bad[:5])
+
+
+@pytest.mark.parametrize("top", [8, 12, 16])
 def test_batch_pcg_of_every_degree(sipg, top):
     """Every degree in one launch, replacements on: each instance meets its
     tolerance on the true residual, as the single solve does; the solution
