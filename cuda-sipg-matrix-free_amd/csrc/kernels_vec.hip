@@ -375,6 +375,28 @@ __global__ __launch_bounds__(NT) void convert_kernel(const S *__restrict__ src, 
         dst[i] = (D)src[i];
 }
 
+// out = x + z in the reference order (node-major): out[q * noe + e] for
+// element e, node q, through 32 x 32 tiles whose rows are contiguous on
+// either side (padded: columns hit distinct banks).
+constexpr int LT = 32;
+__global__ __launch_bounds__(256) void solution_out_kernel(const double *__restrict__ x, const double *__restrict__ z,
+                                                           double *__restrict__ out, int64_t noe, int nq, int nqt) {
+    __shared__ double tile[LT][LT + 1];
+    const int64_t e0 = (int64_t)(blockIdx.x / nqt) * LT;
+    const int q0 = (int)(blockIdx.x % nqt) * LT;
+    const int tx = threadIdx.x % LT, ty = threadIdx.x / LT;
+    for (int i = ty; i < LT; i += 256 / LT) {
+        const int64_t e = e0 + i;
+        if (e < noe && q0 + tx < nq) {
+            const int64_t o = e * nq + q0 + tx;
+            tile[i][tx] = x[o] + z[o];
+        }
+    }
+    __syncthreads();
+    for (int i = ty; i < LT; i += 256 / LT)
+        if (q0 + i < nq && e0 + tx < noe) out[(int64_t)(q0 + i) * noe + e0 + tx] = tile[tx][i];
+}
+
 // Layout conversion between the reference order ((i1*(p+1)+i2)*noe + e) and
 // the element-major device order (e*(p+1)^2 + i1*(p+1)+i2).
 template <typename T>
@@ -699,6 +721,14 @@ int launch_convert(int from_dtype, int to_dtype, const void *src, void *dst, int
         hipLaunchKernelGGL((convert_kernel<double, double>), dim3(nb), dim3(NT), 0, s, (const double *)src, (double *)dst, n);
     else
         hipLaunchKernelGGL((convert_kernel<float, float>), dim3(nb), dim3(NT), 0, s, (const float *)src, (float *)dst, n);
+    SIPG_HIP_TRY(hipGetLastError());
+    return SIPG_OK;
+}
+
+int launch_solution_out(const double *x, const double *z, double *out, int64_t noe, int nq, hipStream_t s) {
+    const int64_t ne = (noe + LT - 1) / LT;
+    const int nqt = (nq + LT - 1) / LT;
+    hipLaunchKernelGGL(solution_out_kernel, dim3((unsigned)(ne * nqt)), dim3(256), 0, s, x, z, out, noe, nq, nqt);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }

@@ -392,6 +392,9 @@ int launch_batch_fold(double *X, double *Z, const batch_chunk *chunks, const int
 // sets kSlotReplaced on the listed instances (after their r = b - A x)
 int launch_batch_mark(const int *list, const int *count, int max_inst, cg_state *states, int slot,
                       hipStream_t s);
+// out = x + z in the reference order; FP64 (weak: without it, on the host)
+__attribute__((weak)) int launch_solution_out(const double *x, const double *z, double *out, int64_t noe, int nq,
+                                              hipStream_t s);
 // reference order <-> element-major device order (to_device = 1: ref -> dev)
 int launch_layout(int dtype, int to_device, const void *src, void *dst, int64_t noe, int nq,
                   hipStream_t s);
