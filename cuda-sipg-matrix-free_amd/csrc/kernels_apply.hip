@@ -169,7 +169,7 @@ int resolve_kernel(int dtype, int p, int kernel) {
 }
 
 int apply_num_blocks(int dtype, int p, int dimx, int dimy, int kernel) {
-    if (p > kMaxDegree) return p <= kMaxGenericDegree ? generic_apply_num_blocks(dimx, dimy) : -1;
+    if (p > kMaxDegree) return p <= kMaxGenericDegree ? generic_apply_num_blocks(dtype, p, dimx, dimy) : -1;
     const int k = resolve_kernel(dtype, p, kernel);
     if (k == SIPG_KERNEL_MFMA) return mfma_apply_num_blocks(dimx, dimy);
     if (k == SIPG_KERNEL_WAVE) return wave_apply_num_blocks(dtype, p, dimx, dimy);

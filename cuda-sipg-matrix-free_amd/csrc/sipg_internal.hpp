@@ -209,7 +209,7 @@ int launch_apply_mfma(int dtype, int p, const void *x, void *y, int dimx, int di
 // lives in the op's table allocation after the tables: such ops allocate
 // generic_table_len elements of their dtype for d_tab, of which the first
 // generic_face_offset hold the tables.
-int generic_apply_num_blocks(int dimx, int dimy);
+int generic_apply_num_blocks(int dtype, int p, int dimx, int dimy);
 size_t generic_face_offset(int p, size_t elem);
 size_t generic_table_len(int dtype, int p, int dimx, int dimy);
 int launch_apply_generic(int dtype, int p, const void *x, void *y, const void *tab, int dimx, int dimy, double pen,
