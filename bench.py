@@ -24,6 +24,7 @@ import numpy as np  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 DIM, P = 256, 8
 TOL = 1e-10
+FLOOR = 4 * TOL                      # where an FP64 solve that ends at its floor may be
 # Iteration caps: the FP64 solve needs about 4.7k iterations here and the
 # mixed one about 40k FP32 iterations; a solve that hits its cap fails
 # loudly instead of running to the default cap of n iterations.
@@ -79,7 +80,10 @@ def gpu_solve(sipg, op, b, x, method, rf2=1e-2):
         st, info = op.cg_ex(x, b, TOL, sipg.TOL_REL, maxit=MAXIT_FP64, replace_factor=3e-3,
                             true_stop=True, restart=0)
     t1 = time.perf_counter()
-    if st != sipg.OK:
+    # CG and block-Jacobi PCG may end at the FP64 floor of b - A x, which
+    # scatters about the tolerance here (of 24 forcings block-Jacobi PCG ends
+    # above it on 8, with any operator kernel); their legs then say so
+    if st != sipg.OK and not (st == sipg.NOT_CONVERGED and method in ("fp64", "pcg")):
         raise RuntimeError(f"{method} solve failed: {sipg.strerror(st)}")
     return t1 - t0, info
 
@@ -682,8 +686,8 @@ def main():
         t64.append(t)
         it64.append(info.iters)
     rel64 = op.true_relres(x64, b)
-    if not rel64 <= TOL:
-        raise RuntimeError(f"FP64 true relative residual {rel64:.3e} above {TOL}")
+    if not rel64 <= FLOOR:
+        raise RuntimeError(f"FP64 true relative residual {rel64:.3e} above {FLOOR}")
     ms64 = 1e3 * float(np.median(t64))
     log(f"fp64 : {ms64:.1f} ms/solve, {it64[-1]} iterations, {info.replacements} replacements, "
         f"{1e3 * ms64 / it64[-1]:.1f} us/iter, true relres {rel64:.2e}")
@@ -697,12 +701,12 @@ def main():
         tp.append(t)
         itp.append(infop.iters)
     relp = op.true_relres(xp, b)
-    if not relp <= TOL:
-        raise RuntimeError(f"PCG true relative residual {relp:.3e} above {TOL}")
+    if not relp <= FLOOR:
+        raise RuntimeError(f"PCG true relative residual {relp:.3e} above {FLOOR}")
     msp = 1e3 * float(np.median(tp))
     xp_h, x64_h = op.download(xp), op.download(x64)
     pcg = {"dof_per_s": n / (msp * 1e-3), "ms_per_solve": msp, "iterations": itp[-1],
-           "replacements": infop.replacements, "true_relres": relp,
+           "replacements": infop.replacements, "true_relres": relp, "converged": relp <= TOL,
            "us_per_iteration": 1e3 * msp / itp[-1],
            "rel_l2_vs_cg_solution": float(np.linalg.norm(xp_h - x64_h) / np.linalg.norm(x64_h)),
            "time_vs_cg": msp / ms64}
@@ -767,7 +771,8 @@ def main():
         mixed = {"status": f"failed: {exc}"}
         log(f"mixed: {exc}")
     # the timed solver: the fastest of the three
-    times = {"fp64": ms64, "pcg": msp, "pcg2": ms2}
+    times = {"pcg2": ms2}
+    times.update({m: t for m, t, rel in (("fp64", ms64, rel64), ("pcg", msp, relp)) if rel <= TOL})
     if mixed.get("status") == "ok":
         times["mixed"] = mixed["ms_per_solve"]
     solver = min(times, key=times.get)
@@ -831,7 +836,7 @@ def main():
             "solver": SOLVERS[solver] + " (the fastest of CG, PCG, two-level PCG and mixed here)",
             "iterations": it, "true_relres": relres,
             "error_vs_exact": {k: float(v) for k, v in err.items()},
-            "fp64_plain": {"dof_per_s": n / (ms64 * 1e-3), "ms_per_solve": ms64,
+            "fp64_plain": {"dof_per_s": n / (ms64 * 1e-3), "ms_per_solve": ms64, "converged": rel64 <= TOL,
                            "iterations": it64[-1], "true_relres": rel64},
             "pcg": pcg,
             "pcg2": pcg2,
