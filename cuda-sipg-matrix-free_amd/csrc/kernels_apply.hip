@@ -23,8 +23,8 @@
 // each XCD walks neighbouring strips of consecutive bands and the rows they
 // share are mostly in its own L2.
 #include "strip_apply.hpp"
+#include "strip_bands.hpp"
 
-#include <algorithm>
 #include <atomic>
 
 namespace sipg_internal {
@@ -75,30 +75,13 @@ int resident_groups() {
     return g;
 }
 
-// Bands per strip.  A wave costs its rows and about one more for the first
-// row's latency and the band's outer rows, and the workgroups run in rounds
-// of what the device holds: the count (at most one band per four rows, and
-// at most 4096 block sums while rows remain) that minimises rounds x rows.
-// Measured, us for bands so chosen / twice as many / half as many: FP64
-// 201 x 150, p = 7 8.7 / 10.9 / 10.0; 131 x 77, p = 12 11.8 / 12.3 / 13.7.
+// Bands per strip (strip_bands.hpp).  Measured, us for bands so chosen /
+// twice as many / half as many: FP64 201 x 150, p = 7 8.7 / 10.9 / 10.0;
+// 131 x 77, p = 12 11.8 / 12.3 / 13.7.
 template <typename T, int P>
 int num_bands(int dimx, int dimy) {
     constexpr int EPW = StripGeo<T, P>::EPW;
-    const int64_t nstrip = (dimx + EPW - 1) / EPW, res = resident_groups<T, P>();
-    const int most = (dimy + 3) / 4;
-    int best = 1;
-    double cost = 1e300;
-    for (int nb = 1; nb <= most; ++nb) {
-        if (nb > 1 && nstrip * nb > std::max<int64_t>(4 * res, 4096)) break;
-        const double rounds = (double)((nstrip * nb + res - 1) / res);
-        const double rows = (double)((dimy + nb - 1) / nb);
-        const double c = rounds * (((int)rows + 3) / 4 + 1.25);
-        if (c < cost * 0.999) {
-            cost = c;
-            best = nb;
-        }
-    }
-    return best;
+    return strip_bands((dimx + EPW - 1) / EPW, dimy, resident_groups<T, P>(), kMaxPartials);
 }
 
 template <typename T, int P>
