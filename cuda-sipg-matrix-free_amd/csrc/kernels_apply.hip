@@ -11,8 +11,8 @@
 // contiguous at e*(p+1)^2 + i1*(p+1) + i2.
 //
 // This file has the kernel of every compiled degree, strips of whole
-// elements per wave marched in y (strip_apply.hpp).  Even degrees up to 8
-// also have the block-staged kernel of kernels_apply_wave.hip.
+// elements per wave marched in y (strip_apply.hpp).  Even degrees up to 8, in
+// FP32 up to 12, also have the block-staged kernel of kernels_apply_wave.hip.
 //
 // The discrete operator is exactly the reference's (see the oracle and the
 // tests): Y = K1 U W + W U K1 + face terms of flux_term6a/6b, with the
@@ -142,12 +142,12 @@ int resolve_kernel(int dtype, int p, int kernel) {
     if (kernel == SIPG_KERNEL_MFMA) return mfma_apply_available(dtype, p) ? SIPG_KERNEL_MFMA : SIPG_KERNEL_VALU;
     if (kernel == SIPG_KERNEL_VALU) return SIPG_KERNEL_VALU;
     // AUTO: the matrix cores at p = 15 in FP32, the block-staged kernel at
-    // even p <= 8, strips elsewhere.  Strips store a lane's column, 8 (p+1)
-    // bytes to a segment, which costs most where it is short and the lines
-    // leave the caches partly written: 1024 x 1024, p = 8 FP64 330 against
-    // 278 us, FP32 256 x 256, p = 8 16.2 against 12.1.  At p = 15 in FP32
-    // strips take 3.9 against 2.8 us at 4 x 4, 4.5 against 4.8 at 64 x 64 and 8.9
-    // against 10.9 at 128 x 128, and are 5 % further from 64 bits (6.5e-8
+    // even p <= 8 and in FP32 <= 12, strips elsewhere.  Strips store a lane's
+    // column, sizeof(T) (p+1) bytes to a segment, which costs most where it is
+    // short and the lines leave the caches partly written: 1024 x 1024, p = 8
+    // FP64 330 against 278 us, FP32 256 x 256, p = 8 16.2 against 12.1.  At p = 15
+    // in FP32 strips take 3.9 against 2.8 us at 4 x 4, 4.5 against 4.8 at 64 x 64
+    // and 8.9 against 10.9 at 128 x 128, and are 5 % further from 64 bits (6.5e-8
     // against 6.2e-8 on uniform values): the matrix cores stay.
     if (mfma_apply_available(dtype, p)) return SIPG_KERNEL_MFMA;
     if (wave_apply_available(dtype, p)) return SIPG_KERNEL_WAVE;

@@ -1,7 +1,8 @@
 // kernels_apply_wave.hip -- the fused SIPG operator apply y = A x with
 // wave-owned elements on a block staged in LDS (volume + flux_term6a +
 // flux_term6b of the reference, volume_gpu_kernels.hpp:9-86,
-// sipg_sem_2d_gpu_kernels.hpp:189-316), for even degrees up to 8.
+// sipg_sem_2d_gpu_kernels.hpp:189-316), for even degrees up to 8, in FP32
+// up to 12.
 //
 // The same line arithmetic as the strip kernel (line_math.hpp), to the bit,
 // another work split: a wave holds EPW = 64 / (p+1) whole elements (7 at
@@ -21,7 +22,7 @@
 // kernels.  Even degrees (unpadded tiles, which the direct loads need).
 #include "line_math.hpp"
 
-#include <algorithm>
+#include <type_traits>
 
 namespace sipg_internal {
 
@@ -187,41 +188,46 @@ int wave_blocks(int dimx, int dimy) {
     return ((dimx + BX - 1) / BX) * ((dimy + BY - 1) / BY);
 }
 
+// f(std::integral_constant<int, P>) for a degree that has the kernel, else
+// `none`.  FP32 at p = 10 and 12 too: strips there take 8.7 against 6.8 us and
+// 10.7 against 7.6 at 128 x 128, 27.4 against 17.7 and 36.8 against 23.9 at
+// 300 x 300.  In FP64 they are level or ahead (p = 12, 200 x 200: 23.9 against
+// 25.8).
+template <typename T, class F>
+int by_wave_degree(int p, F f, int none) {
+    if (p == 2) return f(std::integral_constant<int, 2>{});
+    if (p == 4) return f(std::integral_constant<int, 4>{});
+    if (p == 6) return f(std::integral_constant<int, 6>{});
+    if (p == 8) return f(std::integral_constant<int, 8>{});
+    if constexpr (sizeof(T) == 4) {
+        if (p == 10) return f(std::integral_constant<int, 10>{});
+        if (p == 12) return f(std::integral_constant<int, 12>{});
+    }
+    return none;
+}
+
 template <typename T>
 int dispatch(int p, const void *x, void *y, int dimx, int dimy, double pen, double *partials, const cg_state *st,
              int slot, hipStream_t s)
 {
-    switch (p) {
-#define SIPG_WAVE_CASE(PP)                                                                 \
-    case PP:                                                                               \
-        if (partials) launch_wave<T, PP, true>(x, y, dimx, dimy, pen, partials, st, slot, s); \
-        else launch_wave<T, PP, false>(x, y, dimx, dimy, pen, partials, st, slot, s);         \
-        return SIPG_OK;
-        SIPG_WAVE_CASE(2)
-        SIPG_WAVE_CASE(4)
-        SIPG_WAVE_CASE(6)
-        SIPG_WAVE_CASE(8)
-#undef SIPG_WAVE_CASE
-    default:
-        return SIPG_ERR_UNSUPPORTED;
-    }
+    return by_wave_degree<T>(p, [&](auto deg) {
+        constexpr int P = decltype(deg)::value;
+        if (partials) launch_wave<T, P, true>(x, y, dimx, dimy, pen, partials, st, slot, s);
+        else launch_wave<T, P, false>(x, y, dimx, dimy, pen, partials, st, slot, s);
+        return (int)SIPG_OK;
+    }, SIPG_ERR_UNSUPPORTED);
 }
 
 template <typename T>
 int blocks(int p, int dimx, int dimy) {
-    switch (p) {
-    case 2: return wave_blocks<T, 2>(dimx, dimy);
-    case 4: return wave_blocks<T, 4>(dimx, dimy);
-    case 6: return wave_blocks<T, 6>(dimx, dimy);
-    case 8: return wave_blocks<T, 8>(dimx, dimy);
-    default: return -1;
-    }
+    return by_wave_degree<T>(p, [&](auto deg) { return wave_blocks<T, decltype(deg)::value>(dimx, dimy); }, -1);
 }
 
 }  // namespace
 
 bool wave_apply_available(int dtype, int p) {
-    return (dtype == SIPG_F64 || dtype == SIPG_F32) && (p == 2 || p == 4 || p == 6 || p == 8);
+    auto yes = [](auto) { return 1; };
+    return dtype == SIPG_F64 ? by_wave_degree<double>(p, yes, 0) : by_wave_degree<float>(p, yes, 0);
 }
 
 int wave_apply_num_blocks(int dtype, int p, int dimx, int dimy) {
