@@ -109,7 +109,7 @@ namespace {
 
 int items_for(const sipg_batch &b, int i, int shape, std::vector<batch_item> &out) {
     int BX, BY;
-    batch_extent(b.p[i], shape, &BX, &BY);
+    batch_item_extent(b.p[i], shape, &BX, &BY);
     const int nbx = (b.dimx[i] + BX - 1) / BX, nby = (b.dimy[i] + BY - 1) / BY;
     for (int by = 0; by < nby; ++by)
         for (int bx = 0; bx < nbx; ++bx) out.push_back({i, bx * BX, by * BY, BY});
@@ -186,44 +186,25 @@ batch_groups groups_of(sipg_batch &b, int set) {
 // y = A x over the instances of a list set; with p.Ap, of those that have
 // not finished at `slot`
 int apply_set(sipg_batch &b, int set, const double *x, double *y, double *item_part = nullptr, int slot = 0) {
-    const cg_state *st = item_part ? b.d_state : nullptr;
-    if (launch_batch_apply_groups)
-        return launch_batch_apply_groups(groups_of(b, set), b.item_total, x, y, b.d_inst, item_part, st, slot,
-                                         b.stream);
-    for (size_t g = 0; g < b.groups.size(); ++g) {
-        auto &G = b.groups[g];
-        int rc = launch_batch_apply(G.p, G.shape, x, y, b.d_inst, G.d_items[set], b.count(set, 2 + (int)g),
-                                    G.cap, item_part ? item_part + G.base : nullptr, st, slot, b.stream);
-        if (rc) return rc;
-    }
-    return SIPG_OK;
+    return launch_batch_apply_groups(groups_of(b, set), b.item_total, x, y, b.d_inst, item_part,
+                                     item_part ? b.d_state : nullptr, slot, b.stream);
 }
 
-// z = M^-1 r over the items of a list set (PCG; pv non-null: also p = z)
-int prec_set(sipg_batch &b, int set, double *pv, const cg_state *states, int slot) {
-    if (launch_batch_prec_groups)
-        return launch_batch_prec_groups(groups_of(b, set), b.item_total, b.R(), b.d_zq, pv, b.d_inst, b.d_item_rr,
-                                        b.d_item_rz, states, slot, b.stream);
-    for (size_t g = 0; g < b.groups.size(); ++g) {
-        auto &G = b.groups[g];
-        int rc = launch_batch_prec(G.p, G.shape, b.R(), b.d_zq, pv, b.d_inst, G.d_items[set],
-                                   b.count(set, 2 + (int)g), G.cap, b.d_item_rr + G.base, b.d_item_rz + G.base,
-                                   states, slot, b.stream);
-        if (rc) return rc;
-    }
-    return SIPG_OK;
+// z = p = M^-1 r over the items of a list set (PCG)
+int prec_set(sipg_batch &b, int set) {
+    return launch_batch_prec_groups(groups_of(b, set), b.item_total, b.R(), b.d_zq, b.Pv(), b.d_inst, b.d_item_rr,
+                                    b.d_item_rz, b.stream);
 }
 
 // One CG iteration of the active instances.  With `repl`, the instances of
 // the replacement set get r = b - A x between the x/r update and the p
-// update (reliable update; the set is empty in most replays).  With `pcg`,
-// z = M^-1 r follows (after any replacement), beta comes from r.z, and
-// p = z + beta p.
+// update (reliable update; the set is empty in most replays).  With `pcg`
+// the iteration is kernels_batch_pcg.hip's: beta from r.z, p = M^-1 r + beta p.
 int enqueue_iteration(sipg_batch &b, double *X, const double *Bv, int slot, bool repl, bool pcg) {
     const int A = SET_ACTIVE, Q = SET_REPL;
     int rc;
     if ((rc = apply_set(b, A, b.Pv(), b.AP(), b.d_item_part, slot))) return rc;
-    if (pcg && launch_batch_pcg_step) {
+    if (pcg) {
         // alpha and beta in the launches that use them; the replacement set
         // (marked by the fold) has A x in Ap and takes b - A x for its r
         if (repl && ((rc = launch_batch_pcg_fold(X, b.Z(), b.Pv(), b.d_chunks[Q], b.count(Q, 1), b.chunk_cap,
@@ -253,14 +234,6 @@ int enqueue_iteration(sipg_batch &b, double *X, const double *Bv, int slot, bool
                                         b.d_part2, b.d_part3, b.stream)) ||
             (rc = launch_batch_mark(b.d_list[Q], b.count(Q, 0), b.ninst, b.d_state, slot, b.stream)))
             return rc;
-    }
-    if (pcg) {
-        if ((rc = prec_set(b, A, nullptr, b.d_state, slot)) ||
-            (rc = launch_batch_beta_pcg(b.d_list[A], b.count(A, 0), b.ninst, b.d_item_range[A], b.d_item_rr,
-                                        b.d_item_rz, b.d_state, slot, b.stream)))
-            return rc;
-        return launch_batch_update_p(b.d_zq, b.Pv(), b.d_chunks[A], b.count(A, 1), b.chunk_cap, b.d_state, slot,
-                                     b.stream);
     }
     if ((rc = launch_batch_beta(b.d_list[A], b.count(A, 0), b.ninst, b.d_chunk_range[A], b.d_chunk_part,
                                 b.d_chunk_range[Q], b.d_part2, b.d_state, slot, b.stream)))
@@ -476,7 +449,7 @@ int batch_solve(sipg_batch *b, void *x, const void *rhs, const sipg_cg_opts *opt
     if ((rc = launch_batch_residual(Bv, B.AP(), B.R(), B.Pv(), B.d_chunks[SET_ALL], B.count(SET_ALL, 1),
                                     B.chunk_cap, B.d_part2, B.d_part3, B.stream)))
         return rc;
-    if (pcg && (rc = prec_set(B, SET_ALL, B.Pv(), nullptr, 0))) return rc;      // z = M^-1 r, p = z
+    if (pcg && (rc = prec_set(B, SET_ALL))) return rc;      // z = M^-1 r, p = z
     if ((rc = launch_batch_init(B.d_list[SET_ALL], B.count(SET_ALL, 0), ni, B.d_chunk_range[SET_ALL], B.d_part2,
                                 B.d_part3, B.d_state, B.d_ctl, pcg ? B.d_item_range[SET_ALL] : nullptr,
                                 pcg ? B.d_item_rz : nullptr, B.stream)))

@@ -51,18 +51,18 @@ __device__ __forceinline__ double wave_range_sum(const double *__restrict__ part
     return wave_total(s);
 }
 
-// z = M^-1 r for the items of all groups (COPYP: also p = z); an item's sums
-// of r.r and r.z go to item_rr and item_rz.  With states, items of instances
-// already finished at `slot` are skipped.  STEP: first alpha = r.z / p.Ap and
-// r -= alpha Ap, or r = b - Ap for an instance marked replaced (Ap holds A x
-// then).  A breakdown (p.Ap not positive, or not finite) skips the instance;
-// the update that follows sets its err.
+// z = M^-1 r for the items of all groups, and p = z at the start of a solve;
+// an item's sums of r.r and r.z go to item_rr and item_rz.  STEP (inside an
+// iteration): first alpha = r.z / p.Ap and r -= alpha Ap, or r = b - Ap for an
+// instance marked replaced (Ap holds A x then); items of instances already
+// finished at `slot` are skipped.  A breakdown (p.Ap not positive, or not
+// finite) skips the instance; the update that follows sets its err.
 //
 // A wave streams the runs of its item's rows on its own (prec_block.hpp).
 // With STEP four passes over memory, where the update of x and r and the
 // preconditioner took eight in two sets of launches: 46 + 74 us an iteration
 // on average over a solve of 128 instances of nine degrees, 44 now.
-template <int PMAX, bool STEP, bool COPYP>
+template <int PMAX, bool STEP>
 __global__ __launch_bounds__(256, PMAX <= 12 ? 3 : 2)
 void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__restrict__ AP,
                        const double *__restrict__ B, double *__restrict__ Zq, double *__restrict__ Pv,
@@ -86,7 +86,7 @@ void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__res
         const int i = k - __builtin_amdgcn_readfirstlane(first[g]);
         const batch_item it = G.g[g].items[i];
         cg_state *st = states + it.inst;
-        if (states && (st->s[slot].done | st->err)) continue;     // uniform over the workgroup
+        if (STEP && (st->s[slot].done | st->err)) continue;     // uniform over the workgroup
         const batch_inst in = inst[it.inst];
         const int at = G.g[g].base + i;
         const int tid = opaque(threadIdx.x);
@@ -114,7 +114,7 @@ void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__res
             double x0, x1;
             for (int gy = it.y0 + w; gy < yb; gy += 4) {
                 const int64_t o = in.off + ((int64_t)gy * in.dimx + it.x0) * Run::NQ;
-                prec_run<double, P, STEP, COPYP, true, false>((replaced ? B : R) + o, R + o, AP + o, Zq + o, Pv + o, nv,
+                prec_run<double, P, STEP, !STEP, true, false>((replaced ? B : R) + o, R + o, AP + o, Zq + o, Pv + o, nv,
                                                               [&] { return alpha; }, nullptr, tab + linv_at(P),
                                                               lds + w * Run::BUF, lane, srr, srz, x0, x1);
             }
@@ -134,7 +134,7 @@ void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__res
     }
 }
 
-template <int PMAX, bool STEP, bool COPYP>
+template <int PMAX, bool STEP>
 int resident_prec_groups(int pmax, size_t lds) {
     static std::atomic<int> cache[64][kMaxDegree + 1];
     int dev = 0;
@@ -144,28 +144,28 @@ int resident_prec_groups(int pmax, size_t lds) {
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&batch_prec_kernel<PMAX, STEP, COPYP>), 256, lds) != hipSuccess)
+            &per, reinterpret_cast<const void *>(&batch_prec_kernel<PMAX, STEP>), 256, lds) != hipSuccess)
         per = 0;
     g = (cus > 0 ? cus : 1) * (per > 0 ? per : 1);
     cache[dev][pmax].store(g, std::memory_order_relaxed);
     return g;
 }
 
-template <int PMAX, bool STEP, bool COPYP>
+template <int PMAX, bool STEP>
 int launch_prec_kernel(const batch_groups &G, int pmax, int max_items, double *R, const double *AP, const double *B,
                        double *Zq, double *Pv, const batch_inst *inst, const int2 *item_range,
                        const double *item_part, double *item_rr, double *item_rz, cg_state *states, int slot,
                        hipStream_t s) {
     const int tiles = prec_tiles_upto(pmax);
     const size_t lds = (size_t)(tiles + linv_at(pmax + 1)) * sizeof(double);
-    const dim3 grid(std::min(max_items, resident_prec_groups<PMAX, STEP, COPYP>(pmax, lds)));
-    hipLaunchKernelGGL((batch_prec_kernel<PMAX, STEP, COPYP>), grid, dim3(256), lds, s, G, tiles, R, AP, B, Zq, Pv,
+    const dim3 grid(std::min(max_items, resident_prec_groups<PMAX, STEP>(pmax, lds)));
+    hipLaunchKernelGGL((batch_prec_kernel<PMAX, STEP>), grid, dim3(256), lds, s, G, tiles, R, AP, B, Zq, Pv,
                        inst, item_range, item_part, item_rr, item_rz, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
 
-template <bool STEP, bool COPYP, class... A>
+template <bool STEP, class... A>
 int launch_prec_any(const batch_groups &G, int max_items, A... args) {
     int pmax = 0;
     for (int g = 0; g < G.n; ++g) {
@@ -173,9 +173,9 @@ int launch_prec_any(const batch_groups &G, int max_items, A... args) {
         pmax = std::max(pmax, G.g[g].p);
     }
     if (max_items <= 0 || pmax == 0) return SIPG_OK;
-    if (pmax <= 8) return launch_prec_kernel<8, STEP, COPYP>(G, pmax, max_items, args...);
-    if (pmax <= 12) return launch_prec_kernel<12, STEP, COPYP>(G, pmax, max_items, args...);
-    return launch_prec_kernel<16, STEP, COPYP>(G, pmax, max_items, args...);
+    if (pmax <= 8) return launch_prec_kernel<8, STEP>(G, pmax, max_items, args...);
+    if (pmax <= 12) return launch_prec_kernel<12, STEP>(G, pmax, max_items, args...);
+    return launch_prec_kernel<16, STEP>(G, pmax, max_items, args...);
 }
 
 // For the listed chunks of instances whose r is to be replaced: x += z +
@@ -308,34 +308,20 @@ bool batch_prec_supported(int p, double pen, int shape) {
 }
 
 int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq, double *Pv,
-                             const batch_inst *inst, double *item_rr, double *item_rz, const cg_state *states,
-                             int slot, hipStream_t s) {
-    auto *r = const_cast<double *>(R);                            // read only without STEP
-    auto *st = const_cast<cg_state *>(states);
+                             const batch_inst *inst, double *item_rr, double *item_rz, hipStream_t s) {
     const double *none = nullptr;
     const int2 *nor = nullptr;
-    return Pv ? launch_prec_any<false, true>(G, max_items, r, none, none, Zq, Pv, inst, nor, none, item_rr, item_rz, st,
-                                             slot, s)
-              : launch_prec_any<false, false>(G, max_items, r, none, none, Zq, Pv, inst, nor, none, item_rr, item_rz, st,
-                                              slot, s);
-}
-
-int launch_batch_prec(int p, int shape, const double *R, double *Zq, double *Pv, const batch_inst *inst,
-                      const batch_item *items, const int *count, int max_items, double *item_rr, double *item_rz,
-                      const cg_state *states, int slot, hipStream_t s) {
-    if (!batch_shape_supported(p, shape)) return SIPG_ERR_UNSUPPORTED;
-    batch_groups G;
-    G.n = 1;
-    G.g[0] = {items, count, 0, p};
-    return launch_batch_prec_groups(G, max_items, R, Zq, Pv, inst, item_rr, item_rz, states, slot, s);
+    cg_state *nos = nullptr;
+    return launch_prec_any<false>(G, max_items, const_cast<double *>(R) /* read only without STEP */, none, none, Zq,
+                                  Pv, inst, nor, none, item_rr, item_rz, nos, 0, s);
 }
 
 int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
                           double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
                           double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s) {
     double *nop = nullptr;
-    return launch_prec_any<true, false>(G, max_items, R, AP, B, Zq, nop, inst, item_range, item_part, item_rr, item_rz,
-                                        states, slot, s);
+    return launch_prec_any<true>(G, max_items, R, AP, B, Zq, nop, inst, item_range, item_part, item_rr, item_rz, states,
+                                 slot, s);
 }
 
 int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,

@@ -249,7 +249,7 @@ int upload_set(sipg_server &S, int set, const std::vector<int64_t> &ids,
         auto &v = items[R.p];
         const int s0 = (int)v.size();
         int BX, BY;
-        batch_extent(R.p, S.shape[R.p], &BX, &BY);
+        batch_item_extent(R.p, S.shape[R.p], &BX, &BY);
         for (int by = 0; by < (R.dim + BY - 1) / BY; ++by)
             for (int bx = 0; bx < (R.dim + BX - 1) / BX; ++bx) v.push_back({R.slot, bx * BX, by * BY, BY});
         item_range[R.slot] = int2{s0, (int)v.size()};   // based below
@@ -335,38 +335,18 @@ batch_groups groups_of(sipg_server &S, int set, const std::vector<int> &degrees,
 // finished at `slot`
 int apply_set(sipg_server &S, int set, const std::vector<int> &degrees, const double *x, double *y,
               double *item_part = nullptr, int slot = 0) {
-    const cg_state *st = item_part ? S.d_state : nullptr;
-    if (launch_batch_apply_groups) {
-        int most = 0;
-        const batch_groups G = groups_of(S, set, degrees, &most);
-        return launch_batch_apply_groups(G, most, x, y, S.d_inst, item_part, st, slot, S.stream);
-    }
-    for (int p : degrees) {
-        int rc = launch_batch_apply(p, S.shape[p], x, y, S.d_inst, S.d_items[set][p], S.count(set, 2 + p),
-                                    S.item_cap[set][p], item_part ? item_part + S.item_base[set][p] : nullptr, st,
-                                    slot, S.stream);
-        if (rc) return rc;
-    }
-    return SIPG_OK;
+    int most = 0;
+    const batch_groups G = groups_of(S, set, degrees, &most);
+    return launch_batch_apply_groups(G, most, x, y, S.d_inst, item_part, item_part ? S.d_state : nullptr, slot,
+                                     S.stream);
 }
 
-// z = M^-1 r over the items of a set (PCG; pv non-null: also p = z), with
-// per-item r.r and r.z; states non-null: finished requests are skipped
-int prec_set(sipg_server &S, int set, const std::vector<int> &degrees, double *pv, const cg_state *states,
-             int slot) {
-    if (launch_batch_prec_groups) {
-        int most = 0;
-        const batch_groups G = groups_of(S, set, degrees, &most);
-        return launch_batch_prec_groups(G, most, S.pool[2], S.pool[6], pv, S.d_inst, S.d_item_rr[set],
-                                        S.d_item_rz[set], states, slot, S.stream);
-    }
-    for (int p : degrees) {
-        int rc = launch_batch_prec(p, S.shape[p], S.pool[2], S.pool[6], pv, S.d_inst, S.d_items[set][p],
-                                   S.count(set, 2 + p), S.item_cap[set][p], S.d_item_rr[set] + S.item_base[set][p],
-                                   S.d_item_rz[set] + S.item_base[set][p], states, slot, S.stream);
-        if (rc) return rc;
-    }
-    return SIPG_OK;
+// z = p = M^-1 r over the items of a set (PCG), with per-item r.r and r.z
+int prec_set(sipg_server &S, int set, const std::vector<int> &degrees) {
+    int most = 0;
+    const batch_groups G = groups_of(S, set, degrees, &most);
+    return launch_batch_prec_groups(G, most, S.pool[2], S.pool[6], S.pool[3], S.d_inst, S.d_item_rr[set],
+                                    S.d_item_rz[set], S.stream);
 }
 
 std::vector<int> degrees_of(const sipg_server &S, const std::vector<int64_t> &ids) {
@@ -390,7 +370,7 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
     for (int it = 0; it < kServeIters && !rc; ++it) {
         const int slot = it & 1;
         if ((rc = apply_set(S, A, degrees, Pv, AP, S.d_item_part, slot))) break;
-        if (S.method == SIPG_METHOD_PCG && launch_batch_pcg_step) {
+        if (S.method == SIPG_METHOD_PCG) {
             // as in the batched solver: the replacement set is folded and
             // marked, has A x in Ap and takes b - A x for its r
             const int Q = SET_REPL;
@@ -425,16 +405,6 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
                                             S.d_part2, S.d_part3, S.stream)) ||
                 (rc = launch_batch_mark(S.d_list[Q], S.count(Q, 0), kMaxSlots, S.d_state, slot, S.stream)))
                 break;
-        }
-        if (S.method == SIPG_METHOD_PCG) {
-            // z = M^-1 r (after any replacement), beta from r.z, p = z + beta p
-            if ((rc = prec_set(S, A, degrees, nullptr, S.d_state, slot)) ||
-                (rc = launch_batch_beta_pcg(S.d_list[A], S.count(A, 0), kMaxSlots, S.d_item_range[A],
-                                            S.d_item_rr[A], S.d_item_rz[A], S.d_state, slot, S.stream)) ||
-                (rc = launch_batch_update_p(S.pool[6], Pv, S.d_chunks[A], S.count(A, 1), S.chunk_cap, S.d_state,
-                                            slot, S.stream)))
-                break;
-            continue;
         }
         if ((rc = launch_batch_beta(S.d_list[A], S.count(A, 0), kMaxSlots, S.d_chunk_range[A], S.d_chunk_part,
                                     S.d_chunk_range[SET_REPL], S.d_part2, S.d_state, slot, S.stream)) ||
@@ -802,7 +772,7 @@ int sipg_server_progress(sipg_server *S, int *n_done) {
         const bool pcg = S->method == SIPG_METHOD_PCG;
         if ((rc = launch_batch_residual(S->pool[1], S->pool[4], S->pool[2], S->pool[3], S->d_chunks[I],
                                         S->count(I, 1), S->chunk_cap, S->d_part2, S->d_part3, S->stream)) ||
-            (pcg && (rc = prec_set(*S, I, degrees_of(*S, admitted), S->pool[3], nullptr, 0))) ||
+            (pcg && (rc = prec_set(*S, I, degrees_of(*S, admitted)))) ||
             (rc = launch_batch_init(S->d_list[I], S->count(I, 0), kMaxSlots, S->d_chunk_range[I], S->d_part2,
                                     S->d_part3, S->d_state, S->d_ctl, pcg ? S->d_item_range[I] : nullptr,
                                     pcg ? S->d_item_rz[I] : nullptr, S->stream)))
@@ -884,25 +854,16 @@ int sipg_server_take_ex(sipg_server *S, int64_t *id, sipg_cg_info *info, double 
         const int64_t noe = (int64_t)R.dim * R.dim, nq = (int64_t)(R.p + 1) * (R.p + 1);
         // x + z: the increments after the last true residual (none unless the
         // request stopped on its iteration cap)
-        if (launch_solution_out) {
-            // in the reference order already, in the range that the finished
-            // request still holds in Ap's pool: one copy to the host, where two
-            // copies, the sum and the reordering took 7.7 ms for 24 solutions
-            // of 3.4 million values together, this 2.4
-            int rc = launch_solution_out(S->pool[0] + R.off, S->pool[5] + R.off, S->pool[4] + R.off, noe, (int)nq,
-                                         S->stream);
-            if (rc) return rc;
-            SIPG_HIP_TRY(hipMemcpyAsync(x_host, S->pool[4] + R.off, R.len * sizeof(double), hipMemcpyDeviceToHost,
-                                        S->stream));
-            SIPG_HIP_TRY(hipStreamSynchronize(S->stream));
-        } else {
-            std::vector<double> tmp(R.len), z(R.len);
-            SIPG_HIP_TRY(hipStreamSynchronize(S->stream));
-            SIPG_HIP_TRY(hipMemcpy(tmp.data(), S->pool[0] + R.off, R.len * sizeof(double), hipMemcpyDeviceToHost));
-            SIPG_HIP_TRY(hipMemcpy(z.data(), S->pool[5] + R.off, R.len * sizeof(double), hipMemcpyDeviceToHost));
-            for (int64_t e = 0; e < noe; ++e)
-                for (int64_t q = 0; q < nq; ++q) x_host[q * noe + e] = tmp[e * nq + q] + z[e * nq + q];
-        }
+        // in the reference order already, in the range that the finished
+        // request still holds in Ap's pool: one copy to the host, where two
+        // copies, the sum and the reordering took 7.7 ms for 24 solutions
+        // of 3.4 million values together, this 2.4
+        const int rc = launch_solution_out(S->pool[0] + R.off, S->pool[5] + R.off, S->pool[4] + R.off, noe, (int)nq,
+                                           S->stream);
+        if (rc) return rc;
+        SIPG_HIP_TRY(hipMemcpyAsync(x_host, S->pool[4] + R.off, R.len * sizeof(double), hipMemcpyDeviceToHost,
+                                    S->stream));
+        SIPG_HIP_TRY(hipStreamSynchronize(S->stream));
     }
     *id = rid;
     if (info) *info = R.info;

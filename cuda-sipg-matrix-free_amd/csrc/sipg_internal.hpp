@@ -165,16 +165,8 @@ constexpr int kBatchShapes = 3;
 extern const int kBatchShapeBX[kBatchShapes];
 extern const int kBatchShapeBY[kBatchShapes];
 bool batch_shape_supported(int p, int shape);
-// The elements x rows of an item.  Weak: without it, the shape's name.
-__attribute__((weak)) void batch_item_extent(int p, int shape, int *bx, int *rows);
-inline void batch_extent(int p, int shape, int *bx, int *rows) {
-    if (batch_item_extent) {
-        batch_item_extent(p, shape, bx, rows);
-    } else {
-        *bx = kBatchShapeBX[shape];
-        *rows = kBatchShapeBY[shape];
-    }
-}
+// The elements x rows of an item.
+void batch_item_extent(int p, int shape, int *bx, int *rows);
 
 // Reduction partial buffers hold at most this many block sums; consumers
 // add up at most this many themselves (more are first folded into one by a
@@ -235,11 +227,10 @@ int launch_cg_update_p(int dtype, const void *r, void *p, int64_t n, const doubl
                        int np_rr, int nblk, cg_state *st, int slot, hipStream_t s);
 // n_it whole CG iterations of a small problem in one launch
 // (kernels_small.hip), from the slot `slot`; the result is that of n_it
-// times apply, x/r update and p update.  Weak: a build without the kernel
-// iterates by the three launches.
-__attribute__((weak)) bool cg_small_fits(int p, int dimx, int dimy);
-__attribute__((weak)) int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy,
-                                          double pen, int n_it, cg_state *st, int slot, hipStream_t s);
+// times apply, x/r update and p update.
+bool cg_small_fits(int p, int dimx, int dimy);
+int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it,
+                    cg_state *st, int slot, hipStream_t s);
 int launch_residual(int dtype, const void *b, const void *Ax, void *r, int64_t n, hipStream_t s);
 // out = (out dtype)(b - Ax) with b, Ax in in_dtype; optionally p = out;
 // block sums of (b-Ax).(b-Ax) and, when pbb != nullptr, of b.b.
@@ -328,10 +319,10 @@ int launch_batch_apply(int p, int shape, const double *X, double *Y, const batch
                        const batch_item *items, const int *count, int max_items, double *item_part,
                        const cg_state *states, int slot, hipStream_t s);
 // the same over the lists of all degrees in one launch; max_items: the most
-// items they hold together.  Weak: without it, one launch to a degree.
-__attribute__((weak)) int launch_batch_apply_groups(const batch_groups &G, int max_items, const double *X, double *Y,
-                                                    const batch_inst *inst, double *item_part, const cg_state *states,
-                                                    int slot, hipStream_t s);
+// items they hold together
+int launch_batch_apply_groups(const batch_groups &G, int max_items, const double *X, double *Y,
+                              const batch_inst *inst, double *item_part, const cg_state *states, int slot,
+                              hipStream_t s);
 int launch_batch_alpha(const int *list, const int *count, int max_inst, const int2 *item_range,
                        const double *item_part, cg_state *states, int slot, hipStream_t s);
 int launch_batch_update_xr(double *X, const double *Pv, double *Rv, const double *APv,
@@ -351,50 +342,34 @@ int launch_batch_init(const int *list, const int *count, int max_inst, const int
                       const double *part_rr, const double *part_bb, cg_state *states, const batch_ctl *ctl,
                       const int2 *item_range, const double *item_rz, hipStream_t s);
 // ---- batched PCG (kernels_batch_pcg.hip) ----------------------------------
-// z = M^-1 r over the listed blocks of degree p (shape as the operator's;
-// Pv non-null: also p = z), with per-item r.r and r.z; finished instances
-// skipped when states is non-null.  Requires pen = 5 (p+1)^2.
+// Requires pen = 5 (p+1)^2.
 bool batch_prec_supported(int p, double pen, int shape);
-int launch_batch_prec(int p, int shape, const double *R, double *Zq, double *Pv, const batch_inst *inst,
-                      const batch_item *items, const int *count, int max_items, double *item_rr, double *item_rz,
-                      const cg_state *states, int slot, hipStream_t s);
-// An iteration around the operator's launch, over the lists of all degrees
-// (weak: a build has these, or iterates by launch_batch_alpha, update_xr,
-// fold, residual, mark, prec, beta_pcg and update_p).
-// z = M^-1 r (Pv non-null: also p = z), as launch_batch_prec
-__attribute__((weak)) int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq,
-                                                   double *Pv, const batch_inst *inst, double *item_rr,
-                                                   double *item_rz, const cg_state *states, int slot, hipStream_t s);
+// z = p = M^-1 r over the items of all degrees, with per-item r.r and r.z
+int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq, double *Pv,
+                             const batch_inst *inst, double *item_rr, double *item_rz, hipStream_t s);
+// An iteration around the operator's launch, over the lists of all degrees:
 // x += z + alpha p, z = 0 over the chunks of instances whose r is to be
 // replaced, and marks them; AP is to be A x of these before the step
-__attribute__((weak)) int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks,
-                                                const int *count, int max_chunks, const int2 *chunk_range,
-                                                const int2 *item_range, const double *item_part, cg_state *states,
-                                                int slot, hipStream_t s);
+int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,
+                          int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_part,
+                          cg_state *states, int slot, hipStream_t s);
 // alpha = r.z / p.Ap, r -= alpha Ap (marked: r = b - Ap), z = M^-1 r
-__attribute__((weak)) int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP,
-                                                const double *B, double *Zq, const batch_inst *inst,
-                                                const int2 *item_range, const double *item_part, double *item_rr,
-                                                double *item_rz, cg_state *states, int slot, hipStream_t s);
+int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
+                          double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
+                          double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s);
 // beta = r.z(new) / r.z(old), z += alpha p (not where marked), p = zq + beta p;
 // next slot
-__attribute__((weak)) int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks,
-                                                  const int *count, int max_chunks, const int2 *chunk_range,
-                                                  const int2 *item_range, const double *item_rr,
-                                                  const double *item_rz, cg_state *states, int slot, hipStream_t s);
-// beta = r.z(new) / r.z(old) per instance from the item sums; next slot
-__attribute__((weak)) int launch_batch_beta_pcg(const int *list, const int *count, int max_inst,
-                                                const int2 *item_range, const double *item_rr, const double *item_rz,
-                                                cg_state *states, int slot, hipStream_t s);
+int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks, const int *count,
+                            int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_rr,
+                            const double *item_rz, cg_state *states, int slot, hipStream_t s);
 // x += z; z = 0 over the listed chunks (group update)
 int launch_batch_fold(double *X, double *Z, const batch_chunk *chunks, const int *count, int max_chunks,
                       hipStream_t s);
 // sets kSlotReplaced on the listed instances (after their r = b - A x)
 int launch_batch_mark(const int *list, const int *count, int max_inst, cg_state *states, int slot,
                       hipStream_t s);
-// out = x + z in the reference order; FP64 (weak: without it, on the host)
-__attribute__((weak)) int launch_solution_out(const double *x, const double *z, double *out, int64_t noe, int nq,
-                                              hipStream_t s);
+// out = x + z in the reference order; FP64
+int launch_solution_out(const double *x, const double *z, double *out, int64_t noe, int nq, hipStream_t s);
 // reference order <-> element-major device order (to_device = 1: ref -> dev)
 int launch_layout(int dtype, int to_device, const void *src, void *dst, int64_t noe, int nq,
                   hipStream_t s);

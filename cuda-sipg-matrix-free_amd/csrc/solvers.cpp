@@ -220,8 +220,7 @@ struct Engine {
     // Plain CG on a problem that fits one workgroup: iterations without a
     // replacement run as one launch per chunk.
     bool small() const {
-        return !pcg && !xL && opI->kernel == SIPG_KERNEL_AUTO && launch_cg_small != nullptr &&
-               cg_small_fits(opI->p, opI->dimx, opI->dimy);
+        return !pcg && !xL && opI->kernel == SIPG_KERNEL_AUTO && cg_small_fits(opI->p, opI->dimx, opI->dimy);
     }
 
     // n_it iterations, the first of them replacing when asked

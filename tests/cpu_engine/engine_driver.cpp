@@ -14,7 +14,9 @@ extern "C" {
 namespace sipg_internal {
 int &mock_peeks();       // mock_kernels.cpp: solves finished by a peek
 int &mock_p_updates();   // mock_kernels.cpp: iterations enqueued
+int &mock_small_chunks();  // mock_kernels.cpp: launches of whole chunks of iterations
 }
+using sipg_internal::mock_small_chunks;
 using sipg_internal::mock_p_updates;
 using sipg_internal::mock_peeks;
 
@@ -118,6 +120,7 @@ static void run(const char *name, int d, int p, double pen, int mode, double tol
     sipg_cg_info info{};
     mock_peeks() = 0;
     mock_p_updates() = 0;
+    mock_small_chunks() = 0;
     if (mode == 0) {
         int it = 0;
         double res = 0;
@@ -143,9 +146,9 @@ static void run(const char *name, int d, int p, double pen, int mode, double tol
     double dx = 0, nx = 0;
     for (int64_t i = 0; i < n; ++i) { dx += (xh[i] - xo[i]) * (xh[i] - xo[i]); nx += xo[i] * xo[i]; }
     printf("{\"case\":\"%s\",\"rc\":%d,\"iters\":%d,\"reps\":%d,\"oracle_iters\":%d,"
-           "\"relres\":%.6e,\"diff\":%.6e,\"peeks\":%d,\"true_res\":%.6e,\"b_norm\":%.6e,\"launched\":%d}\n",
+           "\"relres\":%.6e,\"diff\":%.6e,\"peeks\":%d,\"true_res\":%.6e,\"b_norm\":%.6e,\"launched\":%d,\"chunks\":%d}\n",
            name, rc, info.iters, info.replacements, ito, relres(d, p, pen, xh, bh), std::sqrt(dx / nx), mock_peeks(),
-           info.true_res_norm, info.b_norm, launched);
+           info.true_res_norm, info.b_norm, launched, mock_small_chunks());
     sipg_free(x);
     sipg_free(b);
     sipg_op_destroy(op);
@@ -224,6 +227,14 @@ int main() {
     run("ex_nearer_floor", 8, 4, 125.0, 1, 1.3e-14, 0, 0.1, 0);
     run("pcg_near_floor", 8, 4, 125.0, 3, 2e-14, 0, 0.1, 0);
     run("pcg2_near_floor", 12, 3, 80.0, 5, 2e-14, 0, 0.1, 0);
+    // problems whose CG runs whole chunks of iterations in one launch
+    run("small_plain", 8, 3, 80.0, 0, 1e-10, 0, 0.0);
+    run("small_cap", 8, 3, 80.0, 0, 1e-12, 37, 0.0);
+    run("small_replace", 6, 4, 125.0, 1, 1e-10, 0, 0.1, 0);
+    run("small_noreplace", 6, 4, 125.0, 1, 1e-10, 0, 0.0, 0);
+    run("small_near_floor", 6, 4, 125.0, 1, 1.5e-14, 0, 0.1, 0);
+    run("small_mixed", 6, 4, 125.0, 2, 1e-10, 0, 0.1);
+    run("small_breakdown", 6, 3, -400.0, 0, 1e-10, 0, 0.0);
     coarse_check(5, 5, 3);
     coarse_check(6, 4, 2);
     coarse_check(4, 5, 1);

@@ -217,6 +217,68 @@ int launch_cg_update_p(int dtype, const void *r, void *p, int64_t n, const doubl
     return SIPG_OK;
 }
 
+// ---- CG inside one workgroup (kernels_small.hip): n_it iterations from slot
+// `slot`, the rules of the three launches above in one.  The limit is lower
+// than the kernel's (4,096 unknowns), so that small cases cover either way of
+// iterating.
+bool cg_small_fits(int p, int dimx, int dimy) {
+    return p >= 1 && p <= kMaxDegree && (int64_t)dimx * dimy * (p + 1) * (p + 1) <= 1024;
+}
+
+// launches of such chunks (read and reset by the engine driver)
+int &mock_small_chunks() {
+    static int n = 0;
+    return n;
+}
+
+template <typename T>
+static void small_t(int deg, T *x, T *r, T *p, int dimx, int dimy, double pen, int n_it, cg_state *st, int slot) {
+    cg_slot cur = st->s[slot];
+    const int last = (slot + n_it) & 1;
+    if (cur.done | st->err) { st->s[last] = cur; return; }
+    const int64_t n = (int64_t)dimx * dimy * (deg + 1) * (deg + 1);
+    std::vector<T> Ap(n);
+    int err = 0;
+    for (int it = 0; it < n_it && !cur.done && !err; ++it) {
+        apply_aos<T>(dimx, dimy, deg, pen, p, Ap.data());
+        double pAp = 0;
+        for (int64_t i = 0; i < n; ++i) pAp += (double)p[i] * (double)Ap[i];
+        const double alpha_d = cur.rr / pAp;
+        if (!(pAp > 0.0) || !std::isfinite(alpha_d)) { err = std::isfinite(pAp) ? 2 : 3; break; }
+        const T a = (T)alpha_d;
+        double rr = 0;
+        for (int64_t i = 0; i < n; ++i) {
+            x[i] = x[i] + a * p[i];
+            r[i] = r[i] - a * Ap[i];
+            rr += (double)r[i] * (double)r[i];
+        }
+        const T b = (T)(rr / cur.rr);
+        const bool met = !(std::sqrt(rr) > st->stop);
+        cg_slot nx{};
+        nx.rr = rr;
+        nx.rz = rr;
+        nx.beta = rr / cur.rr;
+        nx.it = cur.it + 1;
+        nx.done = ((met && !st->true_stop) || nx.it >= st->maxit) ? 1 : 0;
+        nx.flags = (met && st->true_stop) ? kSlotWantCheck : 0;
+        cur = nx;
+        if (!std::isfinite(rr)) err = 3;
+        for (int64_t i = 0; i < n; ++i) p[i] = r[i] + b * p[i];
+    }
+    st->s[last] = cur;
+    if (err) st->err = err;
+}
+
+int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it,
+                    cg_state *st, int slot, hipStream_t) {
+    if (!cg_small_fits(deg, dimx, dimy) || n_it < 1) return SIPG_ERR_INVALID;
+    mock_p_updates() += n_it;
+    ++mock_small_chunks();
+    if (dtype == SIPG_F64) small_t<double>(deg, tp<double>(x), tp<double>(r), tp<double>(p), dimx, dimy, pen, n_it, st, slot);
+    else small_t<float>(deg, tp<float>(x), tp<float>(r), tp<float>(p), dimx, dimy, pen, n_it, st, slot);
+    return SIPG_OK;
+}
+
 int launch_residual(int dtype, const void *b, const void *Ax, void *r, int64_t n, hipStream_t) {
     for (int64_t i = 0; i < n; ++i) {
         if (dtype == SIPG_F64) tp<double>(r)[i] = tp<double>(b)[i] - tp<double>(Ax)[i];

@@ -1,0 +1,62 @@
+"""The sanitised drivers run the host paths that the library has: every
+launcher that the host sources call is defined in them, as it is in the
+library, so none is chosen by whether it exists.  And the chunks of
+iterations that small CG solves run in one launch keep the solver's rules."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import PKG
+from test_cpu_engine import ENG, results  # noqa: F401  (the engine driver's cases)
+
+
+def _undefined_weak(path, *flags):
+    out = subprocess.run(["nm", *flags, path], check=True, capture_output=True, text=True).stdout
+    return [l.split()[-1] for l in out.splitlines() if l.split()[-2:-1] == ["w"] and "sipg" in l]
+
+
+@pytest.mark.parametrize("driver", ["engine_driver", "batch_driver", "serve_driver"])
+def test_no_launcher_is_optional_in_the_drivers(results, driver):  # noqa: F811  (builds them)
+    if shutil.which("nm") is None:
+        pytest.skip("no nm")
+    assert _undefined_weak(os.path.join(ENG, "_build", driver)) == []
+
+
+def test_no_launcher_is_optional_in_the_library():
+    so = os.path.join(PKG, "lib", "libsipg_hip.so")
+    if shutil.which("nm") is None or not os.path.exists(so):
+        pytest.skip("no nm or library")
+    assert _undefined_weak(so, "-D") == []
+
+
+def test_small_plain_cg_is_the_reference_iteration(results):  # noqa: F811
+    r = results["small_plain"]
+    assert r["rc"] == 0 and r["chunks"] > 0 and r["iters"] == r["oracle_iters"] and r["diff"] <= 1e-11, r
+
+
+def test_small_cg_iteration_cap(results):  # noqa: F811
+    r = results["small_cap"]
+    assert r["rc"] == 6 and r["chunks"] > 0 and r["iters"] == 37 and r["diff"] <= 1e-11, r
+
+
+@pytest.mark.parametrize("case", ["small_replace", "small_noreplace", "small_near_floor"])
+def test_small_cg_reaches_its_true_residual(results, case):  # noqa: F811
+    # a replacement interrupts the chunks; the host polls at most two chunks
+    # of 32 iterations behind
+    r = results[case]
+    tol = 1.5e-14 if case == "small_near_floor" else 1e-10
+    assert r["rc"] == 0 and r["chunks"] > 0 and r["reps"] >= 1 and r["relres"] <= tol, r
+    if case != "small_near_floor":
+        assert r["oracle_iters"] <= r["iters"] <= r["oracle_iters"] + 64, r
+
+
+def test_small_mixed_cycles(results):  # noqa: F811
+    r = results["small_mixed"]
+    assert r["rc"] == 0 and r["chunks"] > 0 and r["relres"] <= 1e-10 and r["diff"] <= 1e-8, r
+
+
+def test_small_cg_breakdown(results):  # noqa: F811
+    r = results["small_breakdown"]
+    assert r["rc"] == 8 and r["chunks"] > 0, r
