@@ -82,6 +82,8 @@ struct sipg_batch {
     double *d_item_part = nullptr, *d_chunk_part = nullptr, *d_part2 = nullptr, *d_part3 = nullptr;
     double *d_item_rr = nullptr, *d_item_rz = nullptr;   // PCG: per-item r.r and r.z
     double *d_zq = nullptr;              // PCG: z = M^-1 r (allocated on first use)
+    double *d_total = nullptr;           // PCG: p.Ap, r.r and r.z of the instances with many items (3 x ninst)
+    bool many_items = false;             // some instance has more than kDirectItems
     int item_total = 0, chunk_cap = 0;
     int *d_counts = nullptr;             // NSETS x (2 + ngroups)
     int *d_list[NSETS] = {};
@@ -207,18 +209,26 @@ int enqueue_iteration(sipg_batch &b, double *X, const double *Bv, int slot, bool
     if (pcg) {
         // alpha and beta in the launches that use them; the replacement set
         // (marked by the fold) has A x in Ap and takes b - A x for its r
+        const item_sum pAp{b.d_item_part, b.d_total}, rr{b.d_item_rr, b.d_total + b.ninst},
+            rz{b.d_item_rz, b.d_total + 2 * (size_t)b.ninst};
+        auto totals = [&](item_sum u, item_sum v) {
+            return !b.many_items ? SIPG_OK
+                                 : launch_batch_totals(b.d_list[A], b.count(A, 0), b.ninst, b.d_item_range[A], u, v,
+                                                       b.stream);
+        };
+        if ((rc = totals(pAp, item_sum{}))) return rc;
         if (repl && ((rc = launch_batch_pcg_fold(X, b.Z(), b.Pv(), b.d_chunks[Q], b.count(Q, 1), b.chunk_cap,
-                                                 b.d_chunk_range[Q], b.d_item_range[A], b.d_item_part, b.d_state,
-                                                 slot, b.stream)) ||
+                                                 b.d_chunk_range[Q], b.d_item_range[A], pAp, b.d_state, slot,
+                                                 b.stream)) ||
                      (rc = apply_set(b, Q, X, b.AP()))))
             return rc;
         if ((rc = launch_batch_pcg_step(groups_of(b, A), b.item_total, b.R(), b.AP(), Bv, b.d_zq, b.d_inst,
-                                        b.d_item_range[A], b.d_item_part, b.d_item_rr, b.d_item_rz, b.d_state, slot,
-                                        b.stream)))
+                                        b.d_item_range[A], pAp, b.d_item_rr, b.d_item_rz, b.d_state, slot,
+                                        b.stream)) ||
+            (rc = totals(rr, rz)))
             return rc;
         return launch_batch_pcg_update(b.Z(), b.Pv(), b.d_zq, b.d_chunks[A], b.count(A, 1), b.chunk_cap,
-                                       b.d_chunk_range[A], b.d_item_range[A], b.d_item_rr, b.d_item_rz, b.d_state,
-                                       slot, b.stream);
+                                       b.d_chunk_range[A], b.d_item_range[A], rr, rz, b.d_state, slot, b.stream);
     }
     if ((rc = launch_batch_alpha(b.d_list[A], b.count(A, 0), b.ninst, b.d_item_range[A], b.d_item_part,
                                  b.d_state, slot, b.stream)))
@@ -257,10 +267,15 @@ int dmalloc(Tp **p, size_t n) {
 int alloc_lists(sipg_batch &b) {
     int rc;
     b.item_total = 0;
+    b.many_items = false;
     for (auto &G : b.groups) {
         std::vector<batch_item> tmp;
         G.cap = 0;
-        for (int i : G.inst) G.cap += items_for(b, i, G.shape, tmp);
+        for (int i : G.inst) {
+            const int n = items_for(b, i, G.shape, tmp);
+            G.cap += n;
+            b.many_items = b.many_items || n > kDirectItems;
+        }
         G.base = b.item_total;
         b.item_total += G.cap;
         for (int s = 0; s < NSETS; ++s) {
@@ -424,13 +439,14 @@ int batch_solve(sipg_batch *b, void *x, const void *rhs, const sipg_cg_opts *opt
     int rc = ensure_tuned(*b);
     if (rc) return rc;
     sipg_batch &B = *b;
+    const int ni = B.ninst;
     if (pcg) {
         for (const auto &G : B.groups)
             for (int i : G.inst)
                 if (!batch_prec_supported(G.p, B.pen[i], G.shape)) return SIPG_ERR_UNSUPPORTED;
         if (!B.d_zq && (rc = dmalloc(&B.d_zq, (size_t)B.total()))) return rc;
+        if (!B.d_total && (rc = dmalloc(&B.d_total, 3 * (size_t)ni))) return rc;
     }
-    const int ni = B.ninst;
     double *X = (double *)x;
     const double *Bv = (const double *)rhs;
     const bool true_stop = opts->true_residual_stop != 0;
@@ -691,7 +707,7 @@ int sipg_batch_destroy(sipg_batch *b) {
         for (int s = 0; s < NSETS; ++s)
             if (G.d_items[s]) (void)hipFree(G.d_items[s]);
     void *dev[] = {b->d_inst, b->d_state, b->d_ctl, b->ws, b->d_item_part, b->d_chunk_part,
-                   b->d_part2, b->d_part3, b->d_counts, b->d_modes, b->d_item_rr, b->d_item_rz, b->d_zq};
+                   b->d_part2, b->d_part3, b->d_counts, b->d_modes, b->d_item_rr, b->d_item_rz, b->d_zq, b->d_total};
     for (void *q : dev)
         if (q) (void)hipFree(q);
     for (int s = 0; s < NSETS; ++s) {

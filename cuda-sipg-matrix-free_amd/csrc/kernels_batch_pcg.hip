@@ -8,9 +8,11 @@
 // An iteration is three launches over all degrees: the operator with p.Ap
 // (kernels_batch.hip); alpha, r -= alpha Ap and z = M^-1 r; beta, x += alpha
 // p and p = z + beta p.  Each workgroup sums the p.Ap or r.r and r.z shares
-// of its instance by itself, in a fixed order.  Where some instances' r is
-// replaced by b - A x, a fold of their x and the operator on them come
-// between the first two, and the second takes b - A x for its r.
+// of its instance by itself, in a fixed order; where a large instance is in
+// the lists, a launch after the operator's and one after the second add up
+// its shares (batch_totals_kernel).  Where some instances' r is replaced by
+// b - A x, a fold of their x and the operator on them come before the second,
+// and that takes b - A x for its r.
 //
 // Within a launch, an instance's state is written by the workgroup of its
 // first item or chunk only, in fields that the others do not read: the
@@ -44,11 +46,43 @@ int prec_tiles_upto(int p) {
     return *std::max_element(need.begin(), need.begin() + p);
 }
 
-// sum of part[b, e) in a fixed order, in every lane of the wave
-__device__ __forceinline__ double wave_range_sum(const double *__restrict__ part, int b, int e, int lane) {
+// the instance's sum, in every lane of the wave, in a fixed order
+__device__ __forceinline__ double instance_sum(item_sum q, const int2 *__restrict__ item_range, int inst, int lane) {
+    const int2 r = item_range[inst];
+    if (r.y - r.x > kDirectItems) return q.total[inst];
     double s = 0.0;
-    for (int i = b + lane; i < e; i += 64) s += part[i];
+    for (int i = r.x + lane; i < r.y; i += 64) s += q.part[i];
     return wave_total(s);
+}
+
+// The sums of the listed instances that have more than kDirectItems items,
+// one workgroup to each.
+//
+// Without it every item and every chunk of such an instance adds up all its
+// items, three times an iteration, which grows with the square of its size:
+// us an iteration so, and now: one instance of 512 x 512 elements, p = 8 622,
+// 458; 2048 x 2048, p = 2 3755, 825; 3000 x 3000, p = 1 4480, 811.  kDirectItems:
+// with fewer items the two launches cost as much as they save (384 items, 192 x
+// 192, p = 4: 35.9 directly, 36.6 with them; 672, 192 x 192, p = 8: 71.8, 70.0).
+template <int K>
+__global__ __launch_bounds__(VT) void batch_totals_kernel(const int *__restrict__ list, const int *__restrict__ count,
+                                                          const int2 *__restrict__ item_range, item_sum a,
+                                                          item_sum b) {
+    const int n = *count;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const int inst = list[k];
+        const int2 r = item_range[inst];
+        const int m = r.y - r.x;
+        if (m <= kDirectItems) continue;                          // uniform over the workgroup
+        double out[K];
+        if constexpr (K == 1) multi_sum<VT, 1>({a.part + r.x}, {m}, out);
+        else multi_sum<VT, 2>({a.part + r.x, b.part + r.x}, {m, m}, out);
+        if (threadIdx.x == 0) {
+            a.total[inst] = out[0];
+            if constexpr (K == 2) b.total[inst] = out[K - 1];
+        }
+        __syncthreads();                                          // the next instance's sums take the same LDS
+    }
 }
 
 // z = M^-1 r for the items of all groups, and p = z at the start of a solve;
@@ -67,8 +101,8 @@ __global__ __launch_bounds__(256, PMAX <= 12 ? 3 : 2)
 void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__restrict__ AP,
                        const double *__restrict__ B, double *__restrict__ Zq, double *__restrict__ Pv,
                        const batch_inst *__restrict__ inst, const int2 *__restrict__ item_range,
-                       const double *__restrict__ item_part, double *__restrict__ item_rr,
-                       double *__restrict__ item_rz, cg_state *states, int slot)
+                       item_sum part, double *__restrict__ item_rr, double *__restrict__ item_rz, cg_state *states,
+                       int slot)
 {
     extern __shared__ __attribute__((aligned(16))) double lds[];
     __shared__ double red[2][4];
@@ -94,10 +128,9 @@ void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__res
         const bool replaced = STEP && (st->s[slot].flags & kSlotReplaced);
         double alpha = 0.0;
         if (STEP) {
-            const int2 range = item_range[it.inst];
-            const double pAp = wave_range_sum(item_part, range.x, range.y, lane);
+            const double pAp = instance_sum(part, item_range, it.inst, lane);
             alpha = st->s[slot].rz / pAp;
-            if (at == range.x && tid == 0) {
+            if (at == item_range[it.inst].x && tid == 0) {
                 st->s[slot].alpha = alpha;
                 st->s[slot].pAp = pAp;
                 st->s[slot].flags |= kSlotStepped;
@@ -154,13 +187,12 @@ int resident_prec_groups(int pmax, size_t lds) {
 template <int PMAX, bool STEP>
 int launch_prec_kernel(const batch_groups &G, int pmax, int max_items, double *R, const double *AP, const double *B,
                        double *Zq, double *Pv, const batch_inst *inst, const int2 *item_range,
-                       const double *item_part, double *item_rr, double *item_rz, cg_state *states, int slot,
-                       hipStream_t s) {
+                       item_sum part, double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s) {
     const int tiles = prec_tiles_upto(pmax);
     const size_t lds = (size_t)(tiles + linv_at(pmax + 1)) * sizeof(double);
     const dim3 grid(std::min(max_items, resident_prec_groups<PMAX, STEP>(pmax, lds)));
     hipLaunchKernelGGL((batch_prec_kernel<PMAX, STEP>), grid, dim3(256), lds, s, G, tiles, R, AP, B, Zq, Pv,
-                       inst, item_range, item_part, item_rr, item_rz, states, slot);
+                       inst, item_range, part, item_rr, item_rz, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
@@ -186,16 +218,14 @@ __global__ __launch_bounds__(VT) void batch_pcg_fold_kernel(double *__restrict__
                                                             const batch_chunk *__restrict__ chunks,
                                                             const int *__restrict__ count,
                                                             const int2 *__restrict__ chunk_range,
-                                                            const int2 *__restrict__ item_range,
-                                                            const double *__restrict__ item_part, cg_state *states,
-                                                            int slot) {
+                                                            const int2 *__restrict__ item_range, item_sum part,
+                                                            cg_state *states, int slot) {
     const int n = *count;
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
         const batch_chunk c = chunks[k];
         cg_state *st = states + c.inst;
         if (st->s[slot].done | st->err) continue;
-        const int2 r = item_range[c.inst];
-        const double pAp = wave_range_sum(item_part, r.x, r.y, threadIdx.x & 63);
+        const double pAp = instance_sum(part, item_range, c.inst, threadIdx.x & 63);
         const double alpha = st->s[slot].rz / pAp;
         if (!(pAp > 0.0) || !isfinite(alpha)) continue;
         if (k == chunk_range[c.inst].x && threadIdx.x == 0) {
@@ -225,9 +255,7 @@ __global__ __launch_bounds__(VT) void batch_pcg_update_kernel(double *__restrict
                                                               const int *__restrict__ count,
                                                               const int2 *__restrict__ chunk_range,
                                                               const int2 *__restrict__ item_range,
-                                                              const double *__restrict__ item_rr,
-                                                              const double *__restrict__ item_rz, cg_state *states,
-                                                              int slot) {
+                                                              item_sum rr, item_sum rz, cg_state *states, int slot) {
     const int n = *count;
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
         const batch_chunk c = chunks[k];
@@ -244,10 +272,9 @@ __global__ __launch_bounds__(VT) void batch_pcg_update_kernel(double *__restrict
             }
             continue;
         }
-        const int2 r = item_range[c.inst];
         const int lane = threadIdx.x & 63;
-        const double rr_new = wave_range_sum(item_rr, r.x, r.y, lane);
-        const double rz_new = wave_range_sum(item_rz, r.x, r.y, lane);
+        const double rr_new = instance_sum(rr, item_range, c.inst, lane);
+        const double rz_new = instance_sum(rz, item_range, c.inst, lane);
         const double alpha = cur.alpha, beta = rz_new / cur.rz;
         const bool replaced = (cur.flags & kSlotReplaced) != 0;
         if (lead) {
@@ -313,31 +340,42 @@ int launch_batch_prec_groups(const batch_groups &G, int max_items, const double 
     const int2 *nor = nullptr;
     cg_state *nos = nullptr;
     return launch_prec_any<false>(G, max_items, const_cast<double *>(R) /* read only without STEP */, none, none, Zq,
-                                  Pv, inst, nor, none, item_rr, item_rz, nos, 0, s);
+                                  Pv, inst, nor, item_sum{}, item_rr, item_rz, nos, 0, s);
+}
+
+int launch_batch_totals(const int *list, const int *count, int max_inst, const int2 *item_range, item_sum a,
+                        item_sum b, hipStream_t s) {
+    const dim3 grid(std::max(1, std::min(max_inst, 2048)));
+    if (b.part)
+        hipLaunchKernelGGL(batch_totals_kernel<2>, grid, dim3(VT), 0, s, list, count, item_range, a, b);
+    else
+        hipLaunchKernelGGL(batch_totals_kernel<1>, grid, dim3(VT), 0, s, list, count, item_range, a, b);
+    SIPG_HIP_TRY(hipGetLastError());
+    return SIPG_OK;
 }
 
 int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
-                          double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
-                          double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s) {
+                          double *Zq, const batch_inst *inst, const int2 *item_range, item_sum pAp, double *item_rr,
+                          double *item_rz, cg_state *states, int slot, hipStream_t s) {
     double *nop = nullptr;
-    return launch_prec_any<true>(G, max_items, R, AP, B, Zq, nop, inst, item_range, item_part, item_rr, item_rz, states,
+    return launch_prec_any<true>(G, max_items, R, AP, B, Zq, nop, inst, item_range, pAp, item_rr, item_rz, states,
                                  slot, s);
 }
 
 int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,
-                          int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_part,
+                          int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum pAp,
                           cg_state *states, int slot, hipStream_t s) {
     hipLaunchKernelGGL(batch_pcg_fold_kernel, dim3(std::max(1, std::min(max_chunks, 2048))), dim3(VT), 0, s, X, Z, Pv,
-                       chunks, count, chunk_range, item_range, item_part, states, slot);
+                       chunks, count, chunk_range, item_range, pAp, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }
 
 int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks, const int *count,
-                            int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_rr,
-                            const double *item_rz, cg_state *states, int slot, hipStream_t s) {
+                            int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum rr,
+                            item_sum rz, cg_state *states, int slot, hipStream_t s) {
     hipLaunchKernelGGL(batch_pcg_update_kernel, dim3(std::max(1, std::min(max_chunks, 2048))), dim3(VT), 0, s, Z, Pv,
-                       Zq, chunks, count, chunk_range, item_range, item_rr, item_rz, states, slot);
+                       Zq, chunks, count, chunk_range, item_range, rr, rz, states, slot);
     SIPG_HIP_TRY(hipGetLastError());
     return SIPG_OK;
 }

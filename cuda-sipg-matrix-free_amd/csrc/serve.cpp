@@ -110,6 +110,7 @@ struct sipg_server {
     int *d_counts = nullptr;                 // NSETS x (2 + kMaxDegree + 1)
     double *d_item_part = nullptr, *d_chunk_part = nullptr, *d_part2 = nullptr, *d_part3 = nullptr;
     double *d_item_rr[NSETS] = {}, *d_item_rz[NSETS] = {};
+    double *d_total = nullptr;               // PCG: p.Ap, r.r, r.z of requests with many items (3 x kMaxSlots)
     char *h_stage[NSETS] = {};
     size_t stage_bytes[NSETS] = {};
     hipEvent_t stage_ev[NSETS] = {};
@@ -119,6 +120,7 @@ struct sipg_server {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<int> graph_degrees;
+    bool graph_totals = false;               // it adds up the sums of requests with many items
     bool graph_stale = true;
     bool repl_empty = false;                 // the replacement lists on the device are so
     bool replayed = false;                   // h_state holds a replay's outcome
@@ -358,6 +360,19 @@ std::vector<int> degrees_of(const sipg_server &S, const std::vector<int64_t> &id
     return d;
 }
 
+// Whether a running request has more items than its launches add up by
+// themselves (PCG).
+bool many_items(const sipg_server &S) {
+    if (S.method != SIPG_METHOD_PCG) return false;
+    for (int64_t id : S.active) {
+        const Request &R = S.reqs.at(id);
+        int BX, BY;
+        batch_item_extent(R.p, S.shape[R.p], &BX, &BY);
+        if ((int64_t)((R.dim + BX - 1) / BX) * ((R.dim + BY - 1) / BY) > kDirectItems) return true;
+    }
+    return false;
+}
+
 int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
     if (S.exec) (void)hipGraphExecDestroy(S.exec);
     if (S.graph) (void)hipGraphDestroy(S.graph);
@@ -365,6 +380,14 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
     S.graph = nullptr;
     double *X = S.pool[0], *Rv = S.pool[2], *Pv = S.pool[3], *AP = S.pool[4];
     const int A = SET_ACTIVE;
+    const bool with_totals = many_items(S);
+    const item_sum pAp{S.d_item_part, S.d_total}, rr{S.d_item_rr[A], S.d_total + kMaxSlots},
+        rz{S.d_item_rz[A], S.d_total + 2 * kMaxSlots};
+    auto totals = [&](item_sum u, item_sum v) {
+        return !with_totals ? SIPG_OK
+                            : launch_batch_totals(S.d_list[A], S.count(A, 0), kMaxSlots, S.d_item_range[A], u, v,
+                                                  S.stream);
+    };
     int rc = SIPG_OK;
     SIPG_HIP_TRY(hipStreamBeginCapture(S.stream, hipStreamCaptureModeRelaxed));
     for (int it = 0; it < kServeIters && !rc; ++it) {
@@ -376,18 +399,18 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
             const int Q = SET_REPL;
             int most = 0;
             const batch_groups G = groups_of(S, A, degrees, &most);
+            if ((rc = totals(pAp, item_sum{}))) break;
             if (it == 0 &&
                 ((rc = launch_batch_pcg_fold(X, S.pool[5], Pv, S.d_chunks[Q], S.count(Q, 1), S.chunk_cap,
-                                             S.d_chunk_range[Q], S.d_item_range[A], S.d_item_part, S.d_state, slot,
-                                             S.stream)) ||
+                                             S.d_chunk_range[Q], S.d_item_range[A], pAp, S.d_state, slot, S.stream)) ||
                  (rc = apply_set(S, Q, degrees, X, AP))))
                 break;
-            if ((rc = launch_batch_pcg_step(G, most, Rv, AP, S.pool[1], S.pool[6], S.d_inst, S.d_item_range[A],
-                                            S.d_item_part, S.d_item_rr[A], S.d_item_rz[A], S.d_state, slot,
-                                            S.stream)) ||
+            if ((rc = launch_batch_pcg_step(G, most, Rv, AP, S.pool[1], S.pool[6], S.d_inst, S.d_item_range[A], pAp,
+                                            S.d_item_rr[A], S.d_item_rz[A], S.d_state, slot, S.stream)) ||
+                (rc = totals(rr, rz)) ||
                 (rc = launch_batch_pcg_update(S.pool[5], Pv, S.pool[6], S.d_chunks[A], S.count(A, 1), S.chunk_cap,
-                                              S.d_chunk_range[A], S.d_item_range[A], S.d_item_rr[A], S.d_item_rz[A],
-                                              S.d_state, slot, S.stream)))
+                                              S.d_chunk_range[A], S.d_item_range[A], rr, rz, S.d_state, slot,
+                                              S.stream)))
                 break;
             continue;
         }
@@ -424,6 +447,7 @@ int capture_graph(sipg_server &S, const std::vector<int> &degrees) {
         return SIPG_ERR_HIP;
     }
     S.graph_degrees = degrees;
+    S.graph_totals = with_totals;
     S.graph_stale = false;
     return SIPG_OK;
 }
@@ -479,7 +503,7 @@ int sipg_server_destroy(sipg_server *S) {
     for (double *p : S->pool)
         if (p) (void)hipFree(p);
     void *dev[] = {S->d_inst, S->d_state, S->d_ctl, S->d_modes, S->d_counts, S->d_item_part,
-                   S->d_chunk_part, S->d_part2, S->d_part3};
+                   S->d_chunk_part, S->d_part2, S->d_part3, S->d_total};
     for (void *q : dev)
         if (q) (void)hipFree(q);
     for (int s = 0; s < NSETS; ++s) {
@@ -528,7 +552,7 @@ int sipg_server_create(sipg_server **out, double hbm_budget_bytes, void *stream)
         (rc = dmalloc(&S->d_ctl, kMaxSlots)) ||
         (rc = dmalloc(&S->d_modes, (size_t)kMaxSlots * 192)) || (rc = dmalloc(&S->d_counts, NSETS * S->NC)) ||
         (rc = dmalloc(&S->d_chunk_part, S->chunk_cap)) || (rc = dmalloc(&S->d_part2, S->chunk_cap)) ||
-        (rc = dmalloc(&S->d_part3, S->chunk_cap)))
+        (rc = dmalloc(&S->d_part3, S->chunk_cap)) || (rc = dmalloc(&S->d_total, 3 * (size_t)kMaxSlots)))
         return fail(rc);
     for (int s = 0; s < NSETS; ++s) {
         if ((rc = dmalloc(&S->d_chunks[s], S->chunk_cap)) || (rc = dmalloc(&S->d_list[s], kMaxSlots)) ||
@@ -790,11 +814,13 @@ int sipg_server_progress(sipg_server *S, int *n_done) {
         if ((rc = upload_set(*S, SET_ACTIVE, S->active))) return rc;
         // The graph stands while it has the degrees running (lists of the
         // others are empty) and their highest, which its launches are sized
-        // for: a new one is 27 launches' capture.
+        // for, and adds up the sums of any request that needs it: a new one is
+        // 27 launches' capture.
         const std::vector<int> deg = degrees_of(*S, S->active), &has = S->graph_degrees;
         if (!deg.empty() && (has.empty() || deg.back() != has.back() ||
                              !std::includes(has.begin(), has.end(), deg.begin(), deg.end())))
             S->graph_stale = true;
+        if (!S->graph_totals && many_items(*S)) S->graph_stale = true;
     }
     if (!S->active.empty()) {
         if (S->graph_stale && (rc = capture_graph(*S, degrees_of(*S, S->active)))) return rc;

@@ -347,21 +347,36 @@ bool batch_prec_supported(int p, double pen, int shape);
 // z = p = M^-1 r over the items of all degrees, with per-item r.r and r.z
 int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq, double *Pv,
                              const batch_inst *inst, double *item_rr, double *item_rz, hipStream_t s);
+// Sums over an instance of per-item shares.  An instance of at most
+// kDirectItems items has them added up by each workgroup that needs the sum;
+// for one with more, where that would grow with the square of its size,
+// launch_batch_totals adds them up once and the others read total[inst].
+// The order of an instance's sum depends on its own items only.
+constexpr int kDirectItems = 512;
+struct item_sum {
+    const double *part;      // per item
+    double *total;           // per instance
+};
+// totals of the listed instances with more than kDirectItems items (b.part
+// null: of a alone); needed before a launch below wherever such an instance
+// is listed
+int launch_batch_totals(const int *list, const int *count, int max_inst, const int2 *item_range, item_sum a,
+                        item_sum b, hipStream_t s);
 // An iteration around the operator's launch, over the lists of all degrees:
 // x += z + alpha p, z = 0 over the chunks of instances whose r is to be
 // replaced, and marks them; AP is to be A x of these before the step
 int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,
-                          int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_part,
+                          int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum pAp,
                           cg_state *states, int slot, hipStream_t s);
 // alpha = r.z / p.Ap, r -= alpha Ap (marked: r = b - Ap), z = M^-1 r
 int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
-                          double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
-                          double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t s);
+                          double *Zq, const batch_inst *inst, const int2 *item_range, item_sum pAp, double *item_rr,
+                          double *item_rz, cg_state *states, int slot, hipStream_t s);
 // beta = r.z(new) / r.z(old), z += alpha p (not where marked), p = zq + beta p;
 // next slot
 int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks, const int *count,
-                            int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_rr,
-                            const double *item_rz, cg_state *states, int slot, hipStream_t s);
+                            int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum rr,
+                            item_sum rz, cg_state *states, int slot, hipStream_t s);
 // x += z; z = 0 over the listed chunks (group update)
 int launch_batch_fold(double *X, double *Z, const batch_chunk *chunks, const int *count, int max_chunks,
                       hipStream_t s);

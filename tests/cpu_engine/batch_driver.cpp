@@ -7,6 +7,7 @@
 
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <vector>
 
 extern "C" int orc_cg(int, int, int, double, const double *, double *, double, int, int, double *);
@@ -82,6 +83,68 @@ static void run(const char *name, const std::vector<int> &dim, const std::vector
     sipg_batch_destroy(B);
 }
 
+namespace sipg_internal {
+int &mock_totals();      // mock_batch.cpp: instances whose items were added up in a launch of their own
+}
+
+// PCG on a batch of long, thin instances about kDirectItems items of four
+// rows, each also solved alone
+static void run_items(const std::vector<int> &dx, const std::vector<int> &dy, const std::vector<int> &p) {
+    auto solve = [&](const std::vector<int> &which, std::vector<std::vector<double>> &out,
+                     std::vector<sipg_cg_info> &info) {
+        std::vector<int> x, y, q;
+        std::vector<double> pen;
+        for (int i : which) {
+            x.push_back(dx[i]);
+            y.push_back(dy[i]);
+            q.push_back(p[i]);
+            pen.push_back(5.0 * (p[i] + 1) * (p[i] + 1));
+        }
+        const int ni = (int)which.size();
+        sipg_batch *B = nullptr;
+        if (sipg_batch_create(&B, ni, x.data(), y.data(), q.data(), pen.data(), nullptr)) std::abort();
+        for (int k : q) sipg_batch_set_shape(B, k, 8, 2);
+        int64_t n = 0;
+        sipg_batch_size(B, &n);
+        void *xd, *bd;
+        sipg_malloc(&xd, n * 8);
+        sipg_malloc(&bd, n * 8);
+        sipg_memset_zero(xd, n * 8);
+        for (int k = 0; k < ni; ++k)
+            sipg_batch_upload(B, k, rhs((int64_t)x[k] * y[k] * (q[k] + 1) * (q[k] + 1), 31 + which[k]).data(), bd);
+        sipg_cg_opts o{1e-10, SIPG_TOL_REL, 0, 1e-2, 1, 0};
+        info.resize(ni);
+        sipg_batch_pcg(B, xd, bd, &o, info.data());
+        out.resize(ni);
+        for (int k = 0; k < ni; ++k) {
+            out[k].resize((size_t)x[k] * y[k] * (q[k] + 1) * (q[k] + 1));
+            sipg_batch_download(B, k, xd, out[k].data());
+        }
+        sipg_free(xd);
+        sipg_free(bd);
+        sipg_batch_destroy(B);
+    };
+    std::vector<int> all;
+    for (int i = 0; i < (int)dx.size(); ++i) all.push_back(i);
+    std::vector<std::vector<double>> mix, one;
+    std::vector<sipg_cg_info> info, info1;
+    solve(all, mix, info);
+    for (int i : all) {
+        sipg_internal::mock_totals() = 0;
+        solve({i}, one, info1);
+        double diff = 0;
+        for (size_t k = 0; k < mix[i].size(); ++k) diff = std::fmax(diff, std::fabs(mix[i][k] - one[0][k]));
+        const std::vector<double> b = rhs((int64_t)mix[i].size(), 31 + i);
+        std::vector<double> Ax(b.size());
+        orc_apply(dx[i], dy[i], p[i], 5.0 * (p[i] + 1) * (p[i] + 1), mix[i].data(), Ax.data());
+        double rr = 0, bb = 0;
+        for (size_t k = 0; k < b.size(); ++k) { rr += (b[k] - Ax[k]) * (b[k] - Ax[k]); bb += b[k] * b[k]; }
+        printf("{\"case\":\"batch_items\",\"inst\":%d,\"status\":%d,\"reps\":%d,\"relres\":%.6e,\"alone_maxdiff\":%.3e,"
+               "\"totals\":%d}\n",
+               i, info[i].status, info[i].replacements, std::sqrt(rr / bb), diff, sipg_internal::mock_totals());
+    }
+}
+
 int main() {
     // asynchronous work runs only when the engine synchronises (the
     // runtime's ordering, with host buffers and graphs read late)
@@ -93,6 +156,7 @@ int main() {
     run("batch_breakdown", {6, 6, 5}, {3, 3, 4}, {80.0, -500.0, 125.0}, 0);
     run("batch_pcg", {6, 4, 5, 3, 7, 4, 2}, {3, 2, 4, 5, 2, 13, 16}, {}, 0, true);
     run("batch_pcg_other_pen", {6, 4}, {3, 2}, {81.0, 45.0}, 0, true);
+    run_items({1, 5, 1, 1}, {2048, 5, 2052, 2100}, {1, 3, 1, 1});
     // nothing may be left queued once every call has returned
     printf("{\"case\":\"deferred_queue\",\"pending\":%zu}\n", mock_pending());
     return 0;

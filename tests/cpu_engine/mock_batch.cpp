@@ -332,11 +332,36 @@ static int prec_tables(const batch_groups &G, std::vector<std::vector<double>> &
     return SIPG_OK;
 }
 
-// sum of part over an instance's range of items
+// the sum over an instance's items
 static double range_sum(const double *part, int2 r) {
     double s = 0.0;
     for (int i = r.x; i < r.y; ++i) s += part[i];
     return s;
+}
+static double instance_sum(item_sum q, const int2 *item_range, int inst) {
+    const int2 r = item_range[inst];
+    return r.y - r.x > kDirectItems ? q.total[inst] : range_sum(q.part, r);
+}
+
+// instances whose items were added up (read and reset by the drivers)
+int &mock_totals() {
+    static int n = 0;
+    return n;
+}
+
+int launch_batch_totals(const int *list, const int *count, int max_inst, const int2 *item_range, item_sum a,
+                        item_sum b, hipStream_t) {
+    mock_run([=]() {
+        if (*count > max_inst) std::abort();
+        for (int k = 0; k < *count; ++k) {
+            const int2 r = item_range[list[k]];
+            if (r.y - r.x <= kDirectItems) continue;
+            a.total[list[k]] = range_sum(a.part, r);
+            if (b.part) b.total[list[k]] = range_sum(b.part, r);
+            ++mock_totals();
+        }
+    });
+    return SIPG_OK;
 }
 
 int launch_batch_prec_groups(const batch_groups &G, int max_items, const double *R, double *Zq, double *Pv,
@@ -366,8 +391,8 @@ int launch_batch_prec_groups(const batch_groups &G, int max_items, const double 
 // alpha, r -= alpha Ap (an instance marked replaced: r = b - Ap), z = M^-1 r;
 // the first item of an instance writes its slot
 int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const double *AP, const double *B,
-                          double *Zq, const batch_inst *inst, const int2 *item_range, const double *item_part,
-                          double *item_rr, double *item_rz, cg_state *states, int slot, hipStream_t) {
+                          double *Zq, const batch_inst *inst, const int2 *item_range, item_sum part, double *item_rr,
+                          double *item_rz, cg_state *states, int slot, hipStream_t) {
     std::vector<std::vector<double>> tab;
     if (const int rc = prec_tables(G, tab)) return rc;
     if (max_items <= 0) return SIPG_OK;
@@ -375,7 +400,7 @@ int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const
         all_items(G, max_items, [&](const batch_group &g, const batch_item &it, int at) {
             cg_state *st = states + it.inst;
             if (finished(st, slot)) return;
-            const double pAp = range_sum(item_part, item_range[it.inst]);
+            const double pAp = instance_sum(part, item_range, it.inst);
             const double alpha = st->s[slot].rz / pAp;
             const bool replaced = st->s[slot].flags & kSlotReplaced;
             if (at == item_range[it.inst].x) {
@@ -402,7 +427,7 @@ int launch_batch_pcg_step(const batch_groups &G, int max_items, double *R, const
 }
 
 int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_chunk *chunks, const int *count,
-                          int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_part,
+                          int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum part,
                           cg_state *states, int slot, hipStream_t) {
     mock_run([=]() {
         if (*count > max_chunks) std::abort();
@@ -410,7 +435,7 @@ int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_ch
             const batch_chunk c = chunks[k];
             cg_state *st = states + c.inst;
             if (finished(st, slot)) continue;
-            const double pAp = range_sum(item_part, item_range[c.inst]);
+            const double pAp = instance_sum(part, item_range, c.inst);
             const double alpha = st->s[slot].rz / pAp;
             if (!(pAp > 0.0) || !std::isfinite(alpha)) continue;
             if (k == chunk_range[c.inst].x) {
@@ -427,8 +452,8 @@ int launch_batch_pcg_fold(double *X, double *Z, const double *Pv, const batch_ch
 }
 
 int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch_chunk *chunks, const int *count,
-                            int max_chunks, const int2 *chunk_range, const int2 *item_range, const double *item_rr,
-                            const double *item_rz, cg_state *states, int slot, hipStream_t) {
+                            int max_chunks, const int2 *chunk_range, const int2 *item_range, item_sum item_rr,
+                            item_sum item_rz, cg_state *states, int slot, hipStream_t) {
     mock_run([=]() {
         if (*count > max_chunks) std::abort();
         for (int k = 0; k < *count; ++k) {
@@ -444,7 +469,7 @@ int launch_batch_pcg_update(double *Z, double *Pv, const double *Zq, const batch
                 }
                 continue;
             }
-            const double rr = range_sum(item_rr, item_range[c.inst]), rz = range_sum(item_rz, item_range[c.inst]);
+            const double rr = instance_sum(item_rr, item_range, c.inst), rz = instance_sum(item_rz, item_range, c.inst);
             const bool replaced = (cur.flags & kSlotReplaced) != 0;
             const double beta = rz / cur.rz;
             if (lead) {

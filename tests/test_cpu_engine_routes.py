@@ -1,7 +1,9 @@
 """The sanitised drivers run the host paths that the library has: every
 launcher that the host sources call is defined in them, as it is in the
-library, so none is chosen by whether it exists.  And the chunks of
-iterations that small CG solves run in one launch keep the solver's rules."""
+library, so none is chosen by whether it exists.  The chunks of iterations
+that small CG solves run in one launch keep the solver's rules, and batched
+PCG gives the same solution alone and in a batch on either side of the item
+count above which an instance's sums are added up in launches of their own."""
 import os
 import shutil
 import subprocess
@@ -9,7 +11,7 @@ import subprocess
 import pytest
 
 from conftest import PKG
-from test_cpu_engine import ENG, results  # noqa: F401  (the engine driver's cases)
+from test_cpu_engine import ENG, batch_results, results  # noqa: F401  (the drivers' cases)
 
 
 def _undefined_weak(path, *flags):
@@ -60,3 +62,11 @@ def test_small_mixed_cycles(results):  # noqa: F811
 def test_small_cg_breakdown(results):  # noqa: F811
     r = results["small_breakdown"]
     assert r["rc"] == 8 and r["chunks"] > 0, r
+
+
+def test_batched_pcg_about_the_item_limit(batch_results):  # noqa: F811
+    # 512, 9 (of degree 3), 513 and 525 items
+    rows = batch_results["batch_items"]
+    for r in rows:
+        assert r["status"] == 0 and r["relres"] <= 1e-10 and r["reps"] >= 1 and r["alone_maxdiff"] == 0.0, r
+    assert [r["totals"] > 0 for r in rows] == [False, False, True, True], rows
