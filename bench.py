@@ -24,7 +24,7 @@ import numpy as np  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 DIM, P = 256, 8
 TOL = 1e-10
-FLOOR = 4 * TOL                      # where an FP64 solve that ends at its floor may be
+FLOOR = 4 * TOL                      # where a solve that may end at the FP64 floor may be
 # Iteration caps: the FP64 solve needs about 4.7k iterations here and the
 # mixed one about 40k FP32 iterations; a solve that hits its cap fails
 # loudly instead of running to the default cap of n iterations.
@@ -50,11 +50,13 @@ SOLVERS = {
 }
 
 
-def gpu_solve(sipg, op, b, x, method, rf2=1e-2):
+def gpu_solve(sipg, op, b, x, method, rf2=1e-2, floor_ok=False):
     """One solve from x = 0 to a 1e-10 true relative residual; method is
     "fp64" (CG), "pcg" (block-Jacobi PCG), "pcg2" (two-level PCG, a true
     residual every time the recursive one has fallen by the factor rf2) or
-    "mixed"."""
+    "mixed".  A solve that does not get there raises; with floor_ok, CG and
+    block-Jacobi PCG may end at the FP64 floor of b - A x instead, short of
+    their iteration cap."""
     x.zero()
     sipg.synchronize()
     t0 = time.perf_counter()
@@ -80,12 +82,15 @@ def gpu_solve(sipg, op, b, x, method, rf2=1e-2):
         st, info = op.cg_ex(x, b, TOL, sipg.TOL_REL, maxit=MAXIT_FP64, replace_factor=3e-3,
                             true_stop=True, restart=0)
     t1 = time.perf_counter()
-    # CG and block-Jacobi PCG may end at the FP64 floor of b - A x, which
-    # scatters about the tolerance here (of 24 forcings block-Jacobi PCG ends
-    # above it on 8, with any operator kernel); their legs then say so
-    if st != sipg.OK and not (st == sipg.NOT_CONVERGED and method in ("fp64", "pcg")):
-        raise RuntimeError(f"{method} solve failed: {sipg.strerror(st)}")
+    at_floor = st == sipg.NOT_CONVERGED and method in ("fp64", "pcg") and info.iters < MAXIT_FP64
+    if st != sipg.OK and not (floor_ok and at_floor):
+        raise RuntimeError(f"{method} solve failed: {sipg.strerror(st)} after {info.iters} iterations")
     return t1 - t0, info
+
+
+def time_ratio(ms, vs):
+    """ms / vs, or None where either solve (None) did not reach its tolerance."""
+    return None if ms is None or vs is None else ms / vs
 
 
 def _cpu_model():
@@ -278,7 +283,10 @@ def c1_leg(sipg):
         t, info = gpu_solve(sipg, op, b, x, method)
         t, info = gpu_solve(sipg, op, b, x, method)
         xh = op.download(x)
-        out[method] = {"ms_per_solve": 1e3 * t, "iterations": info.iters, "true_relres": op.true_relres(x, b),
+        relres = op.true_relres(x, b)
+        if not relres <= TOL:
+            raise RuntimeError(f"c1 {method}: true relative residual {relres:.3e} above {TOL}")
+        out[method] = {"ms_per_solve": 1e3 * t, "iterations": info.iters, "true_relres": relres,
                        "rel_l2_vs_lapack": float(np.linalg.norm(xh - u) / np.linalg.norm(u)),
                        "rel_max_vs_lapack": float(np.max(np.abs(xh - u)) / np.max(np.abs(u)))}
     log(f"c1: CG {out['fp64']['iterations']} it, rel L2 vs LAPACK {out['fp64']['rel_l2_vs_lapack']:.2e}; "
@@ -678,40 +686,46 @@ def main():
     log(f"apply: {ms_apply * 1e3:.2f} us/launch, {apply_gbs:.0f} GB/s algorithmic")
 
     # ---- plain FP64 solver (the comparison line) -------------------------
+    # CG and block-Jacobi PCG may end at the FP64 floor of b - A x, which
+    # scatters about the tolerance here (of 24 forcings block-Jacobi PCG ends
+    # above it on 8, with any operator kernel).  Their legs then say so, and
+    # no ratio is formed with them.
     x64 = op.vector()
-    gpu_solve(sipg, op, b, x64, "fp64")                           # warm-up
+    gpu_solve(sipg, op, b, x64, "fp64", floor_ok=True)            # warm-up
     t64, it64 = [], []
     for _ in range(args.steps):
-        t, info = gpu_solve(sipg, op, b, x64, "fp64")
+        t, info = gpu_solve(sipg, op, b, x64, "fp64", floor_ok=True)
         t64.append(t)
         it64.append(info.iters)
     rel64 = op.true_relres(x64, b)
     if not rel64 <= FLOOR:
         raise RuntimeError(f"FP64 true relative residual {rel64:.3e} above {FLOOR}")
     ms64 = 1e3 * float(np.median(t64))
+    vs64 = ms64 if rel64 <= TOL else None
     log(f"fp64 : {ms64:.1f} ms/solve, {it64[-1]} iterations, {info.replacements} replacements, "
         f"{1e3 * ms64 / it64[-1]:.1f} us/iter, true relres {rel64:.2e}")
 
     # ---- block-Jacobi PCG (FP64) -------------------------------------------
     xp = op.vector()
-    gpu_solve(sipg, op, b, xp, "pcg")                             # warm-up
+    gpu_solve(sipg, op, b, xp, "pcg", floor_ok=True)              # warm-up
     tp, itp = [], []
     for _ in range(args.steps):
-        t, infop = gpu_solve(sipg, op, b, xp, "pcg")
+        t, infop = gpu_solve(sipg, op, b, xp, "pcg", floor_ok=True)
         tp.append(t)
         itp.append(infop.iters)
     relp = op.true_relres(xp, b)
     if not relp <= FLOOR:
         raise RuntimeError(f"PCG true relative residual {relp:.3e} above {FLOOR}")
     msp = 1e3 * float(np.median(tp))
+    vsp = msp if relp <= TOL else None
     xp_h, x64_h = op.download(xp), op.download(x64)
     pcg = {"dof_per_s": n / (msp * 1e-3), "ms_per_solve": msp, "iterations": itp[-1],
            "replacements": infop.replacements, "true_relres": relp, "converged": relp <= TOL,
            "us_per_iteration": 1e3 * msp / itp[-1],
            "rel_l2_vs_cg_solution": float(np.linalg.norm(xp_h - x64_h) / np.linalg.norm(x64_h)),
-           "time_vs_cg": msp / ms64}
+           "time_vs_cg": time_ratio(vsp, vs64)}
     log(f"pcg  : {msp:.1f} ms/solve, {itp[-1]} iterations, {infop.replacements} replacements, "
-        f"{pcg['us_per_iteration']:.1f} us/iter, true relres {relp:.2e}, time vs CG {pcg['time_vs_cg']:.2f}")
+        f"{pcg['us_per_iteration']:.1f} us/iter, true relres {relp:.2e}, time vs CG {pcg['time_vs_cg']}")
 
     # ---- two-level PCG (FP64) ---------------------------------------------
     x2 = op.vector()
@@ -729,10 +743,10 @@ def main():
             "replacements": info2.replacements, "true_relres": rel2,
             "us_per_iteration": 1e3 * ms2 / it2[-1],
             "rel_l2_vs_cg_solution": float(np.linalg.norm(op.download(x2) - x64_h) / np.linalg.norm(x64_h)),
-            "time_vs_cg": ms2 / ms64, "time_vs_pcg": ms2 / msp}
+            "time_vs_cg": time_ratio(ms2, vs64), "time_vs_pcg": time_ratio(ms2, vsp)}
     log(f"pcg2 : {ms2:.1f} ms/solve, {it2[-1]} iterations, {info2.replacements} replacements, "
-        f"{pcg2['us_per_iteration']:.1f} us/iter, true relres {rel2:.2e}, time vs CG {pcg2['time_vs_cg']:.3f}, "
-        f"vs PCG {pcg2['time_vs_pcg']:.3f}")
+        f"{pcg2['us_per_iteration']:.1f} us/iter, true relres {rel2:.2e}, time vs CG {pcg2['time_vs_cg']}, "
+        f"vs PCG {pcg2['time_vs_pcg']}")
 
     # ---- mixed-precision solver -------------------------------------------
     # time_vs_fp64 is like for like: the mixed solver runs two-level PCG
@@ -762,11 +776,11 @@ def main():
                  "error_vs_exact": {k: float(v) for k, v in op.err_norms_fourier(modes, xm).items()},
                  "time_vs_fp64": tm / (ms2 * 1e-3),
                  "time_vs_fp64_note": "mixed two-level PCG / FP64 two-level PCG (same algorithm)",
-                 "time_vs_fp64_plain_cg": tm / (ms64 * 1e-3), "time_vs_fp64_pcg": tm / (msp * 1e-3)}
+                 "time_vs_fp64_plain_cg": time_ratio(1e3 * tm, vs64), "time_vs_fp64_pcg": time_ratio(1e3 * tm, vsp)}
         log(f"mixed: {1e3 * tm:.1f} ms/solve, {infom.iters} FP32 iterations, "
             f"{infom.replacements} refinement cycles, true relres {relm:.2e}, "
             f"time ratio vs FP64 two-level PCG {mixed['time_vs_fp64']:.2f} (vs FP64 CG "
-            f"{mixed['time_vs_fp64_plain_cg']:.3f}, vs FP64 PCG {mixed['time_vs_fp64_pcg']:.2f})")
+            f"{mixed['time_vs_fp64_plain_cg']}, vs FP64 PCG {mixed['time_vs_fp64_pcg']})")
     except RuntimeError as exc:
         mixed = {"status": f"failed: {exc}"}
         log(f"mixed: {exc}")
