@@ -29,8 +29,10 @@ __device__ __forceinline__ int opaque(int v) {
 }
 
 // first[g] = items of the groups before g; returns the number of all items.
-// One barrier; first stays valid to the kernel's end.
+// One barrier, and none for a single group, whose first is not stored; first
+// stays valid to the kernel's end.
 __device__ __forceinline__ int batch_offsets(const batch_groups &G, int (&first)[kMaxDegree + 1]) {
+    if (G.n == 1) return *G.g[0].count;
     if (threadIdx.x < 64) {
         const int l = threadIdx.x;
         int c = 0;
@@ -49,11 +51,16 @@ __device__ __forceinline__ int batch_offsets(const batch_groups &G, int (&first)
     return __builtin_amdgcn_readfirstlane(first[G.n]);
 }
 
-// the group of item k, uniform over the wave
-__device__ __forceinline__ int batch_group_at(const batch_groups &G, const int (&first)[kMaxDegree + 1], int k) {
+// the group of item k, uniform over the wave, and the item's place in it
+__device__ __forceinline__ int batch_group_at(const batch_groups &G, const int (&first)[kMaxDegree + 1], int k,
+                                              int &at) {
+    at = k;
+    if (G.n == 1) return 0;
     const int l = threadIdx.x & 63;
     const bool in = l >= 1 && l < G.n && k >= first[min(l, kMaxDegree)];
-    return __builtin_amdgcn_readfirstlane(__popcll(__ballot(in)));
+    const int g = __builtin_amdgcn_readfirstlane(__popcll(__ballot(in)));
+    at = k - __builtin_amdgcn_readfirstlane(first[g]);
+    return g;
 }
 
 }  // namespace sipg_internal

@@ -55,8 +55,8 @@ void batch_apply_kernel(batch_groups G, const double *__restrict__ X, double *__
     __shared__ int first[kMaxDegree + 1];
     const int n = batch_offsets(G, first);
     for (int k = xcd_remap(blockIdx.x, gridDim.x); k < n; k += gridDim.x) {
-        const int g = batch_group_at(G, first, k);
-        const int i = k - __builtin_amdgcn_readfirstlane(first[g]);
+        int i;
+        const int g = batch_group_at(G, first, k, i);
         const batch_item it = G.g[g].items[i];
         if (DOT) {
             const cg_state *st = states + it.inst;

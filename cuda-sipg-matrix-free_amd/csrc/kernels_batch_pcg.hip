@@ -116,8 +116,8 @@ void batch_prec_kernel(batch_groups G, int tiles, double *R, const double *__res
         });
     __syncthreads();
     for (int k = xcd_remap(blockIdx.x, gridDim.x); k < n; k += gridDim.x) {
-        const int g = batch_group_at(G, first, k);
-        const int i = k - __builtin_amdgcn_readfirstlane(first[g]);
+        int i;
+        const int g = batch_group_at(G, first, k, i);
         const batch_item it = G.g[g].items[i];
         cg_state *st = states + it.inst;
         if (STEP && (st->s[slot].done | st->err)) continue;     // uniform over the workgroup

@@ -37,6 +37,22 @@ def test_batch_on_either_side_of_the_limit(sipg):
         assert np.array_equal(_solve(sipg, dims, ps, bs, [i])[0], got[i]), (d, p)
 
 
+@pytest.mark.parametrize("p", [3, 12])
+def test_batch_of_one_degree_with_more_items_than_workgroups(sipg, p):
+    # one list only: 6 items to an instance (2 strips, 3 bands)
+    d = (64 // (p + 1) + 1, 9)
+    x0 = np.random.default_rng(p).uniform(-1, 1, d[0] * d[1] * (p + 1) ** 2)
+    B = sipg.Batch([d[0]] * 700, [d[1]] * 700, [p] * 700, [sipg.pen_sigma(p)] * 700)
+    assert B.set_shape(p, 8, 2) == sipg.OK
+    x, y = B.vector(), B.vector()
+    for i in range(700):
+        B.upload(i, x0 * (1 + i % 3), x)
+    assert B.apply(x, y) == sipg.OK
+    op = sipg.Operator(d[0], d[1], p, sipg.pen_sigma(p), sipg.F64)
+    want = [op.apply_host(x0 * (1 + k)) for k in range(3)]
+    assert all(np.array_equal(B.download(i, y), want[i % 3]) for i in range(700))
+
+
 def test_server_takes_a_large_request_among_small_ones(sipg):
     # 300 x 300 of degree 2: 570 items, after the iterations were captured
     # for small requests of the same degrees
