@@ -93,6 +93,10 @@ def time_ratio(ms, vs):
     return None if ms is None or vs is None else ms / vs
 
 
+def ratio_text(r):
+    return "not formed" if r is None else f"{r:.3f}"
+
+
 def _cpu_model():
     try:
         with open("/proc/cpuinfo") as fh:
@@ -725,7 +729,7 @@ def main():
            "rel_l2_vs_cg_solution": float(np.linalg.norm(xp_h - x64_h) / np.linalg.norm(x64_h)),
            "time_vs_cg": time_ratio(vsp, vs64)}
     log(f"pcg  : {msp:.1f} ms/solve, {itp[-1]} iterations, {infop.replacements} replacements, "
-        f"{pcg['us_per_iteration']:.1f} us/iter, true relres {relp:.2e}, time vs CG {pcg['time_vs_cg']}")
+        f"{pcg['us_per_iteration']:.1f} us/iter, true relres {relp:.2e}, time vs CG {ratio_text(pcg['time_vs_cg'])}")
 
     # ---- two-level PCG (FP64) ---------------------------------------------
     x2 = op.vector()
@@ -745,8 +749,8 @@ def main():
             "rel_l2_vs_cg_solution": float(np.linalg.norm(op.download(x2) - x64_h) / np.linalg.norm(x64_h)),
             "time_vs_cg": time_ratio(ms2, vs64), "time_vs_pcg": time_ratio(ms2, vsp)}
     log(f"pcg2 : {ms2:.1f} ms/solve, {it2[-1]} iterations, {info2.replacements} replacements, "
-        f"{pcg2['us_per_iteration']:.1f} us/iter, true relres {rel2:.2e}, time vs CG {pcg2['time_vs_cg']}, "
-        f"vs PCG {pcg2['time_vs_pcg']}")
+        f"{pcg2['us_per_iteration']:.1f} us/iter, true relres {rel2:.2e}, time vs CG {ratio_text(pcg2['time_vs_cg'])}, "
+        f"vs PCG {ratio_text(pcg2['time_vs_pcg'])}")
 
     # ---- mixed-precision solver -------------------------------------------
     # time_vs_fp64 is like for like: the mixed solver runs two-level PCG
@@ -780,7 +784,7 @@ def main():
         log(f"mixed: {1e3 * tm:.1f} ms/solve, {infom.iters} FP32 iterations, "
             f"{infom.replacements} refinement cycles, true relres {relm:.2e}, "
             f"time ratio vs FP64 two-level PCG {mixed['time_vs_fp64']:.2f} (vs FP64 CG "
-            f"{mixed['time_vs_fp64_plain_cg']}, vs FP64 PCG {mixed['time_vs_fp64_pcg']})")
+            f"{ratio_text(mixed['time_vs_fp64_plain_cg'])}, vs FP64 PCG {ratio_text(mixed['time_vs_fp64_pcg'])})")
     except RuntimeError as exc:
         mixed = {"status": f"failed: {exc}"}
         log(f"mixed: {exc}")
@@ -869,7 +873,7 @@ def main():
             "frac": apply_gbs / HBM_PEAK_GBS,
             "traffic": traffic,
             "traffic_note": traffic_note,
-            "kernel": "apply_kernel_wave<double,8,4,false,CxCoef<double,8>> (fused volume + flux_term6a + "
+            "kernel": "apply_kernel_wave<double,8,4,false> (fused volume + flux_term6a + "
                       "flux_term6b; a wave owns 7 whole elements of a 7x4-element block, the block and its "
                       "halo staged into LDS by direct global->LDS loads, two workgroup barriers per block)",
             "algorithmic_bytes_per_launch": apply_bytes,

@@ -60,14 +60,13 @@ struct BlockGeo {
     static constexpr int LDS = NS * TS;                 // elements of T
 };
 
-// Direct global -> LDS staging (global_load_lds_dword): used where the LDS
-// image of a block is the concatenation of its row runs and halo-column
-// tiles (no row padding, TS == NQ) and two images fit in LDS, so the next
-// block streams in while the current one is computed.
+// Direct global -> LDS staging (global_load_lds_dword) takes a block whose
+// LDS image is the concatenation of its row runs and halo-column tiles: no
+// row padding, TS == NQ, and whole waves to issue it.
 template <typename T, int P, int BX, int BY>
 struct BlockDma {
     using G = BlockGeo<T, P, BX, BY>;
-    static constexpr bool ok = G::TS == G::NQ && G::NT >= 64 && 2 * G::LDS * sizeof(T) <= 160 * 1024;
+    static constexpr bool ok = G::TS == G::NQ && G::NT >= 64;
 };
 
 typedef __attribute__((address_space(3))) unsigned lds_dword;

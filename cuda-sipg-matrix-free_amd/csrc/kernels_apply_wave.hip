@@ -26,7 +26,7 @@
 
 namespace sipg_internal {
 
-template <typename T, int P, int BY, bool DOT, class C>
+template <typename T, int P, int BY, bool DOT>
 __global__ __launch_bounds__(64 * BY)
 void apply_kernel_wave(const T *__restrict__ x, T *__restrict__ y, int dimx, int dimy, int nbx, int nblk, T pen,
                        double *__restrict__ partials, const cg_state *__restrict__ st, int slot)
@@ -44,7 +44,7 @@ void apply_kernel_wave(const T *__restrict__ x, T *__restrict__ y, int dimx, int
     const int x0 = (b % nbx) * BX, y0 = (b / nbx) * BY;
     block_issue<T, P, BX, BY, BY>(lds, x, dimx, dimy, x0, y0);      // every wave issues
 
-    const C coef{};
+    const CxCoef<T, P> coef{};
     const int lane = threadIdx.x & 63;
     const int ey = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int s = lane / N1, j = lane - s * N1;
@@ -160,31 +160,26 @@ void apply_kernel_wave(const T *__restrict__ x, T *__restrict__ y, int dimx, int
 
 namespace {
 
-// Rows of elements per workgroup (waves), one LDS image of (BY + 2) * BX +
-// 2 BY tiles per workgroup, and where the coefficients come from.
-// Measured at 256 x 256 and 1024 x 1024, p = 8, FP64 (us per apply):
-// BY = 2: 22.2 / 281, 3: 21.7 / 277, 4: 21.1 / 277, 6: 24.3 / 301,
-// 8: 22.8 / 297, 10: 26.9 / 374.
-template <typename T, int P>
-struct WaveShape {
-    static constexpr int BY = 4;
-    using Coef = CxCoef<T, P>;
-};
+// Rows of elements per workgroup (waves), with one LDS image of (rows + 2) *
+// BX + 2 rows tiles.  Measured at 256 x 256 and 1024 x 1024, p = 8, FP64, before
+// a run's loads were issued ahead of its use (us per apply): 2: 22.2 / 281,
+// 3: 21.7 / 277, 4: 21.1 / 277, 6: 24.3 / 301, 8: 22.8 / 297, 10: 26.9 / 374.
+constexpr int kRows = 4;
 
 template <typename T, int P, bool DOT>
 void launch_wave(const void *x, void *y, int dimx, int dimy, double pen, double *partials, const cg_state *st,
                  int slot, hipStream_t s)
 {
-    constexpr int BX = 64 / (P + 1), BY = WaveShape<T, P>::BY;
+    constexpr int BX = 64 / (P + 1), BY = kRows;
     const int nbx = (dimx + BX - 1) / BX, nby = (dimy + BY - 1) / BY;
     const int nblk = nbx * nby;
-    hipLaunchKernelGGL((apply_kernel_wave<T, P, BY, DOT, typename WaveShape<T, P>::Coef>), dim3(nblk),
-                       dim3(64 * BY), 0, s, (const T *)x, (T *)y, dimx, dimy, nbx, nblk, (T)pen, partials, st, slot);
+    hipLaunchKernelGGL((apply_kernel_wave<T, P, BY, DOT>), dim3(nblk), dim3(64 * BY), 0, s, (const T *)x, (T *)y, dimx,
+                       dimy, nbx, nblk, (T)pen, partials, st, slot);
 }
 
 template <typename T, int P>
 int wave_blocks(int dimx, int dimy) {
-    constexpr int BX = 64 / (P + 1), BY = WaveShape<T, P>::BY;
+    constexpr int BX = 64 / (P + 1), BY = kRows;
     return ((dimx + BX - 1) / BX) * ((dimy + BY - 1) / BY);
 }
 

@@ -604,10 +604,9 @@ int launch_coarse_add(int dtype, int p, void *v, int dimx, int64_t n, const coar
     return dispatch_p<1>(p, dtype, 1, a);
 }
 
-int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_pAp,
-                         int np_pAp, const double *part_rr, const double *part_rz, int np, int npc, int dimx,
-                         const coarse_tables &c, int nblk, cg_state *st, int slot, hipStream_t s, void *xlo) {
-    (void)part_pAp, (void)np_pAp, (void)nblk;           // alpha: recorded in the slot by launch_pcg_rz
+int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_rr,
+                         const double *part_rz, int np, int npc, int dimx, const coarse_tables &c, cg_state *st,
+                         int slot, hipStream_t s, void *xlo) {
     coarse_args a{};
     a.x = x;
     a.xlo = xlo;

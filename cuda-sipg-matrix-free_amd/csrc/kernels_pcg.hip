@@ -448,10 +448,8 @@ int launch_pcg_rz(int dtype, int p, double pen, int mode, void *r, const void *A
                                      part_rz, st, slot, E4, s);
 }
 
-int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_pAp,
-                        int np_pAp, const double *part_rr, const double *part_rz, int np, int nblk,
-                        cg_state *st, int slot, hipStream_t s, void *xlo) {
-    (void)part_pAp, (void)np_pAp;                       // alpha: recorded in the slot by launch_pcg_rz
+int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_rr,
+                        const double *part_rz, int np, int nblk, cg_state *st, int slot, hipStream_t s, void *xlo) {
     if (dtype == SIPG_F64)
         hipLaunchKernelGGL(pcg_update_p_kernel<double>, dim3(nblk), dim3(VT), 0, s, (double *)x, (double *)p,
                            (const double *)z, n, part_rr, part_rz, np, st, slot, (double *)xlo);

@@ -138,7 +138,7 @@ struct batch_ctl {
     double tol;
     int tol_mode, maxit;
 };
-// A block of an instance for the operator kernel: `rows` mesh rows from
+// A strip of an instance for the operator kernel: `rows` mesh rows from
 // (x0, y0), as wide as the kernel takes them.
 struct batch_item {
     int inst, x0, y0, rows;
@@ -159,8 +159,9 @@ struct batch_chunk {
     int inst, pad;
     int64_t begin, end;
 };
-// Candidate block shapes of the batched operator (the autotuner picks one
-// per degree), named 16x4, 8x4 and 8x2.
+// Candidate item shapes of the batched operator (the autotuner picks one
+// per degree).  BX x BY are their names in the interface, 16x4, 8x4 and 8x2;
+// batch_item_extent says what they cover.
 constexpr int kBatchShapes = 3;
 extern const int kBatchShapeBX[kBatchShapes];
 extern const int kBatchShapeBY[kBatchShapes];
@@ -177,7 +178,7 @@ constexpr int kVecThreads = 256;
 
 // ---- launchers (kernels_apply.hip, kernels_mfma.hip) ----------------------
 // The contraction kernel an apply of (dtype, p) runs for a requested
-// SIPG_KERNEL_* setting: SIPG_KERNEL_VALU or SIPG_KERNEL_MFMA.
+// SIPG_KERNEL_* setting: SIPG_KERNEL_VALU, _MFMA or _WAVE.
 int resolve_kernel(int dtype, int p, int kernel);
 // Number of thread blocks the fused apply uses for a mesh (= partial count).
 int apply_num_blocks(int dtype, int p, int dimx, int dimy, int kernel = SIPG_KERNEL_AUTO);
@@ -186,7 +187,7 @@ int apply_num_blocks(int dtype, int p, int dimx, int dimy, int kernel = SIPG_KER
 int launch_apply(int dtype, int p, const void *x, void *y, const void *tab, int dimx, int dimy,
                  double pen, double *partials, const cg_state *st, int slot, hipStream_t s,
                  int kernel = SIPG_KERNEL_AUTO);
-// the vector-ALU apply with wave-owned elements (kernels_apply_wave.hip)
+// the vector-ALU apply on blocks staged in LDS (kernels_apply_wave.hip)
 bool wave_apply_available(int dtype, int p);
 int wave_apply_num_blocks(int dtype, int p, int dimx, int dimy);
 int launch_apply_wave(int dtype, int p, const void *x, void *y, int dimx, int dimy, double pen, double *partials,
@@ -264,11 +265,11 @@ bool pcg_rz_fuses_restrict(int dtype, int p, double pen);
 int launch_pcg_rz(int dtype, int p, double pen, int mode, void *r, const void *Ap, void *z, void *pcopy,
                   int64_t noe, const void *prec, const double *part_pAp, int np_pAp, double *part_rr,
                   double *part_rz, cg_state *st, int slot, hipStream_t s, double *E4 = nullptr);
-// p = z + beta p (and x += alpha p unless r was replaced this iteration);
-// writes the next slot
-int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_pAp,
-                        int np_pAp, const double *part_rr, const double *part_rz, int np, int nblk,
-                        cg_state *st, int slot, hipStream_t s, void *xlo = nullptr);
+// p = z + beta p (and x += alpha p, alpha as launch_pcg_rz recorded it, unless
+// r was replaced this iteration); writes the next slot
+int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_rr,
+                        const double *part_rz, int np, int nblk, cg_state *st, int slot, hipStream_t s,
+                        void *xlo = nullptr);
 // x += alpha p, before a true residual replaces r in the same iteration
 int launch_pcg_x(int dtype, void *x, const void *p, int64_t n, const double *part_pAp, int np_pAp, int nblk,
                  const cg_state *st, int slot, hipStream_t s, void *xlo = nullptr);
@@ -296,9 +297,9 @@ int launch_coarse_solve(int dtype, int p, const void *r, int dimx, int dimy, con
 int launch_coarse_add(int dtype, int p, void *v, int dimx, int64_t n, const coarse_tables &c, int nblk,
                       hipStream_t s);
 // the PCG p update with the coarse level (r.z gains S.C, p gains P0^T C)
-int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_pAp,
-                         int np_pAp, const double *part_rr, const double *part_rz, int np, int npc, int dimx,
-                         const coarse_tables &c, int nblk, cg_state *st, int slot, hipStream_t s, void *xlo = nullptr);
+int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_rr,
+                         const double *part_rz, int np, int npc, int dimx, const coarse_tables &c, cg_state *st,
+                         int slot, hipStream_t s, void *xlo = nullptr);
 // host tables of the coarse solve: Q (n x n, n = dim - 1), and the 1-D
 // eigenvalues of K and of the GLL-quadrature Q1 mass
 void coarse_dst(int dim, std::vector<double> &Q, std::vector<double> &lamK, std::vector<double> &lamM, int p);

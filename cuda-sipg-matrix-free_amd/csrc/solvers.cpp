@@ -159,10 +159,10 @@ struct Engine {
             if ((rc = launch_mark_replaced(st, slot, restart_p ? 1 : 0, s))) return rc;
         }
         if (coarse)
-            rc = launch_pcg2_update_p(opI->dtype, opI->p, xI, p, z, opI->n, src, np, P.rr, P.rz, nrz, ncp, opI->dimx,
-                                      *coarse, nb, st, slot, s, xLu);
+            rc = launch_pcg2_update_p(opI->dtype, opI->p, xI, p, z, opI->n, P.rr, P.rz, nrz, ncp, opI->dimx, *coarse,
+                                      st, slot, s, xLu);
         else
-            rc = launch_pcg_update_p(opI->dtype, xI, p, z, opI->n, src, np, P.rr, P.rz, nrz, nb, st, slot, s, xLu);
+            rc = launch_pcg_update_p(opI->dtype, xI, p, z, opI->n, P.rr, P.rz, nrz, nb, st, slot, s, xLu);
         if (rc) return rc;
         ++launched;
         return SIPG_OK;

@@ -497,6 +497,7 @@ static void pcg_rz_t(int p, int mode, T *r, const T *Ap, T *z, T *pcopy, int64_t
         const double pAp = sum_partials(ppAp, np);
         const double a = st->s[slot].rz / pAp;
         if (!(pAp > 0.0) || !std::isfinite(a)) { st->err = std::isfinite(pAp) ? 2 : 3; return; }
+        st->s[slot].alpha = a;                       // for the p update
         const int64_t n = noe * (p + 1) * (p + 1);
         for (int64_t i = 0; i < n; ++i) r[i] = r[i] - (T)a * Ap[i];
     }
@@ -555,12 +556,11 @@ int launch_pcg_rz(int dtype, int p, double, int mode, void *r, const void *Ap, v
 }
 
 template <typename T>
-static void pcg_update_p_t(T *x, T *p, const T *z, int64_t n, const double *ppAp, int np_pAp,
-                           const double *prr, const double *prz, int np, cg_state *st, int slot, T *xlo) {
+static void pcg_update_p_t(T *x, T *p, const T *z, int64_t n, const double *prr, const double *prz, int np,
+                           cg_state *st, int slot, T *xlo) {
     const cg_slot cur = st->s[slot];
     if (cur.done | st->err) { st->s[slot ^ 1] = cur; return; }
     const double rr_new = sum_partials(prr, np), rz_new = sum_partials(prz, np);
-    const double pAp = sum_partials(ppAp, np_pAp);
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
     const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rz_new / cur.rz;
     const bool met = !(std::sqrt(rr_new) > st->stop);
@@ -577,7 +577,7 @@ static void pcg_update_p_t(T *x, T *p, const T *z, int64_t n, const double *ppAp
     if (replaced) st->rr_ref = rr_new;
     if (!std::isfinite(rr_new) || !std::isfinite(rz_new)) st->err = 3;
     else if (!(rz_new > 0.0) && rr_new > 0.0) st->err = 2;
-    const T a = (T)(cur.rz / pAp), b = (T)beta_d;
+    const T a = (T)cur.alpha, b = (T)beta_d;
     for (int64_t i = 0; i < n; ++i) {
         const T pi = p[i];
         if (!replaced) {
@@ -588,16 +588,15 @@ static void pcg_update_p_t(T *x, T *p, const T *z, int64_t n, const double *ppAp
     }
 }
 
-int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_pAp,
-                        int np_pAp, const double *part_rr, const double *part_rz, int np, int, cg_state *st,
-                        int slot, hipStream_t, void *xlo) {
+int launch_pcg_update_p(int dtype, void *x, void *p, const void *z, int64_t n, const double *part_rr,
+                        const double *part_rz, int np, int, cg_state *st, int slot, hipStream_t, void *xlo) {
     ++mock_p_updates();
     if (dtype == SIPG_F64)
-        pcg_update_p_t<double>(tp<double>(x), tp<double>(p), tp<double>(z), n, part_pAp, np_pAp, part_rr, part_rz,
-                               np, st, slot, tp<double>(xlo));
+        pcg_update_p_t<double>(tp<double>(x), tp<double>(p), tp<double>(z), n, part_rr, part_rz, np, st, slot,
+                               tp<double>(xlo));
     else
-        pcg_update_p_t<float>(tp<float>(x), tp<float>(p), tp<float>(z), n, part_pAp, np_pAp, part_rr, part_rz, np,
-                              st, slot, tp<float>(xlo));
+        pcg_update_p_t<float>(tp<float>(x), tp<float>(p), tp<float>(z), n, part_rr, part_rz, np, st, slot,
+                              tp<float>(xlo));
     return SIPG_OK;
 }
 
@@ -675,9 +674,9 @@ int launch_coarse_add(int dtype, int p, void *v, int dimx, int64_t n, const coar
     return SIPG_OK;
 }
 
-int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_pAp,
-                         int np_pAp, const double *part_rr, const double *part_rz, int np, int npc, int dimx,
-                         const coarse_tables &c, int, cg_state *st, int slot, hipStream_t, void *xlo) {
+int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int64_t n, const double *part_rr,
+                         const double *part_rz, int np, int npc, int dimx, const coarse_tables &c, cg_state *st,
+                         int slot, hipStream_t, void *xlo) {
     ++mock_p_updates();
     if (dtype != SIPG_F64) return SIPG_ERR_UNSUPPORTED;
     // z + P0^T C through a scratch copy, then the plain update with r.z + S.C
@@ -685,8 +684,8 @@ int launch_pcg2_update_p(int dtype, int p, void *x, void *pv, const void *z, int
     for (int64_t i = 0; i < n; ++i) zc[i] += mock_prolong(c, dimx, p + 1, i);
     std::vector<double> prz(part_rz, part_rz + np);
     if (np > 0) prz[np - 1] += sum_partials(c.part, npc);
-    pcg_update_p_t<double>(tp<double>(x), tp<double>(pv), zc.data(), n, part_pAp, np_pAp, part_rr, prz.data(), np,
-                           st, slot, tp<double>(xlo));
+    pcg_update_p_t<double>(tp<double>(x), tp<double>(pv), zc.data(), n, part_rr, prz.data(), np, st, slot,
+                           tp<double>(xlo));
     return SIPG_OK;
 }
 
