@@ -23,7 +23,7 @@
 //                  the tolerance, which then finishes only on that true
 //                  residual), and finished instances leave the lists.
 //
-// The block shape of the operator kernel is chosen per degree by timing the
+// The item shape of the operator kernel is chosen per degree by timing the
 // candidates on the batch's own instances (sipg_batch_tune).
 #include "sipg_internal.hpp"
 
@@ -316,7 +316,7 @@ int alloc_lists(sipg_batch &b) {
     return SIPG_OK;
 }
 
-// Times each candidate block shape on all instances of each degree and
+// Times each candidate item shape on all instances of each degree and
 // keeps the fastest (2 warm-up + 5 timed applies per candidate).
 // Tuning results kept for the life of the process, keyed by the device's
 // architecture, the degree and the size class of that degree's work (the

@@ -18,12 +18,13 @@
 // loaded twice.  The next row's loads are in flight while a row is
 // computed.
 //
-// Bound: the issue of vector-memory instructions (27 a row: columns of p+1
-// values are stored as they sit in the lanes, 8 (p+1) bytes to a segment)
-// and the FP64 arithmetic, 218 instructions a row at p = 8; with its stores
-// removed the kernel ran in 108 instead of 150 us at 1024 x 1024, p = 8.
-// Storing through LDS as whole rows instead cost more LDS time than it
-// saved.
+// Bound: on meshes past the caches the stores, columns of p+1 values as they
+// sit in the lanes, sizeof(T) (p+1) bytes to a segment: 322 us at 1024 x 1024,
+// p = 8 FP64, 151 with the stores left out, where a copy takes 258.  On cached
+// ones the issue of vector-memory instructions (3 (p+1) a row) and the FP64
+// arithmetic, 218 instructions a row at p = 8: 18.8 us at 256 x 256, 12.8
+// without the stores.  Storing through LDS as whole rows instead cost more LDS
+// time than it saved.
 #pragma once
 #include "line_math.hpp"
 

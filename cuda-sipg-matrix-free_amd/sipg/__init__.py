@@ -287,7 +287,7 @@ class Operator:
         return lib().sipg_to_reference_layout(self.h, dev.ptr, ref.ptr)
 
     def set_kernel(self, kernel):
-        """KERNEL_AUTO, KERNEL_VALU or KERNEL_MFMA (sipg_op_set_kernel)."""
+        """KERNEL_AUTO, KERNEL_VALU, KERNEL_MFMA or KERNEL_WAVE (sipg_op_set_kernel)."""
         check(lib().sipg_op_set_kernel(self.h, kernel), "op_set_kernel")
 
     def kernel(self, dtype=None):

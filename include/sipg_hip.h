@@ -101,8 +101,9 @@ int sipg_op_tables(const sipg_op *op, double *nodes, double *weights, double *D,
 
 /* Contraction kernel of the op's applies.  No counterpart in the
  * reference: SIPG_KERNEL_VALU runs the element contractions on the vector
- * ALUs with an element's lines spread over a workgroup, SIPG_KERNEL_WAVE
- * on the vector ALUs with whole elements per wave (p = 8), SIPG_KERNEL_MFMA
+ * ALUs with each wave marching a strip of whole elements through the mesh,
+ * SIPG_KERNEL_WAVE on the vector ALUs over blocks of elements staged in LDS
+ * (p = 2, 4, 6, 8; in FP32 also 10 and 12), SIPG_KERNEL_MFMA
  * on the matrix cores (FP32, p = 15); a kernel that does not exist for the
  * op's dtype and degree falls back to SIPG_KERNEL_VALU.  SIPG_KERNEL_AUTO
  * (the default) picks the fastest.  A mixed-precision solve passes the
@@ -281,9 +282,10 @@ int sipg_batch_create(sipg_batch **out, int ninst, const int *dimx, const int *d
 int sipg_batch_destroy(sipg_batch *b);
 int sipg_batch_size(const sipg_batch *b, int64_t *total_n);
 int sipg_batch_offset(const sipg_batch *b, int inst, int64_t *offset, int64_t *n);
-/* Chooses the operator kernel's block shape for every degree of the batch
- * by timing the candidates (16x4, 8x4, 8x2 elements) on the batch's own
- * instances, and records the choice in a process-wide cache keyed by the
+/* Chooses the shape of the operator kernel's work items for every degree of
+ * the batch by timing the candidates, named 16x4, 8x4 and 8x2 (strips of
+ * 64 / (p+1) elements by 16, 8 and 4 rows; 16x4 up to p = 12), on the batch's
+ * own instances, and records the choice in a process-wide cache keyed by the
  * device architecture, the degree and the size class of that degree's
  * work (the binary order of its element count).  On first use without a
  * call, a batch whose every degree is in the cache takes those shapes
@@ -293,7 +295,7 @@ int sipg_batch_offset(const sipg_batch *b, int inst, int64_t *offset, int64_t *n
  * tuning). */
 int sipg_batch_tune(sipg_batch *b);
 int sipg_batch_tuning(const sipg_batch *b, int p, int *bx, int *by, double *us_per_apply);
-/* Fixes the block shape (bx x by elements, one of the candidates) for the
+/* Fixes the item shape (one of the candidates, by its name bx x by) for the
  * instances of degree p, in place of tuning (for callers that tune offline,
  * and for tests of every shape). */
 int sipg_batch_set_shape(sipg_batch *b, int p, int bx, int by);
@@ -343,8 +345,8 @@ int sipg_batch_pcg(sipg_batch *b, void *x, const void *rhs, const sipg_cg_opts *
 typedef struct sipg_server sipg_server;
 int sipg_server_create(sipg_server **out, double hbm_budget_bytes, void *stream);
 int sipg_server_destroy(sipg_server *s);
-/* Block shape of the operator kernel for degree p (a sipg_batch_tune
- * result; 8x4 by default), while no request of degree p is running. */
+/* Item shape of the operator kernel for degree p (a sipg_batch_tune result;
+ * 8x4 by default), while no request of degree p is running. */
 int sipg_server_set_shape(sipg_server *s, int p, int bx, int by);
 /* Solver of every request: SIPG_METHOD_CG (the default) or SIPG_METHOD_PCG,
  * the block-Jacobi preconditioned CG of sipg_batch_pcg
@@ -352,7 +354,7 @@ int sipg_server_set_shape(sipg_server *s, int p, int bx, int by);
  * Only while the server holds no request (else SIPG_ERR_INVALID).  Under
  * PCG a request of n unknowns needs 56 n bytes (one more vector), submit
  * refuses a penalty other than 5 (p+1)^2 with SIPG_ERR_UNSUPPORTED, and so
- * does set_shape a block shape the preconditioner kernel lacks. */
+ * does set_shape an item shape the preconditioner kernel lacks. */
 enum { SIPG_METHOD_CG = 0, SIPG_METHOD_PCG = 1 };
 int sipg_server_set_method(sipg_server *s, int method);
 /* Queue a request: dim x dim mesh of degree p, penalty pen, Fourier forcing
