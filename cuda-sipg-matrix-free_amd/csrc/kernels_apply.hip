@@ -145,7 +145,7 @@ int resolve_kernel(int dtype, int p, int kernel) {
     // even p <= 8 and in FP32 <= 12, strips elsewhere.  Strips store a lane's
     // column, sizeof(T) (p+1) bytes to a segment, which costs most where it is
     // short and the lines leave the caches partly written: 1024 x 1024, p = 8
-    // FP64 330 against 278 us, FP32 256 x 256, p = 8 16.2 against 12.1.  At p = 15
+    // FP64 322 against 279 us, FP32 256 x 256, p = 8 16.2 against 12.1.  At p = 15
     // in FP32 strips take 3.9 against 2.8 us at 4 x 4, 4.5 against 4.8 at 64 x 64
     // and 8.9 against 10.9 at 128 x 128, and are 5 % further from 64 bits (6.5e-8
     // against 6.2e-8 on uniform values): the matrix cores stay.
