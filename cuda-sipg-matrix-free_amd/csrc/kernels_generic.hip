@@ -23,17 +23,18 @@
 // v_mfma_f32_16x16x4f32, 32 cycles each), and FP32 sums in that order were 5 %
 // further off than one multiply-add after the other.  A workgroup has one wave
 // to a row of output tiles; K1 stays in registers for all elements, so that a
-// step of four i costs NT + 1 LDS reads for 2 NT instructions.  The face terms are two more steps: [D0 DN g h]
-// times [ev; fv; D0; DN], and the corrections with the unit vectors of the
-// boundary lines in the place of D0 and DN.  The next element's values are
+// step of four i costs NT + 1 LDS reads for 2 NT instructions.  The face terms are one more step, [D0 DN g h]
+// times [ev; fv; D0; DN]; the corrections are added on the boundary lines only
+// (as products with unit vectors they carried a NaN or an infinity of a
+// neighbour's into whole lines: 0 times NaN).  The next element's values are
 // in flight meanwhile.
 //
 // Bound: latency, with two or three waves per SIMD beside K1 in registers (20
-// million unknowns in FP64 at p = 20: 154 us here and 65 in face_derivs, for
+// million unknowns in FP64 at p = 20: 148 us here and 65 in face_derivs, for
 // 160 MB read by each and 160 MB written).  us an apply, with a thread to an
 // output and every operand of its 4 (p+1) multiply-adds from memory and LDS
-// before, and now: FP64 213 x 213, p = 20 780, 219; 135 x 135, p = 32 1016, 268;
-// 70 x 70, p = 63 1334, 189; 6 x 6, p = 20 14.1, 9.3; FP32 213 x 213, p = 20
+// before, and now: FP64 213 x 213, p = 20 780, 213; 135 x 135, p = 32 1016, 263;
+// 70 x 70, p = 63 1334, 186; 6 x 6, p = 20 14.3, 9.4; FP32 213 x 213, p = 20
 // 574, 193.  Waves per SIMD (launch bounds): without the bound p = 20 240, p = 32
 // 338.
 //
@@ -154,8 +155,11 @@ __global__ __launch_bounds__(64 * NT, NT == 2 ? 3 : NT == 3 ? 2 : 1) void apply_
 
     int col[NT];                                                  // this lane's column of tile t
     double K[NK][NT], dE[NT], wc[NT], wr[4];
-    const int o = lk & 1, lineO = o ? N : 0;                      // this lane's side of a pair, and its boundary line
+    const int o = lk & 1;                                         // this lane's side of a pair
     const bool own = lk < 2;
+    // the tile that holds row (or column) N, another than tile 0 (N > 16), and
+    // where this wave's boundary row sits in it
+    const int tN = N >> 4, rS = ti == 0 ? 0 : (N & 15) >> 2, lkS = ti == 0 ? 0 : N & 3;
 #pragma unroll
     for (int c = 0; c < NT; ++c) {
         const int tj = ti + c < NT ? ti + c : ti + c - NT;
@@ -233,15 +237,28 @@ __global__ __launch_bounds__(64 * NT, NT == 2 ? 3 : NT == 3 ? 2 : 1) void apply_
 
         }
         __syncthreads();                                          // the faces are complete
-        // k = 0, 1: along x (factors D0 or DN, then the boundary lines, of i1), k = 2, 3: along y
-        const double a1 = own ? dE[0] : F[4 + o][col[0]], a2 = own ? (col[0] == lineO ? 1.0 : 0.0) : F[6 + o][col[0]];
+        // k = 0, 1: along x (factors D0 or DN of i1), k = 2, 3: along y; then
+        // the corrections, on the boundary lines alone
+        const double a1 = own ? dE[0] : F[4 + o][col[0]];
         T *ye = y + (int64_t)e * nq;
 #pragma unroll
         for (int c = 0; c < NT; ++c) {
             gd4 s = gmul(a1, own ? F[o][col[c]] : dE[c], gd4{0, 0, 0, 0});
+            const int tj = ti + c < NT ? ti + c : ti + c - NT;
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[r] += wc[c] * ax[c][r] + wr[r] * ay[c][r];
-            s = gmul(a2, own ? F[2 + o][col[c]] : (col[c] == lineO ? 1.0 : 0.0), s);
+            if (ti == 0 || ti == tN) {                            // this wave's tiles have row 0 or N
+                const double v = F[ti == 0 ? 2 : 3][col[c]];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r == rS && lk == lkS) s[r] += v;
+            }
+            if (tj == 0 || tj == tN) {                            // column 0 or N
+                if (li == (tj == 0 ? 0 : N & 15)) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[r] += F[tj == 0 ? 6 : 7][16 * ti + 4 * r + lk];
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * ti + 4 * r + lk;
