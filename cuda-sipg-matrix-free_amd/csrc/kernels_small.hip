@@ -10,7 +10,11 @@
 // the chunk ends.  The iteration is the one of conjugate_gradient
 // (conjugate_gradient_gpu.hpp:69-100) with the slot rules of
 // cg_update_xr_kernel / cg_update_p_kernel, so the host's chunk loop, its
-// replacements and its stopping decisions are unchanged.
+// replacements and its stopping decisions are unchanged.  A chunk is long: it
+// stops where the recursion first wants its final check (hold), where
+// iterations past that could use up the iteration cap, or run a few unknowns
+// until p.Ap is zero.  Where the host lets it go on all the same, a zero p.Ap
+// is an exact solution that waits for its check, not a breakdown.
 //
 // Bound: latency of four barriers and the dependent LDS reads between them.
 // Measured 8 x 8, p = 3 (1,024 unknowns): 15 -> 3.1 us per iteration, a solve
@@ -40,7 +44,8 @@ __device__ __forceinline__ double group_total(double v, double *red) {
 
 template <typename T, int P>
 __global__ __launch_bounds__(NT) void cg_small_kernel(T *__restrict__ x, T *__restrict__ r, T *__restrict__ p, int dimx,
-                                                      int dimy, T pen, int n_it, cg_state *st, int slot)
+                                                      int dimy, T pen, int n_it, int hold, cg_state *st,
+                                                      int slot)
 {
     constexpr int N1 = P + 1, NQ = N1 * N1;
     constexpr int RS = N1 % 2 ? N1 : N1 + 1, TS = N1 * RS;       // odd row stride: rows hit distinct banks
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(NT) void cg_small_kernel(T *__restrict__ x, T *__re
     }
     __syncthreads();
     int err = 0;
-    for (int it = 0; it < n_it && !cur.done; ++it) {
+    for (int it = 0; it < n_it && !cur.done && !(hold && (cur.flags & kSlotWantCheck)); ++it) {
         // both directions' lines
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
@@ -143,6 +148,7 @@ __global__ __launch_bounds__(NT) void cg_small_kernel(T *__restrict__ x, T *__re
             }
         }
         const double pAp = group_total(s, red[0]);
+        if (pAp == 0.0 && (cur.flags & kSlotWantCheck)) break;    // solved exactly: only the final check is left
         const double alpha_d = cur.rr / pAp;
         if (!(pAp > 0.0) || !isfinite(alpha_d)) {                 // the same in every thread
             err = isfinite(pAp) ? 2 : 3;
@@ -199,18 +205,18 @@ __global__ __launch_bounds__(NT) void cg_small_kernel(T *__restrict__ x, T *__re
 }
 
 template <typename T, int P>
-void launch_one(void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it, cg_state *st, int slot,
-                hipStream_t s) {
+void launch_one(void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it, bool hold, cg_state *st,
+                int slot, hipStream_t s) {
     hipLaunchKernelGGL((cg_small_kernel<T, P>), dim3(1), dim3(NT), 0, s, (T *)x, (T *)r, (T *)p, dimx, dimy, (T)pen,
-                       n_it, st, slot);
+                       n_it, hold ? 1 : 0, st, slot);
 }
 
 template <typename T, int P = 1>
-int dispatch(int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it, cg_state *st, int slot,
-             hipStream_t s) {
+int dispatch(int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it, bool hold, cg_state *st,
+             int slot, hipStream_t s) {
     if constexpr (P <= kMaxDegree) {
-        if (deg != P) return dispatch<T, P + 1>(deg, x, r, p, dimx, dimy, pen, n_it, st, slot, s);
-        launch_one<T, P>(x, r, p, dimx, dimy, pen, n_it, st, slot, s);
+        if (deg != P) return dispatch<T, P + 1>(deg, x, r, p, dimx, dimy, pen, n_it, hold, st, slot, s);
+        launch_one<T, P>(x, r, p, dimx, dimy, pen, n_it, hold, st, slot, s);
         SIPG_HIP_TRY(hipGetLastError());
         return SIPG_OK;
     }
@@ -224,10 +230,10 @@ bool cg_small_fits(int p, int dimx, int dimy) {
 }
 
 int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it,
-                    cg_state *st, int slot, hipStream_t s) {
+                    bool hold, cg_state *st, int slot, hipStream_t s) {
     if (!cg_small_fits(deg, dimx, dimy) || n_it < 1) return SIPG_ERR_INVALID;
-    return dtype == SIPG_F64 ? dispatch<double>(deg, x, r, p, dimx, dimy, pen, n_it, st, slot, s)
-                             : dispatch<float>(deg, x, r, p, dimx, dimy, pen, n_it, st, slot, s);
+    return dtype == SIPG_F64 ? dispatch<double>(deg, x, r, p, dimx, dimy, pen, n_it, hold, st, slot, s)
+                             : dispatch<float>(deg, x, r, p, dimx, dimy, pen, n_it, hold, st, slot, s);
 }
 
 }  // namespace sipg_internal

@@ -162,8 +162,11 @@ __global__ __launch_bounds__(NT) void cg_update_xr_kernel(T *__restrict__ x, con
     multi_sum<NT, 1>({ppAp}, {np}, sum);
     const double pAp = sum[0];
     const double rr = st->s[slot].rr;
-    const double alpha_d = rr / pAp;
-    if (!(pAp > 0.0) || !isfinite(alpha_d)) {
+    // a recursion that met the tolerance and went on until p.Ap is zero has
+    // solved exactly: it stands still until its final check
+    const bool exact = pAp == 0.0 && (st->s[slot].flags & kSlotWantCheck);
+    const double alpha_d = exact ? 0.0 : rr / pAp;
+    if ((!(pAp > 0.0) && !exact) || !isfinite(alpha_d)) {
         // every block takes this branch (same pAp); block 0 records it in a
         // word no kernel of this iteration reads at entry
         if (blockIdx.x == 0 && threadIdx.x == 0) st->err = isfinite(pAp) ? 2 : 3;
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(NT) void cg_update_p_kernel(const T *__restrict__ r
     multi_sum<NT, 1>({prr}, {np}, sum);
     const double rr_new = sum[0];
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
-    const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rr_new / cur.rr;
+    const double beta_d = (cur.flags & kSlotRestart) || cur.rr == 0.0 ? 0.0 : rr_new / cur.rr;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const bool met = !(sqrt(rr_new) > st->stop);
         const bool need_true = st->true_stop && !replaced;

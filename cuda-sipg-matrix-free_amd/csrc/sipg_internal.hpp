@@ -228,10 +228,11 @@ int launch_cg_update_p(int dtype, const void *r, void *p, int64_t n, const doubl
                        int np_rr, int nblk, cg_state *st, int slot, hipStream_t s);
 // n_it whole CG iterations of a small problem in one launch
 // (kernels_small.hip), from the slot `slot`; the result is that of n_it
-// times apply, x/r update and p update.
+// times apply, x/r update and p update.  hold: a slot that wants its final
+// check is left as it is (the host has not seen that yet).
 bool cg_small_fits(int p, int dimx, int dimy);
 int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it,
-                    cg_state *st, int slot, hipStream_t s);
+                    bool hold, cg_state *st, int slot, hipStream_t s);
 int launch_residual(int dtype, const void *b, const void *Ax, void *r, int64_t n, hipStream_t s);
 // out = (out dtype)(b - Ax) with b, Ax in in_dtype; optionally p = out;
 // block sums of (b-Ax).(b-Ax) and, when pbb != nullptr, of b.b.

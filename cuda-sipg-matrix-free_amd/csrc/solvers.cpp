@@ -223,13 +223,14 @@ struct Engine {
         return !pcg && !xL && opI->kernel == SIPG_KERNEL_AUTO && cg_small_fits(opI->p, opI->dimx, opI->dimy);
     }
 
-    // n_it iterations, the first of them replacing when asked
-    int iterations(int n_it, bool replace, bool restart_p) {
+    // n_it iterations, the first of them replacing when asked; hold: inside
+    // one workgroup, only as far as a recursion that wants its final check
+    int iterations(int n_it, bool replace, bool restart_p, bool hold) {
         int rc;
         for (int c = 0; c < n_it; ++c) {
             if (one_group && !(replace && c == 0)) {
-                if ((rc = launch_cg_small(opI->dtype, opI->p, xI, r, p, opI->dimx, opI->dimy, opI->pen, n_it - c, st,
-                                          (int)(launched & 1), s)))
+                if ((rc = launch_cg_small(opI->dtype, opI->p, xI, r, p, opI->dimx, opI->dimy, opI->pen, n_it - c, hold,
+                                          st, (int)(launched & 1), s)))
                     return rc;
                 launched += n_it - c;
                 return SIPG_OK;
@@ -407,7 +408,9 @@ struct Engine {
                 drain = true;
                 n_it = 1;
             }
-            if ((rc = iterations(n_it, want_rep, restart_p))) break;
+            // (hold: unless the host has seen the want and goes on for a
+            // larger drop)
+            if ((rc = iterations(n_it, want_rep, restart_p, want_rep || !(cs.flags & kSlotWantCheck)))) break;
             if (want_rep) {
                 ++nrep_enq;
                 check_pending = true;

@@ -235,6 +235,12 @@ int main() {
     run("small_near_floor", 6, 4, 125.0, 1, 1.5e-14, 0, 0.1, 0);
     run("small_mixed", 6, 4, 125.0, 2, 1e-10, 0, 0.1);
     run("small_breakdown", 6, 3, -400.0, 0, 1e-10, 0, 0.0);
+    // a few unknowns: the recursion reaches zero before the host has looked
+    run("small_exact", 1, 1, 20.0, 1, 1e-6, 2000, 0.01, 0);
+    run("small_exact_loose", 1, 1, 20.0, 1, 0.4, 2000, 0.0, 0);
+    run("small_exact_p2", 1, 2, 45.0, 1, 1e-3, 2000, 0.0, 0);
+    // a cap a few iterations above what the tolerance takes
+    run("small_near_cap", 6, 4, 125.0, 1, 1e-3, 182, 0.0, 0);
     coarse_check(5, 5, 3);
     coarse_check(6, 4, 2);
     coarse_check(4, 5, 1);

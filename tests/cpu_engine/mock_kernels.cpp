@@ -161,8 +161,9 @@ static void update_xr_t(T *x, const T *p, T *r, const T *Ap, int64_t n, const do
     if (st->s[slot].done | st->err) return;
     const double pAp = sum_partials(ppAp, np);
     const double rr = st->s[slot].rr;
-    const double alpha_d = rr / pAp;
-    if (!(pAp > 0.0) || !std::isfinite(alpha_d)) { st->err = std::isfinite(pAp) ? 2 : 3; return; }
+    const bool exact = pAp == 0.0 && (st->s[slot].flags & kSlotWantCheck);
+    const double alpha_d = exact ? 0.0 : rr / pAp;
+    if ((!(pAp > 0.0) && !exact) || !std::isfinite(alpha_d)) { st->err = std::isfinite(pAp) ? 2 : 3; return; }
     const T a = (T)alpha_d;
     double s = 0;
     for (int64_t i = 0; i < n; ++i) {
@@ -192,7 +193,7 @@ static void update_p_t(const T *r, T *p, int64_t n, const double *prr, int np, c
     if (cur.done | st->err) { st->s[slot ^ 1] = cur; return; }
     const double rr_new = sum_partials(prr, np);
     const bool replaced = (cur.flags & kSlotReplaced) != 0;
-    const double beta_d = (cur.flags & kSlotRestart) ? 0.0 : rr_new / cur.rr;
+    const double beta_d = (cur.flags & kSlotRestart) || cur.rr == 0.0 ? 0.0 : rr_new / cur.rr;
     const bool met = !(std::sqrt(rr_new) > st->stop);
     const bool need_true = st->true_stop && !replaced;
     cg_slot nx{};
@@ -232,17 +233,19 @@ int &mock_small_chunks() {
 }
 
 template <typename T>
-static void small_t(int deg, T *x, T *r, T *p, int dimx, int dimy, double pen, int n_it, cg_state *st, int slot) {
+static void small_t(int deg, T *x, T *r, T *p, int dimx, int dimy, double pen, int n_it, bool hold, cg_state *st,
+                    int slot) {
     cg_slot cur = st->s[slot];
     const int last = (slot + n_it) & 1;
     if (cur.done | st->err) { st->s[last] = cur; return; }
     const int64_t n = (int64_t)dimx * dimy * (deg + 1) * (deg + 1);
     std::vector<T> Ap(n);
     int err = 0;
-    for (int it = 0; it < n_it && !cur.done && !err; ++it) {
+    for (int it = 0; it < n_it && !cur.done && !err && !(hold && (cur.flags & kSlotWantCheck)); ++it) {
         apply_aos<T>(dimx, dimy, deg, pen, p, Ap.data());
         double pAp = 0;
         for (int64_t i = 0; i < n; ++i) pAp += (double)p[i] * (double)Ap[i];
+        if (pAp == 0.0 && (cur.flags & kSlotWantCheck)) break;
         const double alpha_d = cur.rr / pAp;
         if (!(pAp > 0.0) || !std::isfinite(alpha_d)) { err = std::isfinite(pAp) ? 2 : 3; break; }
         const T a = (T)alpha_d;
@@ -270,12 +273,12 @@ static void small_t(int deg, T *x, T *r, T *p, int dimx, int dimy, double pen, i
 }
 
 int launch_cg_small(int dtype, int deg, void *x, void *r, void *p, int dimx, int dimy, double pen, int n_it,
-                    cg_state *st, int slot, hipStream_t) {
+                    bool hold, cg_state *st, int slot, hipStream_t) {
     if (!cg_small_fits(deg, dimx, dimy) || n_it < 1) return SIPG_ERR_INVALID;
     mock_p_updates() += n_it;
     ++mock_small_chunks();
-    if (dtype == SIPG_F64) small_t<double>(deg, tp<double>(x), tp<double>(r), tp<double>(p), dimx, dimy, pen, n_it, st, slot);
-    else small_t<float>(deg, tp<float>(x), tp<float>(r), tp<float>(p), dimx, dimy, pen, n_it, st, slot);
+    if (dtype == SIPG_F64) small_t<double>(deg, tp<double>(x), tp<double>(r), tp<double>(p), dimx, dimy, pen, n_it, hold, st, slot);
+    else small_t<float>(deg, tp<float>(x), tp<float>(r), tp<float>(p), dimx, dimy, pen, n_it, hold, st, slot);
     return SIPG_OK;
 }
 

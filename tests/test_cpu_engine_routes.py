@@ -64,6 +64,21 @@ def test_small_cg_breakdown(results):  # noqa: F811
     assert r["rc"] == 8 and r["chunks"] > 0, r
 
 
+@pytest.mark.parametrize("case,tol", [("small_exact", 1e-6), ("small_exact_loose", 0.4), ("small_exact_p2", 1e-3)])
+def test_small_cg_that_solves_exactly_is_no_breakdown(results, case, tol):  # noqa: F811
+    # 4 and 9 unknowns: within a chunk the recursion falls to zero, or so low
+    # that p.Ap does; the solve still finishes on its true residual
+    r = results[case]
+    assert r["rc"] == 0 and r["chunks"] > 0 and r["reps"] >= 1 and r["relres"] <= tol, r
+
+
+def test_small_cg_does_not_run_past_its_tolerance_into_the_cap(results):  # noqa: F811
+    # the reference iteration takes 177: a cap five above is enough for the
+    # recursion and its final check
+    r = results["small_near_cap"]
+    assert r["oracle_iters"] == 177 and r["rc"] == 0 and r["chunks"] > 0 and r["iters"] <= 182, r
+
+
 def test_batched_pcg_about_the_item_limit(batch_results):  # noqa: F811
     # 512, 9 (of degree 3), 513 and 525 items
     rows = batch_results["batch_items"]
